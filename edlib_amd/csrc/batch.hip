@@ -1258,7 +1258,7 @@ int Batch::submit_lanczos(int sec, const double* v0_dev, int nl) {
   // <v, w>, each 256-byte aligned
   auto al = [](size_t c) { return (c + 31) & ~size_t(31); };
   const size_t nv = al((size_t)j.n), nsc = S_T + 2 * (size_t)nl + 3;
-  j.ntdot = hv_batch_routed_lanczos(s.dev) ? hv_batch_rows_partials(s.tabs.up.D)
+  j.ntdot = hv_batch_routed_lanczos(s.dev) ? hv_batch_rows_partials(s.dev)
                                                        : hv_batch_tasks(s.tabs.up.D, s.tabs.dn.D);
   double* base = dalloc(j, 3 * nv + al(nsc) + (size_t)j.ntdot);
   for (int q = 0; q < 3; ++q) j.lz[q] = j.lzb[q] = base + q * nv;

@@ -101,6 +101,9 @@ constexpr int kColBits = 22;
 constexpr uint32_t kColMask = (1u << kColBits) - 1u;
 constexpr int kMaxValues = 1 << (32 - kColBits);
 constexpr int kSlice = 64;  // sliced-ELL slice height (one wavefront)
+// Entry of the line passes: the column's byte offset in a plane of 16-byte
+// states in the low bits, the value's byte offset in the value table above.
+constexpr int kLineOff = 18;
 
 struct SpinTables {
   int nel = 0;
@@ -155,8 +158,9 @@ struct SectorTables {
 void build_sector(const Model& m, int nup, int ndn, SectorTables& st, bool need_rank);
 
 // H*v variants: single pass (rows, up-spin term from the cache hierarchy) or
-// two passes (rows without the up-spin term, then XCD-aware column slabs for
-// it).  HV_AUTO picks the one timed fastest for the sector.
+// two passes: whole columns, then whole rows gathered in LDS (hv_lines.hip)
+// where several of each fit, else rows without the up-spin term, then
+// XCD-aware column slabs for it.  HV_AUTO picks the sector's faster one.
 enum HvVariant { HV_SINGLE = 0, HV_TWO_PASS = 1, HV_AUTO = -1 };
 
 // Device mirror of one sector.
@@ -169,7 +173,7 @@ struct DevSpin {
   int32_t* sl_ptr = nullptr;
   int32_t* sl_len = nullptr;
   uint32_t* ell = nullptr;
-  uint16_t* ell16 = nullptr;
+  uint32_t* lell = nullptr;  // ell's slots as line-pass entries
   double vt16[4] = {0, 0, 0, 0};
   int nvt16 = 0;
   int32_t* q4_ptr = nullptr;
@@ -185,6 +189,9 @@ struct DevSector {
   double* values = nullptr;
   int nvalues = 0;  // entries of values
   int nkan = 0;     // impurity terms (entries of kan_off and kan_c)
+  bool lines = false;      // the line passes' tables are there
+  bool dn_signed = false;  // the down spin has the signed byte-offset form (ell_s4)
+  double hops = 0;  // mean hopping entries per state, both spins
   int imp_ml = 0;
   int cross_mode = 0;
   double cross_u = 0.0;
@@ -194,6 +201,16 @@ struct DevSector {
   int32_t* kan_ptr = nullptr;
   int64_t* kan_off = nullptr;  // element offset of each term's partner state
   double* kan_c = nullptr;
+  // The impurity terms by target, for row tiles that hold whole runs of the
+  // rows sharing their bath bits (row_tiles: four rows per tile, -1 = none):
+  // up pattern a leads to at most kan_t up patterns; a down pattern b has at
+  // most one term to target j, coefficient kan_tc (0: none) and kan_td =
+  // 8 * (state offset) + 4 + (row offset) at (a kan_t + j) 2^ml + b.
+  // row_tiles null: the terms have no such form, or more than three orbitals.
+  int kan_t = 0, n_row_tiles = 0;
+  int32_t* row_tiles = nullptr;
+  int32_t* kan_td = nullptr;
+  double* kan_tc = nullptr;
   int32_t* row_order = nullptr;  // processing order of up rows
   int variant = HV_SINGLE;       // chosen H*v variant
   int* counters = nullptr;       // work queues of the slab pass (8 ints)
@@ -270,6 +287,22 @@ void launch_hv(const DevSector& ds, const HvArgs& a, hipStream_t s, int variant 
 int hv_num_blocks(const DevSector& ds);
 int hv_autotune(DevSector& ds, hipStream_t s);
 
+// Two passes of LDS gathers over whole lines (hv_lines.hip): rows and columns
+// per work-group, work-group sizes and LDS of each pass, fixed by the sector
+// alone; ok: the lines fit LDS at least two at a time.
+struct HvLinesPlan {
+  int row_b, col_b, row_block, col_block;
+  size_t row_smem, col_smem;
+  bool ok;
+};
+HvLinesPlan hv_lines_plan(const DevSector& ds);
+int hv_lines_threads(int64_t D);
+int hv_lines_partials(const DevSector& ds);  // shares of <v, w> per operand
+bool hv_lines_faster(const DevSector& ds);   // than the single pass, for one operand alone
+constexpr int kLinesMax = 4;  // operands per launch
+constexpr int64_t kLinesLanczos = 2500000;  // smallest sector whose Lanczos operands take them in a batch
+void launch_hv_lines(const DevSector& ds, const HvArgs* ops, int count, hipStream_t s);
+
 // Grouped H*v over many operands (sectors of any models): one launch covers
 // the up-rows of all of them, cut into work units.  A job record is filled
 // on the host (hv_batch_fill) into a buffer of hv_batch_job_bytes() per job
@@ -299,7 +332,7 @@ bool hv_batch_routed(int64_t dup, int64_t ddn);
 // kernel, so that their runs share launches (the decision depends on the
 // sector only, so a run's arithmetic does not depend on the other runs).
 bool hv_batch_routed_lanczos(const DevSector& ds);
-int64_t hv_batch_rows_partials(int64_t dup);
+int64_t hv_batch_rows_partials(const DevSector& ds);
 void launch_hv_batch_rows(const DevSector& ds, const HvArgs& a, hipStream_t s);
 // Several Lanczos operands of one rows-kernel sector in one launch, each with
 // the single-operand launch's arithmetic: hv_batch_rows_multi_fit gives how

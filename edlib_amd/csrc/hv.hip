@@ -29,90 +29,9 @@
 #include <cstdlib>
 #include <cstring>
 
-#include "edh_internal.h"
+#include "hv_params.h"
 
 namespace edh {
-
-struct HvParams {
-  int Ns, nb;  // sites per spin, bath bits (Ns - ml) below the impurity bits
-  int Dup, Ddn;
-  const int32_t* row_order;
-  // up spin
-  const int32_t* up_bits;
-  const double* up_e;
-  const int32_t* up_rowp;
-  const uint32_t* up_packed;
-  // down spin
-  const int32_t* dn_bits;
-  const double* dn_e;
-  const int32_t* dn_slptr;
-  const int32_t* dn_sllen;
-  const uint32_t* dn_ell;
-  const int32_t* dn_q4ptr;
-  const uint64_t* dn_q4;
-  double dn_vt[4];
-  const uint32_t* dn_s4;
-  double dn_s4_scale;
-  const double* values;
-  int nvals;  // entries of values (staged in LDS after the row with EF == 4)
-  int nkan;   // impurity terms (staged in LDS by the multi-operand kernel)
-  // cross term
-  double cross_u;
-  const double* cross_imp;
-  const double* cross_rowtab;
-  // impurity interaction
-  int kan_ml;
-  const int32_t* kan_ptr;
-  const int64_t* kan_off;  // partner state's element offset per term
-  const double* kan_c;
-  // operands
-  const double* v;
-  double* w;
-  const double* wprev;
-  double vscale, wscale;
-  int accumulate;
-  double* dot_partial;
-  const double* dscale;
-  const int* done;
-  // slab kernel geometry; off32: every element offset fits 32 bits
-  int nslabs, rows_per_wg, nrb, off32;
-  int xcd_rows;  // rows kernel: XCD-grouped row assignment (measured 2 % faster on the 16-site sector)
-  // rows kernel in a batch: an eigensolver run's control block (v and w are
-  // then columns col and col + 1 of the basis in v or v_alt; a run whose
-  // state is not 0 is skipped)
-  const double* ctl;
-  const double* v_alt;
-};
-
-template <int CROSS>
-__device__ __forceinline__ double cross_term(const HvParams& p, int u, int bu, int bd, int na) {
-  if (CROSS == CROSS_POPC) return p.cross_u * (double)__builtin_popcount(bu & bd);
-  if (CROSS == CROSS_IMP) return p.cross_imp[(bu >> p.nb) * na + (bd >> p.nb)];
-  if (CROSS == CROSS_GENERAL) {
-    double x = 0.0;
-    const double* r = p.cross_rowtab + (size_t)u * p.Ns;
-    unsigned m = (unsigned)bd;
-    while (m) {
-      int b = __builtin_ctz(m);
-      x += r[b];
-      m &= m - 1;
-    }
-    return x;
-  }
-  return 0.0;
-}
-
-__device__ __forceinline__ void block_reduce_store(double x, double* s_red, double* out) {
-  for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
-  const int wid = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) s_red[wid] = x;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = 0.0;
-    for (int q = 0; q < (int)(blockDim.x >> 6); ++q) t += s_red[q];
-    *out = t;
-  }
-}
 
 // Decodes a compact entry's value: EF == 2 uses one class bit (two values),
 // EF == 1 two class bits (four values).
@@ -122,12 +41,6 @@ __device__ __forceinline__ double q4_value(const HvParams& p, uint32_t e) {
   const double lo = (e & 0x4000u) ? p.dn_vt[1] : p.dn_vt[0];
   const double hi = (e & 0x4000u) ? p.dn_vt[3] : p.dn_vt[2];
   return (e & 0x8000u) ? hi : lo;
-}
-
-// One signed byte-offset slot: a += (+-1) * row[e / 8], the sign in bit 0.
-__device__ __forceinline__ double s4_fma(uint32_t e, const char* sv, double a) {
-  const double sg = __hiloint2double((int)(0x3FF00000u | (e << 31)), 0);
-  return fma(sg, *reinterpret_cast<const double*>(sv + (e & ~1u)), a);
 }
 
 // Quads held in registers per column group (slices with more quads finish
@@ -787,16 +700,6 @@ __global__ __launch_bounds__(kSlabWG) void hv_upslab_kernel(HvParams p, int* cou
 // 4K elements each) listed on the host, and work-group b takes units b,
 // b + grid, ...  The down-spin hopping reads the 32-bit sliced ELL (present
 // for every sector), so any model and value set is handled.
-struct HvBatchJob {
-  HvParams p;
-  int64_t row0;
-  int cross, kan;
-  const double* ctl;    // eigensolver control block or null
-  const double* v_alt;  // second basis buffer (with ctl)
-  double* tdot;         // per-task shares of <v, w>, or null
-  const double* lzk;    // Lanczos run's step counter (buffers in rotation) or null
-};
-
 // One element of the grouped H*v: w[u][d] (written to W) from the operand
 // V scaled by vscale; returns v[u][d] * w[u][d] (scaled v).  With STAGED,
 // R is row u of V copied into LDS, and the element's own value and its
@@ -966,8 +869,6 @@ __global__ __launch_bounds__(512) void hv_batch_wave_kernel(const HvBatchJob* __
   }
 }
 
-namespace {
-
 // Largest dynamic LDS a block may use on the current device (queried once per device).
 size_t lds_budget() {
   static int cached[64] = {0};
@@ -981,6 +882,8 @@ size_t lds_budget() {
   }
   return (size_t)cached[dev] - 1024;  // room for the block's static reduction scratch
 }
+
+namespace {
 
 struct Launch {
   int J, block, grid;
@@ -1082,11 +985,15 @@ HvParams make_params(const DevSector& ds, const HvArgs& a) {
   p.up_e = ds.up.ediag;
   p.up_rowp = ds.up.rowp;
   p.up_packed = ds.up.packed;
+  p.up_slptr = ds.up.sl_ptr;
+  p.up_sllen = ds.up.sl_len;
+  p.up_lell = ds.up.lell;
   p.dn_bits = ds.dn.bits;
   p.dn_e = ds.dn.ediag;
   p.dn_slptr = ds.dn.sl_ptr;
   p.dn_sllen = ds.dn.sl_len;
   p.dn_ell = ds.dn.ell;
+  p.dn_lell = ds.dn.lell;
   p.dn_q4ptr = ds.dn.q4_ptr;
   p.dn_q4 = ds.dn.ell_q4;
   p.dn_s4 = ds.dn.ell_s4;
@@ -1102,6 +1009,10 @@ HvParams make_params(const DevSector& ds, const HvArgs& a) {
   p.kan_ptr = ds.kan_ptr;
   p.kan_off = ds.kan_off;
   p.kan_c = ds.kan_c;
+  p.kan_t = ds.kan_t;
+  p.row_tiles = ds.row_tiles;
+  p.kan_td = ds.kan_td;
+  p.kan_tc = ds.kan_tc;
   p.v = a.v;
   p.w = a.w;
   p.wprev = a.wprev;
@@ -1113,6 +1024,8 @@ HvParams make_params(const DevSector& ds, const HvArgs& a) {
   p.done = a.done;
   slab_geometry(ds, p.nslabs, p.rows_per_wg, p.nrb);
   p.off32 = (uint64_t)ds.N < (uint64_t(1) << 32);
+  p.row_t = hv_lines_threads(ds.dn.D);
+  p.col_t = hv_lines_threads(ds.up.D);
   p.xcd_rows = 1;
   p.ctl = a.ctl;
   p.v_alt = a.v_alt;
@@ -1122,14 +1035,16 @@ HvParams make_params(const DevSector& ds, const HvArgs& a) {
 }  // namespace
 
 int hv_num_blocks(const DevSector& ds) {
+  if (ds.variant != HV_TWO_PASS) return plan(ds).grid;
+  if (hv_lines_plan(ds).ok) return hv_lines_partials(ds);
   int nslabs, rpw, nrb;
-  const int grid = slab_geometry(ds, nslabs, rpw, nrb);
-  return ds.variant == HV_TWO_PASS ? grid : plan(ds).grid;
+  return slab_geometry(ds, nslabs, rpw, nrb);
 }
 
 void launch_hv(const DevSector& ds, const HvArgs& a, hipStream_t s, int variant) {
   if (ds.N == 0) return;
   if (variant == HV_AUTO) variant = ds.variant;
+  if (variant == HV_TWO_PASS && hv_lines_plan(ds).ok) return launch_hv_lines(ds, &a, 1, s);
   Launch L = plan(ds);
   HvParams p = make_params(ds, a);
   const bool kan = ds.kan_ml > 0;
@@ -1150,11 +1065,13 @@ void launch_hv(const DevSector& ds, const HvArgs& a, hipStream_t s, int variant)
   }
 }
 
-// Times both variants on scratch vectors and keeps the faster one (an
+// Where the line passes apply the choice is a rule (hv_lines_faster); else
+// both variants are timed on scratch vectors and the faster one is kept (an
 // environment override EDH_HV_VARIANT=0/1 fixes the choice).
 int hv_autotune(DevSector& ds, hipStream_t s) {
   const char* env = getenv("EDH_HV_VARIANT");
   if (env && (env[0] == '0' || env[0] == '1')) return env[0] - '0';
+  if (hv_lines_plan(ds).ok) return hv_lines_faster(ds) ? HV_TWO_PASS : HV_SINGLE;
   if (ds.N < (1 << 22)) return HV_SINGLE;  // short rows: the slab pass never pays
   double *v = nullptr, *w = nullptr;
   if (hipMalloc(&v, ds.N * sizeof(double)) != hipSuccess) return HV_SINGLE;
@@ -1203,17 +1120,22 @@ namespace edh {
 
 size_t hv_batch_job_bytes() { return sizeof(HvBatchJob); }
 
-void hv_batch_fill(const DevSector& ds, const HvArgs& a, int64_t row0, void* out) {
+HvBatchJob make_job(const DevSector& ds, const HvArgs& a) {
   HvBatchJob j;
   std::memset(&j, 0, sizeof(j));
   j.p = make_params(ds, a);
-  j.row0 = row0;
   j.cross = ds.cross_mode;
   j.kan = ds.kan_ml > 0 ? 1 : 0;
   j.ctl = a.ctl;
   j.v_alt = a.v_alt;
   j.tdot = a.tdot;
   j.lzk = a.lzk;
+  return j;
+}
+
+void hv_batch_fill(const DevSector& ds, const HvArgs& a, int64_t row0, void* out) {
+  HvBatchJob j = make_job(ds, a);
+  j.row0 = row0;
   std::memcpy(out, &j, sizeof(j));
 }
 
@@ -1287,15 +1209,26 @@ bool multi_ok(const DevSector& ds) {
 }
 }  // namespace
 
+namespace {
+// Lanczos operands on the line passes: large sectors where they beat the
+// single pass (14-site Kanamori sector (8,7), four operands: 860 us of H*v per step
+// against 944 in the multi-operand rows kernel).
+bool lines_lanczos(const DevSector& ds) { return ds.N >= kLinesLanczos && hv_lines_faster(ds); }
+}  // namespace
+
 bool hv_batch_routed_lanczos(const DevSector& ds) {
+  if (lines_lanczos(ds)) return true;
   const int64_t dup = ds.up.D, ddn = ds.dn.D;
   if (hv_batch_routed(dup, ddn)) return true;
   return dup >= 256 && ddn >= 512 && ddn <= kStageMax && multi_ok(ds);
 }
 
-int64_t hv_batch_rows_partials(int64_t dup) { return std::min<int64_t>(dup, 1 << 20); }
+int64_t hv_batch_rows_partials(const DevSector& ds) {
+  return lines_lanczos(ds) ? hv_lines_partials(ds) : std::min<int64_t>(ds.up.D, 1 << 20);
+}
 
 int hv_batch_rows_multi_fit(const DevSector& ds) {
+  if (lines_lanczos(ds)) return kLinesMax;
   return hv_batch_routed_lanczos(ds) && multi_ok(ds) ? kMultiMax : 0;
 }
 
@@ -1322,8 +1255,16 @@ void launch_multi_c(const HvParams& p, const HvMulti& m, const Launch& L, size_t
 void launch_hv_batch_rows_multi(const DevSector& ds, const HvArgs* a, int count, hipStream_t s) {
   const int fit = hv_batch_rows_multi_fit(ds);
   EDH_CHECK(count >= 2 && count <= fit, EDH_ERR_INTERNAL, "grouped H*v: operand count does not fit one launch");
+  if (lines_lanczos(ds)) {
+    HvArgs b[kLinesMax];
+    for (int k = 0; k < count; ++k) {
+      b[k] = a[k];
+      b[k].dot_partial = a[k].tdot;
+    }
+    return launch_hv_lines(ds, b, count, s);
+  }
   const Launch L = plan(ds);
-  EDH_CHECK(L.grid == hv_batch_rows_partials(ds.up.D), EDH_ERR_INTERNAL, "grouped H*v: rows grid mismatch");
+  EDH_CHECK(L.grid == hv_batch_rows_partials(ds), EDH_ERR_INTERNAL, "grouped H*v: rows grid mismatch");
   HvMulti m;
   std::memset(&m, 0, sizeof(m));
   for (int k = 0; k < count; ++k) {
@@ -1353,11 +1294,14 @@ void launch_hv_batch_rows_multi(const DevSector& ds, const HvArgs* a, int count,
 void launch_hv_batch_rows(const DevSector& ds, const HvArgs& a, hipStream_t s) {
   EDH_CHECK(hv_batch_routed_lanczos(ds), EDH_ERR_INTERNAL,
             "grouped H*v: operand not routed to the rows kernel");
-  EDH_CHECK(plan(ds).grid == hv_batch_rows_partials(ds.up.D), EDH_ERR_INTERNAL, "grouped H*v: rows grid mismatch");
+  const bool lines = !a.ctl && a.tdot && lines_lanczos(ds);
+  EDH_CHECK(lines || !a.tdot || plan(ds).grid == hv_batch_rows_partials(ds), EDH_ERR_INTERNAL,
+            "grouped H*v: rows grid mismatch");
   EDH_CHECK(!a.lzk, EDH_ERR_INTERNAL, "grouped H*v: rows-kernel operands take resolved buffers");
   HvArgs b = a;
   b.dot_partial = a.tdot;  // one share of <v, w> per work-group (row slot)
-  launch_hv(ds, b, s, HV_SINGLE);
+  if (lines) launch_hv_lines(ds, &b, 1, s);
+  else launch_hv(ds, b, s, HV_SINGLE);
 }
 
 }  // namespace edh

@@ -1,0 +1,609 @@
+// H*v in two passes of LDS gathers, for sectors whose lines fit LDS several
+// at a time.
+//
+// The state vector is the D_up x D_dn matrix V[u][d].  The down-spin hopping
+// mixes the elements of a row, the up-spin hopping those of a column, both
+// through a sparse table with one line of entries per basis state.  A
+// work-group stages B whole lines (columns, then rows) in LDS with the B
+// values of a basis state side by side, so that
+//   * one table entry (index, value), loaded and decoded once, serves B
+//     elements, and a gather is a 16-byte LDS read per two of them;
+//   * neighbour rows of the up-spin term are never re-read from L2 or beyond:
+//     each pass reads V once.
+// Pass 1 (columns): w = up-spin hopping (+ w_in when that is w itself).
+// Pass 2 (rows): w += diag v + w_in + down-spin hopping + impurity terms, and
+// the shares of <v, w>.
+//
+// An element's sum runs in table order in one register whatever the other
+// operands of the launch, and a row tile's share of <v, w> depends on the
+// sector alone: an operand's result is bit-identical alone and in any mix.
+//
+// What bounds it (14-site sectors, 3432 x 3432, MI355X): a column pass moves
+// 16 N bytes and a row pass 24 N (32 N with an accumulated input in another
+// buffer), 37 and 60 us of their 55 and 70 us with 7 entries per state
+// (Anderson); every further entry costs 2.6 us a pass, the LDS reads (two
+// 16-byte and one 8-byte read per entry and four elements, half as long again
+// with bank conflicts).  Kanamori sector (7,7): 83 + 107 us against 372 us in
+// the single pass.  B = 2 (two work-groups per CU) took 98 + 137 us on the
+// t, t' torus where B = 4 takes 92 + 108: the entries are decoded twice as
+// often and every row's request is half as long.
+#include <algorithm>
+#include <cstring>
+
+#include "hv_params.h"
+
+namespace edh {
+
+namespace {
+
+// The operand of a job as the device resolves it.
+struct View {
+  const double* V;
+  double* W;
+  const double* Wp;
+  double vs, ws;
+  bool accum, live;
+};
+
+__device__ __forceinline__ View resolve_view(const HvBatchJob& J) {
+  const HvParams& p = J.p;
+  View o;
+  o.V = p.v;
+  o.W = p.w;
+  o.Wp = p.wprev;
+  o.accum = p.accumulate != 0;
+  o.live = !(p.done && *p.done);
+  if (J.ctl) {  // eigensolver run: its basis column and buffer
+    if (J.ctl[kCtlState] != 0.0) o.live = false;
+    const int64_t N = (int64_t)p.Dup * p.Ddn;
+    const double* base = J.ctl[kCtlPhase] != 0.0 ? J.v_alt : p.v;
+    const int64_t col = (int64_t)J.ctl[kCtlCol];
+    o.V = base + col * N;
+    o.W = const_cast<double*>(base) + (col + 1) * N;
+  } else if (J.lzk) {  // Lanczos run: its buffers in rotation by the step counter
+    const int k = (int)*J.lzk;
+    const double* b[3] = {p.v, p.wprev, p.w};
+    const int r0 = lz_buffer(k, 0), r1 = lz_buffer(k, 1), r2 = lz_buffer(k, 2);
+    o.V = r0 == 0 ? b[0] : (r0 == 1 ? b[1] : b[2]);
+    o.Wp = r1 == 0 ? b[0] : (r1 == 1 ? b[1] : b[2]);
+    o.W = const_cast<double*>(r2 == 0 ? b[0] : (r2 == 1 ? b[1] : b[2]));
+    o.accum = k > 1;
+  }
+  o.vs = p.dscale ? p.dscale[0] : p.vscale;
+  o.ws = p.dscale ? p.dscale[1] : p.wscale;
+  return o;
+}
+
+// LDS image of B lines of D elements: planes of two lines, the pair of a
+// basis state in 16 bytes, then a zero state (with all B values side by side a 16-byte read
+// would use every other 16-byte slot of the banks only).
+template <int B>
+__device__ __forceinline__ void put_state(double* s, int ld, int i, const double (&x)[B]) {
+#pragma unroll
+  for (int q = 0; q < B / 2; ++q) reinterpret_cast<double2*>(s)[q * ld + i] = make_double2(x[2 * q], x[2 * q + 1]);
+}
+
+template <int B>
+__device__ __forceinline__ void get_state(const double* s, int ld, int i, double (&x)[B]) {
+#pragma unroll
+  for (int q = 0; q < B / 2; ++q) {
+    const double2 y = reinterpret_cast<const double2*>(s)[q * ld + i];
+    x[2 * q] = y.x;
+    x[2 * q + 1] = y.y;
+  }
+}
+
+// acc[b] += sum over the entries of basis state i (slice i / 64) of
+// value * line b[column].  An entry holds its column's byte offset in a plane
+// and its value's byte offset in the value table (kLineOff), so decoding it
+// takes two instructions.  The slice's slot count is wavefront-uniform; U
+// entries are decoded together, the next U in flight (B = 4, U = 8 against
+// 4: 14-site Kanamori column pass 111 -> 94 us).
+template <int B, int U>
+__device__ __forceinline__ void gather_line(const double* s, int ld, const double* s_vals, const int32_t* slptr,
+                                            const int32_t* sllen, const uint32_t* ell, int i, double (&acc)[B]) {
+  const int sl = __builtin_amdgcn_readfirstlane(i >> 6);
+  const int len = __builtin_amdgcn_readfirstlane(sllen[sl]);
+  const uint32_t* el = ell + slptr[sl] + (i & 63);
+  const char* const pl = reinterpret_cast<const char*>(s);
+  const char* const vl = reinterpret_cast<const char*>(s_vals);
+  uint32_t e[U];
+#pragma unroll
+  for (int r = 0; r < U; ++r) e[r] = r < len ? el[r * kSlice] : 0u;
+  for (int k = 0; k < len; k += U) {
+    uint32_t n[U];
+#pragma unroll
+    for (int r = 0; r < U; ++r) n[r] = k + U + r < len ? el[(k + U + r) * kSlice] : 0u;
+#pragma unroll
+    for (int r = 0; r < U; ++r) {
+      if (k + r < len) {
+        const uint32_t at = e[r] & ((1u << kLineOff) - 1u);
+        double2 x[B / 2];
+#pragma unroll
+        for (int q = 0; q < B / 2; ++q) x[q] = *reinterpret_cast<const double2*>(pl + (size_t)q * ld * 16 + at);
+        const double h = *reinterpret_cast<const double*>(vl + (e[r] >> kLineOff));
+#pragma unroll
+        for (int q = 0; q < B / 2; ++q) {
+          acc[2 * q] = fma(h, x[q].x, acc[2 * q]);
+          acc[2 * q + 1] = fma(h, x[q].y, acc[2 * q + 1]);
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < U; ++r) e[r] = n[r];
+  }
+}
+
+// The rows of a row tile: listed where the impurity terms' tables need whole
+// runs of rows together, else B consecutive ones.
+template <int B>
+struct Rows {
+  int u[B], n;
+  __device__ __forceinline__ Rows(const HvParams& p, int tile) {
+    if (B == 4 && p.row_tiles) {
+      n = 0;
+#pragma unroll
+      for (int r = 0; r < B; ++r) {
+        u[r] = p.row_tiles[4 * tile + r];
+        n += u[r] >= 0 ? 1 : 0;
+      }
+    } else {
+      n = min(B, p.Dup - tile * B);
+#pragma unroll
+      for (int r = 0; r < B; ++r) u[r] = tile * B + r;
+    }
+#pragma unroll
+    for (int r = 0; r < B; ++r)
+      if (r >= n) u[r] = u[0];
+  }
+};
+
+// (the slot's row for a lane-dependent slot)
+template <int B>
+__device__ __forceinline__ int row_of(const Rows<B>& R, int r) {
+  int u = R.u[0];
+#pragma unroll
+  for (int q = 1; q < B; ++q) u = r == q ? R.u[q] : u;
+  return u;
+}
+
+// Impurity terms of basis state d: acc[r] += sum over the terms of (a_r, b)
+// of c * V[partner], from memory.
+template <int B>
+__device__ __forceinline__ void kan_terms(const HvParams& p, const View& o, const Rows<B>& R, const int (&a)[B], int b,
+                                          int na, int d, double (&acc)[B]) {
+#pragma unroll
+  for (int r = 0; r < B; ++r) {
+    if (r >= R.n) break;
+    const int* kp = p.kan_ptr + a[r] * na + b;
+    const int64_t at = (int64_t)R.u[r] * p.Ddn + d;
+    for (int q = kp[0]; q < kp[1]; ++q) acc[r] = fma(p.kan_c[q], o.V[at + p.kan_off[q]] * o.vs, acc[r]);
+  }
+}
+
+// The same in a tile of whole runs (DevSector::row_tiles): the states sharing
+// their bath bits are neighbouring rows, so every partner is in LDS, and the
+// rows a term leads to are the same for all states of a row.  The rows' reads
+// are in flight together.
+template <int B>
+__device__ __forceinline__ void kan_targets(const HvParams& p, const double* tc, const int* td, const double* s,
+                                            int ld, const int (&a)[B], int b, int na, int n, int d,
+                                            double (&acc)[B]) {
+  for (int j = 0; j < p.kan_t; ++j) {
+    double c[B], x[B];
+    int at[B];
+#pragma unroll
+    for (int r = 0; r < B; ++r) {
+      const int q = (a[r] * p.kan_t + j) * na + b;
+      c[r] = r < n ? tc[q] : 0.0;
+      at[r] = td[q];  // 8 * (state offset) + 4 + (row offset)
+    }
+#pragma unroll
+    for (int r = 0; r < B; ++r) {
+      const int rr = r + (at[r] & 7) - 4;  // the partner's row in the tile
+      x[r] = s[((size_t)(rr >> 1) * ld + d + (at[r] >> 3)) * 2 + (rr & 1)];
+    }
+    // (a state without this term must not pick up 0 * infinity)
+#pragma unroll
+    for (int r = 0; r < B; ++r) acc[r] = c[r] != 0.0 ? fma(c[r], x[r], acc[r]) : acc[r];
+  }
+}
+
+// The work-groups of a launch stay and take tiles in turn; while a tile is
+// worked on, the lines of the work-group's next tile are on their way into
+// registers (NI basis states x B lines per thread), so that neither waits for
+// the other: a tile of four 3432-element lines takes most of a CU's LDS, and
+// one work-group per CU has no other one to fill the wait.
+template <int B, int NI>
+struct Ahead {
+  double x[NI][B];
+};
+
+// The thread's index as a value of this tile: what depends on it is computed
+// in every tile instead of being kept in registers over all of them.
+__device__ __forceinline__ int fresh_tid() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
+// Tables of a row tile in LDS after its lines: the value table, the impurity
+// terms (coefficients, then state offsets), the rows' cross-term vectors (one
+// value per row and site, CROSS_GENERAL).
+template <int B>
+struct RowTables {
+  double *vals, *kc, *ct;
+  int* kd;
+  int nk;  // impurity-term table entries staged
+  __device__ __forceinline__ RowTables(const HvBatchJob& J, double* s, int ld) {
+    const HvParams& p = J.p;
+    const int na = 1 << (p.Ns - p.nb);
+    vals = s + (size_t)B * ld;
+    nk = B == 4 && J.kan && p.row_tiles ? na * na * p.kan_t : 0;
+    kc = vals + p.nvals;
+    kd = reinterpret_cast<int*>(kc + nk);
+    ct = kc + nk + (nk + 1) / 2;
+  }
+};
+
+template <int B, int NI>
+__device__ __forceinline__ void row_fetch(const HvBatchJob& J, const View& o, int tile, Ahead<B, NI>& f, int i0,
+                                          int i1) {
+  const HvParams& p = J.p;
+  const int D = p.Ddn;
+  const Rows<B> R(p, tile);
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    if (i < i0 || i >= i1) continue;
+    const int d = threadIdx.x + i * p.row_t;
+#pragma unroll
+    for (int r = 0; r < B; ++r)
+      f.x[i][r] = (int)threadIdx.x < p.row_t && d < D && r < R.n ? o.V[(size_t)R.u[r] * D + d] : 0.0;
+  }
+}
+
+// One row tile whose lines are in f; the next tile's (tn, when there are more)
+// are fetched into f on the way.
+template <int B, int NI>
+__device__ __forceinline__ void row_tile(const HvBatchJob& J, int tile, bool tables, bool more, int tn,
+                                         Ahead<B, NI>& f, double* s, double* s_red) {
+  const HvParams& p = J.p;
+  const View o = resolve_view(J);
+  const int D = p.Ddn, T = blockDim.x;
+  const int tid = fresh_tid();
+  const int ld = D + 1;
+  const Rows<B> R(p, tile);
+  const int na = 1 << (p.Ns - p.nb);
+  // the accumulated input is read here unless it is w itself (then the
+  // column pass has read it)
+  const bool accum = o.accum && o.Wp != o.W;
+  const RowTables<B> t(J, s, ld);
+  if (tables) {
+    for (int i = tid; i < p.nvals; i += T) t.vals[i] = p.values[i];
+    for (int i = tid; i < t.nk; i += T) {
+      t.kc[i] = p.kan_tc[i];
+      t.kd[i] = p.kan_td[i];
+    }
+  }
+  if (tid < B) s[((size_t)(tid >> 1) * ld + D) * 2 + (tid & 1)] = 0.0;  // the padding entries' state
+  if (J.cross == CROSS_GENERAL)
+    for (int i = tid; i < p.Ns * B; i += T)
+      t.ct[i] = p.cross_rowtab[(size_t)row_of(R, i % B) * p.Ns + i / B];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int d = tid + i * p.row_t;
+    if (tid < p.row_t && d < D) {
+#pragma unroll
+      for (int r = 0; r < B; ++r) f.x[i][r] *= o.vs;
+      put_state<B>(s, ld, d, f.x[i]);
+    }
+  }
+  __syncthreads();
+  int bu[B], au[B];
+  double eu[B];
+#pragma unroll
+  for (int r = 0; r < B; ++r) {
+    bu[r] = p.up_bits[R.u[r]];
+    au[r] = bu[r] >> p.nb;
+    eu[r] = p.up_e[R.u[r]];
+  }
+  double dsum = 0.0;
+  // row_t threads of the work-group take the basis states in turn (the
+  // sector's own number, whatever the launch's work-group size)
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int d = tid + i * p.row_t;
+    if (tid < p.row_t && d < D) {
+      double acc[B], x[B], cr[B], wv[B];
+      // the column pass's part and the accumulated input: added last, so that
+      // the gathers do not wait for them
+#pragma unroll
+      for (int r = 0; r < B; ++r) wv[r] = r < R.n ? o.W[(int64_t)R.u[r] * D + d] : 0.0;
+      if (accum) {
+#pragma unroll
+        for (int r = 0; r < B; ++r)
+          if (r < R.n) wv[r] = fma(o.ws, __builtin_nontemporal_load(o.Wp + (int64_t)R.u[r] * D + d), wv[r]);
+      }
+      const int bd = p.dn_bits[d];
+      const double ed = p.dn_e[d];
+#pragma unroll
+      for (int r = 0; r < B; ++r) cr[r] = 0.0;
+      if (J.cross == CROSS_POPC) {
+#pragma unroll
+        for (int r = 0; r < B; ++r) cr[r] = p.cross_u * (double)__builtin_popcount(bu[r] & bd);
+      } else if (J.cross == CROSS_IMP) {
+#pragma unroll
+        for (int r = 0; r < B; ++r) cr[r] = p.cross_imp[au[r] * na + (bd >> p.nb)];
+      } else if (J.cross == CROSS_GENERAL) {
+        // one walk over the state's electrons for all rows
+        for (unsigned m = (unsigned)bd; m; m &= m - 1) {
+          const double* c = t.ct + (size_t)__builtin_ctz(m) * B;
+#pragma unroll
+          for (int r = 0; r < B; ++r) cr[r] += c[r];
+        }
+      }
+      get_state<B>(s, ld, d, x);
+#pragma unroll
+      for (int r = 0; r < B; ++r) acc[r] = (eu[r] + ed + cr[r]) * x[r];
+      gather_line<B, B == 4 && NI == 1 ? 8 : 4>(s, ld, t.vals, p.dn_slptr, p.dn_sllen, p.dn_lell, d, acc);
+      if (J.kan) {
+        if (t.nk) kan_targets<B>(p, t.kc, t.kd, s, ld, au, bd >> p.nb, na, R.n, d, acc);
+        else kan_terms<B>(p, o, R, au, bd >> p.nb, na, d, acc);
+      }
+#pragma unroll
+      for (int r = 0; r < B; ++r)
+        if (r < R.n) {
+          acc[r] += wv[r];
+          __builtin_nontemporal_store(acc[r], o.W + (int64_t)R.u[r] * D + d);
+          dsum = fma(x[r], acc[r], dsum);
+        }
+    }
+    // the next tile's lines behind the first half of this tile's states
+    __builtin_amdgcn_sched_barrier(0);
+    if (more) {
+      if (NI == 1) row_fetch<B, NI>(J, o, tn, f, 0, 1);
+      else if (i < NI / 2) row_fetch<B, NI>(J, o, tn, f, 2 * i, 2 * i + 2);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (J.tdot) block_reduce_store(dsum, s_red, J.tdot + tile);
+  __syncthreads();  // the next tile's lines replace this one's
+}
+
+// B consecutive lanes read the B columns of a row: a load instruction touches
+// 64 / B rows.  Load q of thread t is element q T + t of the D x B tile.
+template <int B, int NI>
+__device__ __forceinline__ void col_fetch(const HvBatchJob& J, const View& o, int c0, Ahead<B, NI>& f, int i0,
+                                          int i1) {
+  const HvParams& p = J.p;
+  const int nc = min(B, p.Ddn - c0);
+  const int c = threadIdx.x % B, row0 = threadIdx.x / B, rstep = p.col_t / B;
+  const double* __restrict__ src = o.V + c0;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    if (i < i0 || i >= i1) continue;
+#pragma unroll
+    for (int r = 0; r < B; ++r) {
+      const int d = row0 + (i * B + r) * rstep;
+      f.x[i][r] = (int)threadIdx.x < p.col_t && d < p.Dup && c < nc ? src[(size_t)d * p.Ddn + c] : 0.0;
+    }
+  }
+}
+
+// LDS of a column tile after its lines: the value table, then 64 x B results
+// per wavefront.
+template <int B, int NI>
+__device__ __forceinline__ void col_tile(const HvBatchJob& J, int c0, bool tables, bool more, int cn,
+                                         Ahead<B, NI>& f, double* s) {
+  const HvParams& p = J.p;
+  const View o = resolve_view(J);
+  const int D = p.Dup, T = blockDim.x;
+  const int tid = fresh_tid();
+  const int ld = D + 1;
+  const int nc = min(B, p.Ddn - c0);
+  const bool accum = o.accum && o.Wp == o.W;
+  double* s_vals = s + (size_t)B * ld;
+  if (tables)
+    for (int i = tid; i < p.nvals; i += T) s_vals[i] = p.values[i];
+  const int c = tid % B;
+  if (tid < B) s[((size_t)(tid >> 1) * ld + D) * 2 + (tid & 1)] = 0.0;  // the padding entries' state
+  {
+    const int row0 = tid / B, rstep = p.col_t / B;
+    double* const sc = s + ((size_t)(c >> 1) * ld * 2 + (c & 1));
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int r = 0; r < B; ++r) {
+        const int d = row0 + (i * B + r) * rstep;
+        if (tid < p.col_t && d < D) sc[(size_t)d * 2] = f.x[i][r] * o.vs;
+      }
+  }
+  __syncthreads();
+  const int lane = tid & 63;
+  double* const t = s_vals + ((p.nvals + 1) & ~1) + (size_t)(tid >> 6) * (64 * B);
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    // whole wavefronts: lanes past the last row work on it again
+    const int d1 = tid + i * p.col_t;
+    if (tid < p.col_t && d1 - lane < D) {
+      const int d = min(d1, D - 1);
+      double acc[B];
+#pragma unroll
+      for (int r = 0; r < B; ++r) acc[r] = accum && r < nc ? o.ws * o.W[(size_t)d * p.Ddn + c0 + r] : 0.0;
+      gather_line<B, B == 4 ? 8 : 4>(s, ld, s_vals, p.up_slptr, p.up_sllen, p.up_lell, d, acc);
+      // the wavefront's 64 x B results turn through its own piece of LDS, so
+      // that B consecutive lanes store the B columns of a row (one request
+      // per row instead of B / 2: the pass is 129 -> 111 us on the 14-site
+      // Kanamori sector)
+#pragma unroll
+      for (int q = 0; q < B / 2; ++q)
+        reinterpret_cast<double2*>(t)[lane * (B / 2) + q] = make_double2(acc[2 * q], acc[2 * q + 1]);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int q = 0; q < B; ++q) {
+        const int l = q * 64 + lane, row = d1 - lane + l / B;
+        if (row < D && c < nc) o.W[(size_t)row * p.Ddn + c0 + c] = t[l];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (more) {
+      if (NI == 1) col_fetch<B, NI>(J, o, cn, f, 0, 1);
+      else if (i < NI / 2) col_fetch<B, NI>(J, o, cn, f, 2 * i, 2 * i + 2);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __syncthreads();  // the next tile's lines replace this one's
+}
+
+struct LinesArgs {
+  HvBatchJob j[kLinesMax];
+};
+
+// Operand blockIdx.y: row tiles blockIdx.x, blockIdx.x + gridDim.x, ...
+template <int B, int NI>
+__global__ __launch_bounds__(1024) void hv_row_lines_kernel(LinesArgs a, int ntiles) {
+  extern __shared__ double s_line[];
+  __shared__ double s_red[16];
+  const HvBatchJob& j = a.j[blockIdx.y];
+  const View o = resolve_view(j);
+  if (!o.live) return;
+  Ahead<B, NI> f;
+  int t = blockIdx.x;
+  if (t < ntiles) row_fetch<B, NI>(j, o, t, f, 0, NI);
+  for (bool first = true; t < ntiles; first = false) {
+    const int n = t + gridDim.x;
+    row_tile<B, NI>(j, t, first, n < ntiles, n, f, s_line, s_red);
+    t = n;
+  }
+}
+
+// Consecutive column tiles share the 128-byte lines of every row: they go to
+// one XCD (work-groups are dealt to the eight XCDs in turn; the grid is a
+// multiple of eight).
+template <int B, int NI>
+__global__ __launch_bounds__(1024) void hv_col_lines_kernel(LinesArgs a, int ntiles, int per) {
+  extern __shared__ double s_line[];
+  const HvBatchJob& j = a.j[blockIdx.y];
+  const View o = resolve_view(j);
+  if (!o.live) return;
+  const int x = blockIdx.x & 7, step = gridDim.x >> 3;
+  const int t1 = min(ntiles, (x + 1) * per);  // this XCD's tiles: [x per, t1)
+  Ahead<B, NI> f;
+  int t = x * per + (blockIdx.x >> 3);
+  if (t < t1) col_fetch<B, NI>(j, o, t * B, f, 0, NI);
+  for (bool first = true; t < t1; first = false) {
+    const int n = t + step;
+    col_tile<B, NI>(j, t * B, first, n < t1, n * B, f, s_line);
+    t = n;
+  }
+}
+
+// Work-groups that stay on the chip for a launch: as many as the CUs hold at
+// this LDS and work-group size, a multiple of eight.
+int stay_grid(int64_t ntiles, int block, size_t smem) {
+  const int per_cu = (int)std::min<size_t>(std::max<size_t>(1, (lds_budget() + 1024) / (smem + 1024)),
+                                           std::max(1, 2048 / block));
+  return (int)std::min<int64_t>((ntiles + 7) / 8 * 8, (int64_t)256 * per_cu);
+}
+
+void allow_lds(const void* k, size_t smem) {
+  if (smem > 64 * 1024)
+    EDH_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+}
+
+size_t pair_up(size_t n) { return (n + 1) & ~size_t(1); }
+
+size_t row_smem(const DevSector& ds, int B) {
+  size_t d = (size_t)B * (ds.dn.D + 1) + (size_t)ds.nvalues;
+  if (ds.row_tiles && B == 4) {
+    const size_t nk = ((size_t)1 << (2 * ds.kan_ml)) * ds.kan_t;
+    d += nk + (nk + 1) / 2;
+  }
+  if (ds.cross_mode == CROSS_GENERAL) d += (size_t)B * ds.Ns;
+  return pair_up(d) * sizeof(double);
+}
+
+size_t col_smem(const DevSector& ds, int B, int block) {
+  return ((size_t)B * (ds.up.D + 1) + pair_up(ds.nvalues) + (size_t)block * B) * sizeof(double);
+}
+
+}  // namespace
+
+// Threads that share a line of D states: as few rounds as 1024 threads
+// allow, split evenly.
+int hv_lines_threads(int64_t D) {
+  const int64_t it = (D + 1023) / 1024;
+  return (int)std::max<int64_t>(64, ((D + it - 1) / std::max<int64_t>(it, 1) + 63) / 64 * 64);
+}
+
+namespace {
+int row_tiles(const DevSector& ds, const HvLinesPlan& L) {
+  return L.row_b == 4 && ds.row_tiles ? ds.n_row_tiles : (int)((ds.up.D + L.row_b - 1) / L.row_b);
+}
+}  // namespace
+
+HvLinesPlan hv_lines_plan(const DevSector& ds) {
+  HvLinesPlan L;
+  L.row_block = hv_lines_threads(ds.dn.D);
+  L.col_block = hv_lines_threads(ds.up.D);
+  const size_t room = lds_budget();
+  for (L.row_b = 4; L.row_b >= 2; L.row_b /= 2)
+    if (ds.dn.D * L.row_b <= 16 * 1024 && (L.row_smem = row_smem(ds, L.row_b)) <= room) break;
+  for (L.col_b = 4; L.col_b >= 2; L.col_b /= 2)
+    if (ds.up.D * L.col_b <= 16 * 1024 && (L.col_smem = col_smem(ds, L.col_b, L.col_block)) <= room) break;
+  L.ok = ds.lines && ds.N > 0 && L.row_b >= 2 && L.col_b >= 2;
+  return L;
+}
+
+int hv_lines_partials(const DevSector& ds) {
+  const HvLinesPlan L = hv_lines_plan(ds);
+  return L.ok ? row_tiles(ds, L) : 0;
+}
+
+// The two passes against the single pass for one operand (MI355X, us per H*v,
+// single pass : lines; hops = mean entries per state of both spins):
+//   12 sites, 853,776 states: 3x4 torus t, t' (52 hops) 29.9 : 21.3, Kanamori
+//     (30) 27.8 : 21.2, 3x4 torus (26) 18.4 : 18.1, Anderson (12) 13.0 : 15.7
+//   13 sites, 2.9 M: Kanamori (32) 100 : 61, Anderson (13) 45.6 : 40.9, ring
+//     (14, signed uniform hopping) 37.6 : 43.2
+//   14 sites, 11.8 M: Kanamori (36) 378 : 203, Anderson (14) 175 : 125, 2x7
+//     torus (23, signed) 185 : 158, ring (15, signed) 141 : 139
+//   15 sites, 41.4 M, two lines at a time: Kanamori (38) 1443 : 1134, Anderson
+//     (15) 651 : 711; 11 sites, 213,444: Kanamori (26) 10.9 : 14.8.
+// Two launches cost about 8 us before they gain, and the single pass's signed
+// form decodes an entry in half the instructions.
+bool hv_lines_faster(const DevSector& ds) {
+  const HvLinesPlan L = hv_lines_plan(ds);
+  if (!L.ok || ds.N < 400000) return false;
+  if (L.row_b < 4 || L.col_b < 4) return ds.hops >= 30;
+  if (ds.N < 2500000) return ds.hops >= 28;
+  return ds.hops >= (ds.dn_signed ? 20 : 12);
+}
+
+void launch_hv_lines(const DevSector& ds, const HvArgs* ops, int count, hipStream_t s) {
+  const HvLinesPlan L = hv_lines_plan(ds);
+  EDH_CHECK(L.ok, EDH_ERR_INTERNAL, "H*v lines: the sector's lines do not fit LDS");
+  EDH_CHECK(count >= 1 && count <= kLinesMax, EDH_ERR_INTERNAL, "H*v lines: operand count");
+  LinesArgs a;
+  for (int q = 0; q < count; ++q) {
+    a.j[q] = make_job(ds, ops[q]);
+    if (ops[q].dot_partial) a.j[q].tdot = ops[q].dot_partial;
+  }
+  for (int q = count; q < kLinesMax; ++q) a.j[q] = a.j[0];
+  const bool r1 = ds.dn.D <= 1024, c1 = ds.up.D <= 1024;
+  auto kr = L.row_b == 2 ? hv_row_lines_kernel<2, 8> : r1 ? hv_row_lines_kernel<4, 1> : hv_row_lines_kernel<4, 4>;
+  auto kc = L.col_b == 2 ? hv_col_lines_kernel<2, 8> : c1 ? hv_col_lines_kernel<4, 1> : hv_col_lines_kernel<4, 4>;
+  allow_lds((const void*)kr, L.row_smem);
+  allow_lds((const void*)kc, L.col_smem);
+  const int ct = (int)((ds.dn.D + L.col_b - 1) / L.col_b), per = (ct + 7) / 8;
+  hipLaunchKernelGGL(kc, dim3(stay_grid(ct, L.col_block, L.col_smem), count), dim3(L.col_block), L.col_smem, s, a, ct,
+                     per);
+  const int rt = row_tiles(ds, L);
+  hipLaunchKernelGGL(kr, dim3(stay_grid(rt, L.row_block, L.row_smem), count), dim3(L.row_block), L.row_smem, s, a, rt);
+  EDH_HIP(hipGetLastError());
+}
+
+}  // namespace edh

@@ -1,0 +1,121 @@
+// Operand and table descriptors shared by the H*v kernels.
+#pragma once
+
+#include "edh_internal.h"
+
+namespace edh {
+
+struct HvParams {
+  int Ns, nb;  // sites per spin, bath bits (Ns - ml) below the impurity bits
+  int Dup, Ddn;
+  const int32_t* row_order;
+  // up spin
+  const int32_t* up_bits;
+  const double* up_e;
+  const int32_t* up_rowp;
+  const uint32_t* up_packed;
+  const int32_t* up_slptr;
+  const int32_t* up_sllen;
+  const uint32_t* up_lell;
+  // down spin
+  const int32_t* dn_bits;
+  const double* dn_e;
+  const int32_t* dn_slptr;
+  const int32_t* dn_sllen;
+  const uint32_t* dn_ell;
+  const uint32_t* dn_lell;
+  const int32_t* dn_q4ptr;
+  const uint64_t* dn_q4;
+  double dn_vt[4];
+  const uint32_t* dn_s4;
+  double dn_s4_scale;
+  const double* values;
+  int nkan;   // impurity terms (staged in LDS by the multi-operand kernel)
+  int nvals;  // entries of values (staged in LDS after the row with EF == 4)
+  // cross term
+  double cross_u;
+  const double* cross_imp;
+  const double* cross_rowtab;
+  // impurity interaction
+  int kan_ml;
+  const int32_t* kan_ptr;
+  const int64_t* kan_off;  // partner state's element offset per term
+  const double* kan_c;
+  int kan_t;  // the same by target pattern, and the row tiles they need (DevSector)
+  const int32_t* row_tiles;
+  const int32_t* kan_td;
+  const double* kan_tc;
+  // operands
+  const double* v;
+  double* w;
+  const double* wprev;
+  double vscale, wscale;
+  int accumulate;
+  double* dot_partial;
+  const double* dscale;
+  const int* done;
+  // slab kernel geometry; off32: every element offset fits 32 bits
+  int nslabs, rows_per_wg, nrb, off32;
+  int row_t, col_t;  // line passes: threads that share a row, a column (hv_lines_threads)
+  int xcd_rows;  // rows kernel: XCD-grouped row assignment (measured 2 % faster on the 16-site sector)
+  // rows kernel in a batch: an eigensolver run's control block (v and w are
+  // then columns col and col + 1 of the basis in v or v_alt; a run whose
+  // state is not 0 is skipped)
+  const double* ctl;
+  const double* v_alt;
+};
+
+template <int CROSS>
+__device__ __forceinline__ double cross_term(const HvParams& p, int u, int bu, int bd, int na) {
+  if (CROSS == CROSS_POPC) return p.cross_u * (double)__builtin_popcount(bu & bd);
+  if (CROSS == CROSS_IMP) return p.cross_imp[(bu >> p.nb) * na + (bd >> p.nb)];
+  if (CROSS == CROSS_GENERAL) {
+    double x = 0.0;
+    const double* r = p.cross_rowtab + (size_t)u * p.Ns;
+    unsigned m = (unsigned)bd;
+    while (m) {
+      int b = __builtin_ctz(m);
+      x += r[b];
+      m &= m - 1;
+    }
+    return x;
+  }
+  return 0.0;
+}
+
+__device__ __forceinline__ void block_reduce_store(double x, double* s_red, double* out) {
+  for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
+  const int wid = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) s_red[wid] = x;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = 0.0;
+    for (int q = 0; q < (int)(blockDim.x >> 6); ++q) t += s_red[q];
+    *out = t;
+  }
+}
+
+// One signed byte-offset slot: a += (+-1) * row[e / 8], the sign in bit 0.
+__device__ __forceinline__ double s4_fma(uint32_t e, const char* sv, double a) {
+  const double sg = __hiloint2double((int)(0x3FF00000u | (e << 31)), 0);
+  return fma(sg, *reinterpret_cast<const double*>(sv + (e & ~1u)), a);
+}
+
+struct HvBatchJob {
+  HvParams p;
+  int64_t row0;
+  int cross, kan;
+  const double* ctl;    // eigensolver control block or null
+  const double* v_alt;  // second basis buffer (with ctl)
+  double* tdot;         // per-task shares of <v, w>, or null
+  const double* lzk;    // Lanczos run's step counter (buffers in rotation) or null
+};
+
+// Fills the descriptor of one operand (hv.hip).
+HvBatchJob make_job(const DevSector& ds, const HvArgs& a);
+
+// Largest dynamic LDS a block may use on the current device, less the
+// static reduction scratch (hv.hip).
+size_t lds_budget();
+
+}  // namespace edh

@@ -50,7 +50,17 @@ class Packer {
   std::vector<std::function<void(char*)>> set_;
 };
 
-void upload_spin(Packer& pk, const SpinTables& sp, DevSpin& d) {
+// The sliced ELL's slots as line-pass entries (kLineOff), padding slots at the
+// zero state after the line.
+std::vector<uint32_t> line_entries(const SpinTables& sp) {
+  std::vector<uint32_t> out(sp.ell.size());
+  for (size_t q = 0; q < out.size(); ++q)
+    out[q] = ((sp.ell_pad[q] ? (uint32_t)sp.D : sp.ell[q] & kColMask) << 4) |
+             ((sp.ell[q] >> kColBits) << (kLineOff + 3));
+  return out;
+}
+
+void upload_spin(Packer& pk, const SpinTables& sp, DevSpin& d, bool lines) {
   d.D = sp.D;
   pk.add(d.bits, sp.bits);
   pk.add(d.ediag, sp.ediag);
@@ -59,7 +69,7 @@ void upload_spin(Packer& pk, const SpinTables& sp, DevSpin& d) {
   pk.add(d.sl_ptr, sp.sl_ptr);
   pk.add(d.sl_len, sp.sl_len);
   pk.add(d.ell, sp.ell);
-  pk.add(d.ell16, sp.ell16);
+  if (lines) pk.add(d.lell, line_entries(sp));
   for (int q = 0; q < 4; ++q) d.vt16[q] = sp.vt16[q];
   d.nvt16 = sp.nvt16;
   pk.add(d.q4_ptr, sp.q4_ptr);
@@ -100,6 +110,63 @@ std::vector<int32_t> rcm_order(const std::vector<int32_t>& rowp, const std::vect
   }
   std::reverse(order.begin(), order.end());
   return order;
+}
+
+// Impurity terms by target and the row tiles they need (DevSector::row_tiles).
+// A run of rows sharing their bath bits has C(ml, k) <= 3 rows for up to
+// three orbitals; a tile takes a run of several rows and fills up with single
+// ones.
+void add_row_tiles(Packer& pk, const SectorTables& st, const std::vector<double>& kc, DevSector& ds) {
+  const int ml = st.kan_ml, na = 1 << ml, nb = ds.Ns - ml;
+  if (ml > 3) return;
+  std::vector<std::vector<int>> tgt(na);
+  int nt = 0;
+  for (int a = 0; a < na; ++a) {
+    for (int q = st.kan_ptr[a * na]; q < st.kan_ptr[(a + 1) * na]; ++q)
+      if (std::find(tgt[a].begin(), tgt[a].end(), st.kan[q].new_a) == tgt[a].end()) tgt[a].push_back(st.kan[q].new_a);
+    nt = std::max(nt, (int)tgt[a].size());
+  }
+  if (nt == 0) return;
+  std::vector<int32_t> td((size_t)na * nt * na, 4);
+  std::vector<double> tc(td.size(), 0.0);
+  for (int a = 0; a < na; ++a)
+    for (int b = 0; b < na; ++b)
+      for (int q = st.kan_ptr[a * na + b]; q < st.kan_ptr[a * na + b + 1]; ++q) {
+        const size_t j = std::find(tgt[a].begin(), tgt[a].end(), st.kan[q].new_a) - tgt[a].begin();
+        const size_t at = ((size_t)a * nt + j) * na + b;
+        if (tc[at] != 0.0) return;  // two terms of (a, b) lead to this up pattern
+        const int32_t lu = (int32_t)((1ll << (st.nup - __builtin_popcount(a))) - 1);
+        const int32_t ld = (int32_t)((1ll << (st.ndn - __builtin_popcount(b))) - 1);
+        const int du = st.up.rank[lu | (st.kan[q].new_a << nb)] - st.up.rank[lu | (a << nb)];
+        const int dd = st.dn.rank[ld | (st.kan[q].new_b << nb)] - st.dn.rank[ld | (b << nb)];
+        if (du < -2 || du > 2) return;
+        td[at] = 8 * dd + 4 + du;
+        tc[at] = kc[q];
+      }
+  // runs of rows with the same bath bits
+  const int32_t bath = (int32_t)((1ll << nb) - 1);
+  std::vector<int32_t> single, tiles;
+  for (int64_t u = 0; u < st.up.D;) {
+    int64_t e = u + 1;
+    while (e < st.up.D && (st.up.bits[e] & bath) == (st.up.bits[u] & bath)) ++e;
+    if (e - u > 4) return;
+    if (e - u == 1) {
+      single.push_back((int32_t)u);
+    } else {
+      for (int k = 0; k < 4; ++k) tiles.push_back(u + k < e ? (int32_t)(u + k) : -1);
+    }
+    u = e;
+  }
+  size_t next = 0;
+  for (int32_t& t : tiles)
+    if (t < 0 && next < single.size()) t = single[next++];
+  while (next < single.size())
+    for (int k = 0; k < 4; ++k) tiles.push_back(next < single.size() ? single[next++] : -1);
+  ds.kan_t = nt;
+  ds.n_row_tiles = (int)(tiles.size() / 4);
+  pk.add(ds.row_tiles, tiles);
+  pk.add(ds.kan_td, td);
+  pk.add(ds.kan_tc, tc);
 }
 
 }  // namespace
@@ -165,10 +232,20 @@ void upload_sector(const SectorTables& st, int Ns, DevSector& ds, hipStream_t s,
   ds.imp_ml = st.imp_ml;
   ds.table_bytes = st.table_bytes;
   Packer pk;
-  upload_spin(pk, st.up, ds.up);
-  upload_spin(pk, st.dn, ds.dn);
-  pk.add(ds.values, st.values);
   ds.nvalues = (int)st.values.size();
+  ds.hops = (double)st.up.col.size() / (double)std::max<int64_t>(st.up.D, 1) +
+            (double)st.dn.col.size() / (double)std::max<int64_t>(st.dn.D, 1);
+  ds.up.D = st.up.D;
+  ds.dn.D = st.dn.D;
+  ds.dn_signed = !st.dn.ell_s4.empty();
+  // the line passes' tables: in a batch where its Lanczos operands take them,
+  // for a single sector (no stage) wherever they apply, since the caller may
+  // ask for that variant
+  ds.lines = std::max(st.up.D, st.dn.D) < (1 << (kLineOff - 4)) - 1;
+  if (stage) ds.lines = st.N >= kLinesLanczos && hv_lines_faster(ds);
+  upload_spin(pk, st.up, ds.up, ds.lines);
+  upload_spin(pk, st.dn, ds.dn, ds.lines);
+  pk.add(ds.values, st.values);
   ds.cross_mode = st.cross_mode;
   ds.cross_u = st.cross_u;
   pk.add(ds.cross_imp, st.cross_imp);
@@ -206,6 +283,7 @@ void upload_sector(const SectorTables& st, int Ns, DevSector& ds, hipStream_t s,
     pk.add(ds.kan_off, koff);
     pk.add(ds.kan_c, kc);
     ds.nkan = (int)kc.size();
+    if (ds.lines) add_row_tiles(pk, st, kc, ds);
   }
   pk.add(ds.counters, std::vector<int32_t>(64, 0));
   pk.add(ds.row_order, rcm_order(st.up.rowp, st.up.col, st.up.D));
