@@ -57,6 +57,7 @@ Ctx::~Ctx() {
   small.release();
   gtab.release();
   obs.release();
+  if (pin) (void)hipHostFree(pin);
   if (stream) {
     (void)hipStreamSynchronize(stream);  // the tables return to the pool in stream order
     (void)hipStreamDestroy(stream);
@@ -509,87 +510,57 @@ namespace {
 int lanczos_device(Ctx& c, int nl, double* alpha, double* beta, double* step_ms) {
   const int64_t n = c.tabs.N;
   hipStream_t s = c.stream;
-  const int nblk = std::max(hv_num_blocks(c.dev), kMaxPartials);
-  c.partial.ensure((size_t)std::max(nblk, kMaxPartials * kMaxBasis) * sizeof(double));
-  c.scal.ensure((size_t)(8 + 2 * nl + 2) * sizeof(double));
-  double* sc = c.scal.as<double>();
-  int* st = (int*)(sc + 4);
-  double* dalpha = sc + 8;
+  if (n == 0) {  // beta_1 = 0 stops the recurrence
+    std::fill(alpha, alpha + nl, 0.0);
+    std::fill(beta, beta + nl + 1, 0.0);
+    if (step_ms) *step_ms = 0.0;
+    return 1;
+  }
+  const int ndot = hv_num_blocks(c.dev), nshare = lanczos_update_grid(n);
+  c.partial.ensure((size_t)(ndot + nshare) * sizeof(double));
+  double* dot = c.partial.as<double>();
+  double* share = dot + ndot;
+  // {stop state, alpha[nl], beta[nl + 1]} (read back in one copy), scale[nl + 1]
+  const size_t nres = 1 + (size_t)nl + (size_t)nl + 1;
+  c.scal.ensure((nres + (size_t)nl + 1) * sizeof(double));
+  double* res = c.scal.as<double>();
+  int* st = (int*)res;
+  double* dalpha = res + 1;
   double* dbeta = dalpha + nl;
-  EDH_HIP(hipMemsetAsync(dalpha, 0, (size_t)(2 * nl + 1) * sizeof(double), s));
-  dev_lanczos_init(sc, st, s);
-  double* cur = c.lz[0].as<double>();
-  double* prev = c.lz[1].as<double>();
-  double* out = c.lz[2].as<double>();
-  double* partial = c.partial.as<double>();
+  double* scale = dbeta + nl + 1;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (step_ms) {
     EDH_HIP(hipEventCreate(&e0));
     EDH_HIP(hipEventCreate(&e1));
     EDH_HIP(hipEventRecord(e0, s));
   }
-  // One Lanczos step = H*v with the alpha partial sums, the alpha reduction,
-  // then axpy + norm and the beta reduction; every scalar and the step number
-  // live on the device.  The step is captured once per buffer rotation
-  // (period 3) as a hipGraph and replayed; EDH_LANCZOS_GRAPH=0 launches the
-  // kernels directly instead.
-  auto step = [&](double* cu, double* pr, double* ou, int k) {
+  // One Lanczos step = H*v with the shares of alpha, then the update with
+  // the shares of |w|^2; the scalars stay on the device, and the host issues
+  // every step without waiting (kernels of a stopped run return at once).
+  double* cur = c.lz[0].as<double>();
+  double* prev = c.lz[1].as<double>();
+  double* out = c.lz[2].as<double>();
+  for (int k = 1; k <= nl; ++k) {
     HvArgs a{};
-    a.v = cu;
-    a.w = ou;
-    a.wprev = pr;
-    a.mode = 1;  // step 1: the w scale is 0 and the previous vector is zeroed
-    a.dscale = sc;
-    a.dot_partial = partial;
-    a.done = st + 1;
+    a.v = cur;
+    a.w = out;
+    a.wprev = prev;
+    a.mode = k > 1 ? 1 : 0;
+    a.dot_partial = dot;
+    a.step.k = k;
+    a.step.write = 1;
+    a.step.nl = nl;
+    a.step.nshare = nshare;
+    a.step.share = share;
+    a.step.scale = scale;
+    a.step.beta = dbeta;
+    a.step.st = st;
     launch_hv(c.dev, a, s);
-    dev_lanczos_alpha(partial, hv_num_blocks(c.dev), dalpha, k, sc, st, s);
-    dev_lanczos_passB(ou, cu, sc + 2, n, partial, st + 1, dbeta, k, nl, sc, st, s);
-  };
-  dev_fill(prev, n, 0.0, s);
-  const char* genv = getenv("EDH_LANCZOS_GRAPH");
-  const bool use_graph = nl >= 4 && !(genv && genv[0] == '0');
-  bool graphed = false;
-  // executable graphs are destroyed only after the stream has drained: HIP
-  // does not defer the destruction of an exec whose launches still run
-  hipGraphExec_t ex[3] = {nullptr, nullptr, nullptr};
-  if (use_graph) {
-    double* rot[3] = {cur, prev, out};
-    bool ok = true;
-    for (int ph = 0; ph < 3 && ok; ++ph) {
-      hipGraph_t g = nullptr;
-      if (hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed) != hipSuccess) {
-        ok = false;
-        break;
-      }
-      // phase ph: (cur, prev, out) = rotation^ph of the three buffers
-      step(rot[(3 - ph) % 3], rot[(4 - ph) % 3], rot[(5 - ph) % 3], 0);
-      if (hipStreamEndCapture(s, &g) != hipSuccess || !g) {
-        ok = false;
-        break;
-      }
-      if (hipGraphInstantiate(&ex[ph], g, nullptr, nullptr, 0) != hipSuccess) ok = false;
-      (void)hipGraphDestroy(g);
-    }
-    if (ok) {
-      for (int k = 1; k <= nl; ++k) EDH_HIP(hipGraphLaunch(ex[(k - 1) % 3], s));
-      graphed = true;
-    } else {
-      for (auto& e : ex) {
-        if (e) (void)hipGraphExecDestroy(e);
-        e = nullptr;
-      }
-    }
-    (void)hipGetLastError();
-  }
-  if (!graphed) {
-    for (int k = 1; k <= nl; ++k) {
-      step(cur, prev, out, k);
-      double* t = prev;
-      prev = cur;
-      cur = out;
-      out = t;
-    }
+    dev_lanczos_update(out, cur, n, dot, ndot, scale, dalpha, st, k, share, s);
+    double* t = prev;
+    prev = cur;
+    cur = out;
+    out = t;
   }
   if (step_ms) {
     EDH_HIP(hipEventRecord(e1, s));
@@ -600,15 +571,16 @@ int lanczos_device(Ctx& c, int nl, double* alpha, double* beta, double* step_ms)
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
   }
+  double* h = c.pinned(nres);
+  EDH_HIP(hipMemcpyAsync(h, res, nres * sizeof(double), hipMemcpyDeviceToHost, s));
+  EDH_HIP(hipStreamSynchronize(s));
   int host_st[2];
-  EDH_HIP(hipMemcpyAsync(alpha, dalpha, nl * sizeof(double), hipMemcpyDeviceToHost, s));
-  EDH_HIP(hipMemcpyAsync(beta, dbeta, (nl + 1) * sizeof(double), hipMemcpyDeviceToHost, s));
-  EDH_HIP(hipMemcpyAsync(host_st, st, sizeof(host_st), hipMemcpyDeviceToHost, s));
-  const hipError_t se = hipStreamSynchronize(s);
-  for (auto& e : ex)
-    if (e) (void)hipGraphExecDestroy(e);
-  EDH_HIP(se);
-  return host_st[0];
+  std::memcpy(host_st, h, sizeof(host_st));
+  const int taken = host_st[0];
+  // alpha_1..alpha_taken, beta_1..beta_taken (beta_nl is not stored, Lanczos.h:64)
+  for (int q = 0; q < nl; ++q) alpha[q] = q < taken ? h[1 + q] : 0.0;
+  for (int q = 0; q <= nl; ++q) beta[q] = q >= 1 && q <= taken && q < nl ? h[1 + nl + q] : 0.0;
+  return taken;
 }
 
 }  // namespace
@@ -739,22 +711,24 @@ int edh_cf_eval(edh_ctx* ctx, int nz, const double* zre, const double* zim, doub
   Ctx& c = ctx->c;
   use_device(c);
   EDH_CHECK(nz >= 0 && nlanc >= 1 && zre && zim && alpha && beta && out_re && out_im, EDH_ERR_ARG, "bad argument");
-  const size_t need = (size_t)(4 * nz + 2 * nlanc + 2) * sizeof(double);
-  c.small.ensure(need);
+  if (nz == 0) return EDH_OK;
+  // points and coefficients go up in one copy, the values come back in one
+  const size_t nin = 2 * (size_t)nz + 2 * (size_t)nlanc + 1, nout = 2 * (size_t)nz;
+  c.small.ensure((nin + nout) * sizeof(double));
   double* dz = c.small.as<double>();
-  double* dzi = dz + nz;
-  double* da = dzi + nz;
-  double* db = da + nlanc;
-  double* dr = db + nlanc + 1;
-  double* di = dr + nz;
-  EDH_HIP(hipMemcpyAsync(dz, zre, nz * 8, hipMemcpyHostToDevice, c.stream));
-  EDH_HIP(hipMemcpyAsync(dzi, zim, nz * 8, hipMemcpyHostToDevice, c.stream));
-  EDH_HIP(hipMemcpyAsync(da, alpha, nlanc * 8, hipMemcpyHostToDevice, c.stream));
-  EDH_HIP(hipMemcpyAsync(db, beta, (nlanc + 1) * 8, hipMemcpyHostToDevice, c.stream));
-  dev_cf_eval(nz, dz, dzi, ev, nlanc, isign, expb, da, db, dr, di, c.stream);
-  EDH_HIP(hipMemcpyAsync(out_re, dr, nz * 8, hipMemcpyDeviceToHost, c.stream));
-  EDH_HIP(hipMemcpyAsync(out_im, di, nz * 8, hipMemcpyDeviceToHost, c.stream));
+  double* da = dz + 2 * (size_t)nz;
+  double* dr = dz + nin;
+  double* h = c.pinned(nin + nout);
+  std::copy(zre, zre + nz, h);
+  std::copy(zim, zim + nz, h + nz);
+  std::copy(alpha, alpha + nlanc, h + 2 * (size_t)nz);
+  std::copy(beta, beta + nlanc + 1, h + 2 * (size_t)nz + nlanc);
+  EDH_HIP(hipMemcpyAsync(dz, h, nin * sizeof(double), hipMemcpyHostToDevice, c.stream));
+  dev_cf_eval(nz, dz, dz + nz, ev, nlanc, isign, expb, da, da + nlanc, dr, dr + nz, c.stream);
+  EDH_HIP(hipMemcpyAsync(h + nin, dr, nout * sizeof(double), hipMemcpyDeviceToHost, c.stream));
   EDH_HIP(hipStreamSynchronize(c.stream));
+  std::copy(h + nin, h + nin + nz, out_re);
+  std::copy(h + nin + nz, h + nin + nout, out_im);
   API_END
 }
 

@@ -48,6 +48,20 @@ struct Ctx {
   DevBuf gtab;              // gather tables for a_adag / operators
   DevBuf obs;               // static-observable row sums and column tiles
   int n_evecs = 0;
+  // pinned host memory for small reads and writes (one call at a time uses it)
+  double* pin = nullptr;
+  size_t pin_count = 0;
+  double* pinned(size_t count) {
+    if (count > pin_count) {
+      if (pin) EDH_HIP(hipHostFree(pin));
+      pin = nullptr;
+      pin_count = 0;
+      const size_t cap = count < 4096 ? 4096 : count;
+      EDH_HIP(hipHostMalloc((void**)&pin, cap * sizeof(double)));
+      pin_count = cap;
+    }
+    return pin;
+  }
   ~Ctx();
 };
 

@@ -247,6 +247,23 @@ void upload_sector(const SectorTables& st, int Ns, DevSector& ds, hipStream_t s,
 // solve loops costs no driver call and no device-wide wait.
 void configure_mem_pool(int device);
 
+// One step k of a single-sector Lanczos run (Lanczos.h:47-65) as its H*v sees
+// it.  The step before left the shares of |W_k|^2 (W_k: the vector, not
+// normalised); every work-group sums them for beta_{k-1} and takes the scales
+// {1 / beta_{k-1}, -beta_{k-1} / beta_{k-2}} from it, so no launch of its own
+// is needed for them; the first work-group of the step's first launch
+// (`write`) records beta and the scale, or the stop at |beta| < 1e-10.
+struct LzStep {
+  int k = 0;      // 1-based; 0: not a Lanczos step
+  int write = 0;  // this launch records
+  int nl = 0;
+  int nshare = 0;
+  const double* share = nullptr;  // shares of |W_k|^2 (k > 1)
+  double* scale = nullptr;        // scale[k]: of W_k
+  double* beta = nullptr;         // beta[k - 1]
+  int* st = nullptr;              // {steps taken, stopped}
+};
+
 // H*v launch parameters.
 struct HvArgs {
   const double* v;      // gathered operand (scaled by vscale on load)
@@ -272,6 +289,7 @@ struct HvArgs {
   // w = b[(r + 2) % 3] with r = (3 - (k - 1) % 3) % 3, accumulating wprev
   // from the second step on (the buffer rotation of Lanczos.h:47-51)
   const double* lzk = nullptr;
+  LzStep step;  // a step of a single-sector run (then vscale, wscale, dscale, done are not read)
 };
 
 // Buffer of a Lanczos run's three in rotation at step k >= 1: role 0 = the

@@ -27,10 +27,13 @@ void dev_orthogonalize(const double* V, int64_t ldv, int m, double* w, int64_t n
 // Y[:, j] = sum_i C[i + j*m] V[:, i]  (C on the device, column-major m x k)
 void dev_combine(const double* V, int64_t ldv, int m, const double* C, int k, double* Y, int64_t ldy, int64_t n,
                  hipStream_t s);
-void dev_lanczos_init(double* sc, int* st, hipStream_t s);
-void dev_lanczos_alpha(const double* partial, int n, double* alpha, int k, double* sc, const int* st, hipStream_t s);
-void dev_lanczos_passB(double* w, const double* x, const double* coef, int64_t n, double* partial, const int* done,
-                       double* beta, int k, int nl, double* sc, int* st, hipStream_t s);
+// Second half of a single-sector Lanczos step (see LzStep): w -= alpha_k x
+// scale[k] with alpha_k from the H*v's ndot shares, and lanczos_update_grid(n)
+// shares of |w|^2.  w and x 16-byte aligned.
+constexpr int kLzShares = 512;
+int lanczos_update_grid(int64_t n);
+void dev_lanczos_update(double* w, const double* x, int64_t n, const double* dot, int ndot, const double* scale,
+                        double* alpha, const int* st, int k, double* share, hipStream_t s);
 
 // Green's-function helpers (gf.hip)
 void dev_separable_gather(const double* in, int64_t ldin, const int32_t* mu, const int32_t* md, const int8_t* su,

@@ -53,78 +53,78 @@ __device__ __forceinline__ cplx cdiv(cplx a, cplx b) {
   return {(a.re * r + a.im) / den, (a.im * r - a.re) / den};
 }
 
-__global__ void cf_kernel(int nz, const double* zre, const double* zim, double ev, int nlanc, int isign, double expb,
-                          const double* alpha, const double* beta, double* out_re, double* out_im) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nz) return;
-  const cplx z = {zre[q], zim[q]};
+// |d| > big without the overflow-safe hypot where the larger part decides
+// (its cost was most of a recurrence step).
+__device__ __forceinline__ bool exceeds(cplx d, double big) {
+  const double m = fmax(fabs(d.re), fabs(d.im));
+  if (m > big) return true;
+  return m > 0.5 * big && hypot(d.re, d.im) > big;
+}
+
+// Lanczos.h:201-224 at the point z.
+__device__ __forceinline__ cplx fraction(cplx z, int n, int isign, double weight, const double* alpha,
+                                         const double* beta) {
   const double big = (double)FLT_MAX / 2.0;
   const double shift = 1.0 / ((double)FLT_MAX / 1000.0);
-  cplx res;
-  if (nlanc == 1) {
-    const cplx dl0 = {z.re - alpha[0] * isign, z.im};
-    res = cdiv({ev * expb, 0.0}, dl0);
-  } else {
-    const int n = nlanc;
-    const cplx dl1 = {z.re - alpha[n - 1] * isign, z.im};
-    const cplx dl2 = {z.re - alpha[n - 2] * isign, z.im};
-    cplx dA = dl1;                                                    // det[i+2]
-    cplx dB = csub(cmul(dl2, dl1), {beta[n - 1] * beta[n - 1], 0.0});  // det[i+1]
-    for (int i = n - 3; i >= 0; --i) {
-      const cplx dli = {z.re - alpha[i] * isign, z.im};
-      const double b2 = beta[i + 1] * beta[i + 1];
-      cplx d = csub(cmul(dli, dB), cscale(dA, b2));
-      if (hypot(d.re, d.im) > big && i != 0) {
-        d = cscale(d, shift);
-        dB = cscale(dB, shift);
-      }
-      dA = dB;
-      dB = d;
+  if (n == 1) return cdiv({weight, 0.0}, {z.re - alpha[0] * isign, z.im});
+  const cplx dl1 = {z.re - alpha[n - 1] * isign, z.im};
+  const cplx dl2 = {z.re - alpha[n - 2] * isign, z.im};
+  cplx dA = dl1;                                                    // det[i+2]
+  cplx dB = csub(cmul(dl2, dl1), {beta[n - 1] * beta[n - 1], 0.0});  // det[i+1]
+  for (int i = n - 3; i >= 0; --i) {
+    const cplx dli = {z.re - alpha[i] * isign, z.im};
+    const double b2 = beta[i + 1] * beta[i + 1];
+    cplx d = csub(cmul(dli, dB), cscale(dA, b2));
+    if (exceeds(d, big) && i != 0) {
+      d = cscale(d, shift);
+      dB = cscale(dB, shift);
     }
-    res = cdiv(cscale(dA, ev * expb), dB);
+    dA = dB;
+    dB = d;
   }
+  return cdiv(cscale(dA, weight), dB);
+}
+
+// Coefficients of up to kCfLds steps are staged in LDS: the recurrence is a
+// serial chain, and a global read per step was the longest part of it.
+constexpr int kCfLds = 1024;
+
+__device__ __forceinline__ cplx fraction_staged(bool live, cplx z, int n, int isign, double weight,
+                                                const double* alpha, const double* beta, double* s_ab) {
+  if (n > kCfLds) return live ? fraction(z, n, isign, weight, alpha, beta) : z;
+  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    s_ab[i] = alpha[i];
+    s_ab[n + i] = beta[i];
+  }
+  __syncthreads();
+  return live ? fraction(z, n, isign, weight, s_ab, s_ab + n) : z;
+}
+
+__global__ __launch_bounds__(64) void cf_kernel(int nz, const double* zre, const double* zim, double ev, int nlanc,
+                                                int isign, double expb, const double* alpha, const double* beta,
+                                                double* out_re, double* out_im) {
+  __shared__ double s_ab[2 * kCfLds];
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  const int at = min(q, nz - 1);
+  const cplx res = fraction_staged(q < nz, {zre[at], zim[at]}, nlanc, isign, ev * expb, alpha, beta, s_ab);
+  if (q >= nz) return;
   out_re[q] = res.re;
   out_im[q] = res.im;
 }
 
 // Many continued fractions at once: block row j evaluates job j at the
-// points z = excited_j * isign_j + i wn[q] (the same recurrence as cf_kernel).
-__global__ void cf_batch_kernel(int nz, const double* wr, const double* wn, const CfJob* jobs, double* out_re,
-                                double* out_im) {
+// points z = excited_j * isign_j + i wn[q].
+__global__ __launch_bounds__(64) void cf_batch_kernel(int nz, const double* wr, const double* wn, const CfJob* jobs,
+                                                      double* out_re, double* out_im) {
+  __shared__ double s_ab[2 * kCfLds];
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  const int at = min(q, nz - 1);
   const CfJob& J = jobs[blockIdx.y];
-  if (q >= nz) return;
   // z = freq_point + isign * E (Lanczos.h:146-148): i w_n on the Matsubara
   // mesh (wr null), w + i pi/beta on the real axis
-  const cplx z = {(wr ? wr[q] : 0.0) + J.excited * J.isign, wn[q]};
-  const double big = (double)FLT_MAX / 2.0;
-  const double shift = 1.0 / ((double)FLT_MAX / 1000.0);
-  const double* alpha = J.alpha;
-  const double* beta = J.beta;
-  const int isign = J.isign;
-  cplx res;
-  if (J.nlanc == 1) {
-    const cplx dl0 = {z.re - alpha[0] * isign, z.im};
-    res = cdiv({J.ev * J.expb, 0.0}, dl0);
-  } else {
-    const int n = J.nlanc;
-    const cplx dl1 = {z.re - alpha[n - 1] * isign, z.im};
-    const cplx dl2 = {z.re - alpha[n - 2] * isign, z.im};
-    cplx dA = dl1;
-    cplx dB = csub(cmul(dl2, dl1), {beta[n - 1] * beta[n - 1], 0.0});
-    for (int i = n - 3; i >= 0; --i) {
-      const cplx dli = {z.re - alpha[i] * isign, z.im};
-      const double b2 = beta[i + 1] * beta[i + 1];
-      cplx d = csub(cmul(dli, dB), cscale(dA, b2));
-      if (hypot(d.re, d.im) > big && i != 0) {
-        d = cscale(d, shift);
-        dB = cscale(dB, shift);
-      }
-      dA = dB;
-      dB = d;
-    }
-    res = cdiv(cscale(dA, J.ev * J.expb), dB);
-  }
+  const cplx z = {(wr ? wr[at] : 0.0) + J.excited * J.isign, wn[at]};
+  const cplx res = fraction_staged(q < nz, z, J.nlanc, J.isign, J.ev * J.expb, J.alpha, J.beta, s_ab);
+  if (q >= nz) return;
   out_re[(size_t)blockIdx.y * nz + q] = res.re;
   out_im[(size_t)blockIdx.y * nz + q] = res.im;
 }
@@ -132,7 +132,7 @@ __global__ void cf_batch_kernel(int nz, const double* wr, const double* wn, cons
 void dev_cf_batch(int njobs, int nz, const double* wr, const double* wn, const CfJob* jobs, double* out_re,
                   double* out_im, hipStream_t s) {
   if (njobs <= 0 || nz <= 0) return;
-  hipLaunchKernelGGL(cf_batch_kernel, dim3((nz + 127) / 128, njobs), dim3(128), 0, s, nz, wr, wn, jobs, out_re,
+  hipLaunchKernelGGL(cf_batch_kernel, dim3((nz + 63) / 64, njobs), dim3(64), 0, s, nz, wr, wn, jobs, out_re,
                      out_im);
   EDH_HIP(hipGetLastError());
 }
@@ -156,7 +156,7 @@ void dev_separable_scale(const double* in, const double* fu, const double* fd, d
 void dev_cf_eval(int nz, const double* zre, const double* zim, double ev, int nlanc, int isign, double expb,
                  const double* alpha, const double* beta, double* out_re, double* out_im, hipStream_t s) {
   if (nz <= 0) return;
-  hipLaunchKernelGGL(cf_kernel, dim3((nz + 255) / 256), dim3(256), 0, s, nz, zre, zim, ev, nlanc, isign, expb, alpha,
+  hipLaunchKernelGGL(cf_kernel, dim3((nz + 63) / 64), dim3(64), 0, s, nz, zre, zim, ev, nlanc, isign, expb, alpha,
                      beta, out_re, out_im);
   EDH_HIP(hipGetLastError());
 }

@@ -69,9 +69,8 @@ __global__ __launch_bounds__(1024) void hv_rows_kernel(HvParams p) {
   const int tid = threadIdx.x;
   const int Ddn = p.Ddn;
   const int na = 1 << (p.Ns - p.nb);
-  if (p.done && *p.done) return;
-  const double vscale = p.dscale ? p.dscale[0] : p.vscale;
-  const double wscale = p.dscale ? p.dscale[1] : p.wscale;
+  double vscale, wscale;
+  if (!hv_scales(p, s_red, blockIdx.x == 0, vscale, wscale)) return;
   const double* __restrict__ V = p.v;
   double* __restrict__ W = p.w;
   if (CTL) {
@@ -622,8 +621,8 @@ __global__ __launch_bounds__(kSlabWG) void hv_upslab_kernel(HvParams p, int* cou
   __shared__ int s_item;
   __shared__ uint32_t s_off[kSlabEnt];
   __shared__ double s_val[kSlabEnt];
-  if (p.done && *p.done) return;
-  const double vscale = p.dscale ? p.dscale[0] : p.vscale;
+  double vscale, wscale;
+  if (!hv_scales(p, s_red, false, vscale, wscale)) return;
   unsigned xcc;
   asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
   const int home = (int)(xcc & (kXcd - 1));
@@ -1022,6 +1021,7 @@ HvParams make_params(const DevSector& ds, const HvArgs& a) {
   p.dot_partial = a.dot_partial;
   p.dscale = a.dscale;
   p.done = a.done;
+  p.lz = a.step;
   slab_geometry(ds, p.nslabs, p.rows_per_wg, p.nrb);
   p.off32 = (uint64_t)ds.N < (uint64_t(1) << 32);
   p.row_t = hv_lines_threads(ds.dn.D);

@@ -45,14 +45,14 @@ struct View {
   bool accum, live;
 };
 
-__device__ __forceinline__ View resolve_view(const HvBatchJob& J) {
+__device__ __forceinline__ View resolve_view(const HvBatchJob& J, double* s_red, bool first) {
   const HvParams& p = J.p;
   View o;
   o.V = p.v;
   o.W = p.w;
   o.Wp = p.wprev;
   o.accum = p.accumulate != 0;
-  o.live = !(p.done && *p.done);
+  o.live = hv_scales(p, s_red, first, o.vs, o.ws);
   if (J.ctl) {  // eigensolver run: its basis column and buffer
     if (J.ctl[kCtlState] != 0.0) o.live = false;
     const int64_t N = (int64_t)p.Dup * p.Ddn;
@@ -69,8 +69,6 @@ __device__ __forceinline__ View resolve_view(const HvBatchJob& J) {
     o.W = const_cast<double*>(r2 == 0 ? b[0] : (r2 == 1 ? b[1] : b[2]));
     o.accum = k > 1;
   }
-  o.vs = p.dscale ? p.dscale[0] : p.vscale;
-  o.ws = p.dscale ? p.dscale[1] : p.wscale;
   return o;
 }
 
@@ -265,10 +263,9 @@ __device__ __forceinline__ void row_fetch(const HvBatchJob& J, const View& o, in
 // One row tile whose lines are in f; the next tile's (tn, when there are more)
 // are fetched into f on the way.
 template <int B, int NI>
-__device__ __forceinline__ void row_tile(const HvBatchJob& J, int tile, bool tables, bool more, int tn,
+__device__ __forceinline__ void row_tile(const HvBatchJob& J, const View& o, int tile, bool tables, bool more, int tn,
                                          Ahead<B, NI>& f, double* s, double* s_red) {
   const HvParams& p = J.p;
-  const View o = resolve_view(J);
   const int D = p.Ddn, T = blockDim.x;
   const int tid = fresh_tid();
   const int ld = D + 1;
@@ -393,10 +390,9 @@ __device__ __forceinline__ void col_fetch(const HvBatchJob& J, const View& o, in
 // LDS of a column tile after its lines: the value table, then 64 x B results
 // per wavefront.
 template <int B, int NI>
-__device__ __forceinline__ void col_tile(const HvBatchJob& J, int c0, bool tables, bool more, int cn,
+__device__ __forceinline__ void col_tile(const HvBatchJob& J, const View& o, int c0, bool tables, bool more, int cn,
                                          Ahead<B, NI>& f, double* s) {
   const HvParams& p = J.p;
-  const View o = resolve_view(J);
   const int D = p.Dup, T = blockDim.x;
   const int tid = fresh_tid();
   const int ld = D + 1;
@@ -468,14 +464,14 @@ __global__ __launch_bounds__(1024) void hv_row_lines_kernel(LinesArgs a, int nti
   extern __shared__ double s_line[];
   __shared__ double s_red[16];
   const HvBatchJob& j = a.j[blockIdx.y];
-  const View o = resolve_view(j);
+  const View o = resolve_view(j, s_red, false);
   if (!o.live) return;
   Ahead<B, NI> f;
   int t = blockIdx.x;
   if (t < ntiles) row_fetch<B, NI>(j, o, t, f, 0, NI);
   for (bool first = true; t < ntiles; first = false) {
     const int n = t + gridDim.x;
-    row_tile<B, NI>(j, t, first, n < ntiles, n, f, s_line, s_red);
+    row_tile<B, NI>(j, o, t, first, n < ntiles, n, f, s_line, s_red);
     t = n;
   }
 }
@@ -486,8 +482,9 @@ __global__ __launch_bounds__(1024) void hv_row_lines_kernel(LinesArgs a, int nti
 template <int B, int NI>
 __global__ __launch_bounds__(1024) void hv_col_lines_kernel(LinesArgs a, int ntiles, int per) {
   extern __shared__ double s_line[];
+  __shared__ double s_red[16];
   const HvBatchJob& j = a.j[blockIdx.y];
-  const View o = resolve_view(j);
+  const View o = resolve_view(j, s_red, blockIdx.x == 0);
   if (!o.live) return;
   const int x = blockIdx.x & 7, step = gridDim.x >> 3;
   const int t1 = min(ntiles, (x + 1) * per);  // this XCD's tiles: [x per, t1)
@@ -496,7 +493,7 @@ __global__ __launch_bounds__(1024) void hv_col_lines_kernel(LinesArgs a, int nti
   if (t < t1) col_fetch<B, NI>(j, o, t * B, f, 0, NI);
   for (bool first = true; t < t1; first = false) {
     const int n = t + step;
-    col_tile<B, NI>(j, t * B, first, n < t1, n * B, f, s_line);
+    col_tile<B, NI>(j, o, t * B, first, n < t1, n * B, f, s_line);
     t = n;
   }
 }

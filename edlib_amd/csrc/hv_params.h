@@ -54,6 +54,7 @@ struct HvParams {
   double* dot_partial;
   const double* dscale;
   const int* done;
+  LzStep lz;
   // slab kernel geometry; off32: every element offset fits 32 bits
   int nslabs, rows_per_wg, nrb, off32;
   int row_t, col_t;  // line passes: threads that share a row, a column (hv_lines_threads)
@@ -93,6 +94,57 @@ __device__ __forceinline__ void block_reduce_store(double x, double* s_red, doub
     for (int q = 0; q < (int)(blockDim.x >> 6); ++q) t += s_red[q];
     *out = t;
   }
+}
+
+// Sum of n shares, the same value on every thread: thread t takes shares t,
+// t + T, ... in order, then a fixed tree per wavefront and the wavefronts in
+// order.
+__device__ __forceinline__ double block_all_sum(const double* share, int n, double* s_red) {
+  double x = 0.0;
+  for (int i = threadIdx.x; i < n; i += blockDim.x) x += share[i];
+  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+  __syncthreads();  // s_red may still be read from an earlier use
+  if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = x;
+  __syncthreads();
+  double t = 0.0;
+  for (int q = 0; q < (int)(blockDim.x >> 6); ++q) t += s_red[q];
+  return t;
+}
+
+// Scales of an operand; false: the launch does nothing (uniform over the
+// work-group, s_red: one double per wavefront).
+__device__ __forceinline__ bool hv_scales(const HvParams& p, double* s_red, bool first, double& vs, double& ws) {
+  if (p.lz.k == 0) {
+    if (p.done && *p.done) return false;
+    vs = p.dscale ? p.dscale[0] : p.vscale;
+    ws = p.dscale ? p.dscale[1] : p.wscale;
+    return true;
+  }
+  const bool write = first && p.lz.write && threadIdx.x == 0;
+  if (p.lz.k == 1) {
+    vs = 1.0;
+    ws = 0.0;
+    if (write) {
+      p.lz.scale[1] = 1.0;
+      p.lz.st[0] = p.lz.nl;
+      p.lz.st[1] = 0;
+    }
+    return true;
+  }
+  if (p.lz.st[1]) return false;
+  const double beta = sqrt(block_all_sum(p.lz.share, p.lz.nshare, s_red));
+  const bool stop = fabs(beta) < 1e-10;
+  vs = 1.0 / beta;
+  ws = -beta * p.lz.scale[p.lz.k - 1];
+  if (write) {
+    p.lz.beta[p.lz.k - 1] = beta;
+    p.lz.scale[p.lz.k] = vs;
+    if (stop) {
+      p.lz.st[0] = p.lz.k - 1;
+      p.lz.st[1] = 1;
+    }
+  }
+  return !stop;
 }
 
 // One signed byte-offset slot: a += (+-1) * row[e / 8], the sign in bit 0.

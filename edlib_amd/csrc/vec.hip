@@ -5,6 +5,7 @@
 // fixed order.
 #include "edh_internal.h"
 #include "edh_kernels.h"
+#include "hv_params.h"
 
 namespace edh {
 
@@ -37,66 +38,58 @@ __global__ void reduce_partials_kernel(const double* partial, int n, double* out
   if (threadIdx.x == 0) *out = take_sqrt ? sqrt(t) : t;
 }
 
-// w += (*coef) * x ; partial of |w|^2.  Skipped once the recurrence stopped.
-__global__ void axpy_norm_kernel(double* w, const double* x, const double* coef, int64_t n, double* partial,
-                                 const int* done) {
-  __shared__ double s_red[16];
-  if (done && *done) return;
-  const double c = *coef;
-  double acc = 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    double y = fma(c, x[i], w[i]);
-    w[i] = y;
-    acc = fma(y, y, acc);
-  }
-  double t = block_sum(acc, s_red);
-  if (threadIdx.x == 0) partial[blockIdx.x] = t;
-}
-
-// Lanczos bookkeeping (Lanczos.h:55-65).  sc[0] = scale of the current
-// operand (v_k = s_k W_k), sc[1] = additive scale for the next step,
-// sc[2] = pass-B coefficient (-alpha_k s_k).  st[0] = steps taken, st[1] = stop.
-// k <= 0: the step number is read on the device (st[0] + 1), so one launch
-// sequence serves every step (hipGraph replay).
-__global__ void lanczos_alpha_kernel(const double* partial, int n, double* alpha, int k, double* sc, const int* st) {
+// Second half of Lanczos step k (Lanczos.h:56-60) of a single-sector run:
+// alpha_k = the sum of the H*v's shares of <v, w>, formed by every block from
+// the same shares in the same order, then w -= alpha_k v_k (stored as x with
+// scale[k]) and the blocks' shares of |w|^2, from which the next step's H*v
+// takes beta_k.  Two launches a step: the reductions that used to take a
+// launch each read at most a few hundred numbers.
+__global__ __launch_bounds__(kVecBlock) void lanczos_update_kernel(double* __restrict__ w, const double* __restrict__ x,
+                                                                   int64_t n, const double* __restrict__ dot, int ndot,
+                                                                   const double* __restrict__ scale, double* alpha,
+                                                                   const int* __restrict__ st, int k,
+                                                                   double* __restrict__ share) {
   __shared__ double s_red[16];
   if (st[1]) return;
-  if (k <= 0) k = st[0] + 1;
-  double acc = 0.0;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) acc += partial[i];
-  double t = block_sum(acc, s_red);
-  if (threadIdx.x == 0) {
-    alpha[k - 1] = t;
-    sc[2] = -t * sc[0];
+  const double a = block_all_sum(dot, ndot, s_red);
+  if (blockIdx.x == 0 && threadIdx.x == 0) alpha[k - 1] = a;
+  const double c = -a * scale[k];
+  const int64_t step = (int64_t)gridDim.x * blockDim.x, n2 = n >> 1;
+  double2* w2 = reinterpret_cast<double2*>(w);
+  const double2* x2 = reinterpret_cast<const double2*>(x);
+  double s0 = 0.0, s1 = 0.0;
+  int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  for (; i + step < n2; i += 2 * step) {
+    const double2 p = x2[i], q = x2[i + step];
+    double2 y = w2[i], z = w2[i + step];
+    y.x = fma(c, p.x, y.x);
+    y.y = fma(c, p.y, y.y);
+    z.x = fma(c, q.x, z.x);
+    z.y = fma(c, q.y, z.y);
+    w2[i] = y;
+    w2[i + step] = z;
+    s0 = fma(y.x, y.x, s0);
+    s1 = fma(y.y, y.y, s1);
+    s0 = fma(z.x, z.x, s0);
+    s1 = fma(z.y, z.y, s1);
   }
-}
-
-__global__ void lanczos_beta_kernel(const double* partial, int n, double* beta, int k, int nl, double* sc, int* st) {
-  __shared__ double s_red[16];
-  if (st[1]) return;
-  if (k <= 0) k = st[0] + 1;
-  double acc = 0.0;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) acc += partial[i];
-  double t = block_sum(acc, s_red);
-  if (threadIdx.x == 0) {
-    const double bet = sqrt(t);
-    if (k != nl) beta[k] = bet;
-    st[0] = k;
-    if (fabs(bet) < 1e-10) {
-      st[1] = 1;
-    } else {
-      sc[1] = -bet * sc[0];
-      sc[0] = 1.0 / bet;
-    }
+  if (i < n2) {
+    const double2 p = x2[i];
+    double2 y = w2[i];
+    y.x = fma(c, p.x, y.x);
+    y.y = fma(c, p.y, y.y);
+    w2[i] = y;
+    s0 = fma(y.x, y.x, s0);
+    s1 = fma(y.y, y.y, s1);
   }
-}
-
-__global__ void lanczos_init_kernel(double* sc, int* st) {
-  sc[0] = 1.0;
-  sc[1] = 0.0;
-  sc[2] = 0.0;
-  st[0] = 0;
-  st[1] = 0;
+  if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
+    const double y = fma(c, x[n - 1], w[n - 1]);
+    w[n - 1] = y;
+    s0 = fma(y, y, s0);
+  }
+  __syncthreads();  // s_red is read by block_all_sum's callers until here
+  const double t = block_sum(s0 + s1, s_red);
+  if (threadIdx.x == 0) share[blockIdx.x] = t;
 }
 
 // ---- Gram-Schmidt against a block of basis vectors (eigensolver) ----------
@@ -311,21 +304,16 @@ void dev_combine(const double* V, int64_t ldv, int m, const double* C, int k, do
   EDH_HIP(hipGetLastError());
 }
 
-void dev_lanczos_init(double* sc, int* st, hipStream_t s) {
-  hipLaunchKernelGGL(lanczos_init_kernel, dim3(1), dim3(1), 0, s, sc, st);
-  EDH_HIP(hipGetLastError());
+int lanczos_update_grid(int64_t n) {
+  // four elements a thread, at most 512 blocks (their shares are summed by
+  // every work-group of the next H*v)
+  return (int)std::min<int64_t>(std::max<int64_t>((n + 4 * kVecBlock - 1) / (4 * kVecBlock), 1), kLzShares);
 }
 
-void dev_lanczos_alpha(const double* partial, int n, double* alpha, int k, double* sc, const int* st, hipStream_t s) {
-  hipLaunchKernelGGL(lanczos_alpha_kernel, dim3(1), dim3(kVecBlock), 0, s, partial, n, alpha, k, sc, st);
-  EDH_HIP(hipGetLastError());
-}
-
-void dev_lanczos_passB(double* w, const double* x, const double* coef, int64_t n, double* partial, const int* done,
-                       double* beta, int k, int nl, double* sc, int* st, hipStream_t s) {
-  int g = reduce_grid(n);
-  hipLaunchKernelGGL(axpy_norm_kernel, dim3(g), dim3(kVecBlock), 0, s, w, x, coef, n, partial, done);
-  hipLaunchKernelGGL(lanczos_beta_kernel, dim3(1), dim3(kVecBlock), 0, s, partial, g, beta, k, nl, sc, st);
+void dev_lanczos_update(double* w, const double* x, int64_t n, const double* dot, int ndot, const double* scale,
+                        double* alpha, const int* st, int k, double* share, hipStream_t s) {
+  hipLaunchKernelGGL(lanczos_update_kernel, dim3(lanczos_update_grid(n)), dim3(kVecBlock), 0, s, w, x, n, dot, ndot,
+                     scale, alpha, st, k, share);
   EDH_HIP(hipGetLastError());
 }
 
