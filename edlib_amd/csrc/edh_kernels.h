@@ -17,16 +17,17 @@ void dev_fill(double* p, int64_t n, double x, hipStream_t s);  // a kernel, neve
 // Random start vector: uniform [-1, 1) from splitmix64 (seed 0 -> a fixed
 // default), the same values as the sequential host generator.
 void dev_random_uniform(double* x, int64_t n, uint64_t seed, hipStream_t s);
-// w <- w - V V^T w (one classical Gram-Schmidt pass over m columns); h = V^T w
-// (device, m), hsum += h when non-null; *nrm = |w| afterwards (device scalar).
-// nb: also *nb = |w| before the pass; gate: the pass does nothing when *gate
-// is 0; gate_out: *gate_out = 1 when |w| after < 0.717 |w| before (DGKS).
-void dev_orthogonalize(const double* V, int64_t ldv, int m, double* w, int64_t n, double* partial, double* h,
-                       double* hsum, double* nrm, hipStream_t s, double* nb = nullptr, const double* gate = nullptr,
-                       double* gate_out = nullptr);
-// Y[:, j] = sum_i C[i + j*m] V[:, i]  (C on the device, column-major m x k)
-void dev_combine(const double* V, int64_t ldv, int m, const double* C, int k, double* Y, int64_t ldy, int64_t n,
-                 hipStream_t s);
+// Column cnt of V (n rows each) made orthogonal to columns 0..cnt-1 and
+// normalised (see gs_dots_kernel): hcol[0..cnt) = its projections, *nrm = its
+// norm before the normalisation (NaN: repeat with exact); part: 2 (cnt + 1)
+// gs_grid(n) doubles.
+constexpr int kGsShares = 512;
+int gs_grid(int64_t n);
+void dev_orthonormalize(double* V, int64_t n, int cnt, double* part, double* hcol, double* nrm, bool exact,
+                        hipStream_t s);
+// Y[:, j] = sum_i C[i + j*m] V[:, i]  (C on the device, column-major m x k);
+// last: Y[:, k] = V[:, m] too
+void dev_combine(const double* V, int64_t n, int m, const double* C, int k, double* Y, bool last, hipStream_t s);
 // Second half of a single-sector Lanczos step (see LzStep): w -= alpha_k x
 // scale[k] with alpha_k from the H*v's ndot shares, and lanczos_update_grid(n)
 // shares of |w|^2.  w and x 16-byte aligned.

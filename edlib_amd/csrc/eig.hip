@@ -218,14 +218,16 @@ void eigsh_run(Ctx& c, int nev_req, int ncv_req, double tol, int maxitr, uint64_
   const size_t vbytes = (size_t)n * sizeof(double);
   c.krylov[0].ensure((size_t)(m + 1) * vbytes);
   c.krylov[1].ensure((size_t)(m + 1) * vbytes);
-  c.partial.ensure((size_t)kMaxPartials * kMaxBasis * sizeof(double));
-  // device scalars: hsum columns (m x (m+1)), norms (m+1), h scratch
-  c.small.ensure((size_t)(m * (m + 1) + (m + 1) + kMaxBasis + kMaxBasis * kMaxBasis + 2) * sizeof(double));
+  c.partial.ensure((size_t)std::max(2 * kMaxBasis * kGsShares, kMaxPartials) * sizeof(double));
+  // device scalars: projection columns (m x (m+1)) and norms (m+1), read back
+  // in one copy at a cycle end, then the combination's coefficients
+  const size_t nT = (size_t)m * (m + 1) + (m + 1);
+  c.small.ensure((nT + (size_t)kMaxBasis * kMaxBasis) * sizeof(double));
   double* Tcol = c.small.as<double>();             // column j at Tcol + j*(m+1)
   double* norms = Tcol + (size_t)m * (m + 1);      // norm after orthogonalising column j
-  double* hs = norms + (m + 1);                    // scratch h
-  double* Cdev = hs + kMaxBasis;                   // combine coefficients
-  double* dgks = Cdev + kMaxBasis * kMaxBasis;     // norm before the first pass, second-pass gate
+  double* Cdev = Tcol + nT;                        // combine coefficients
+  double* const h_T = c.pinned(nT + (size_t)kMaxBasis * kMaxBasis);
+  double* const h_C = h_T + nT;
   double* V = c.krylov[0].as<double>();
   double* Valt = c.krylov[1].as<double>();
   double* partial = c.partial.as<double>();
@@ -236,11 +238,11 @@ void eigsh_run(Ctx& c, int nev_req, int ncv_req, double tol, int maxitr, uint64_
     dev_norm(V, n, partial, norms + m, s);
     dev_scale_inv(V, norms + m, V, n, s);
   }
-  std::vector<double> T((size_t)m * m, 0.0), Tc((size_t)m * (m + 1)), nr(m + 1), theta, Y;
+  std::vector<double> T((size_t)m * m, 0.0), theta, Y;
   int k = 0;  // kept Ritz vectors at the start of the cycle
   const double eps23 = std::pow(std::numeric_limits<double>::epsilon(), 2.0 / 3.0);
+  bool exact = false;  // the exact form of the orthogonalisation from here on
   for (int iter = 0;; ++iter) {
-    EDH_HIP(hipMemsetAsync(Tcol, 0, (size_t)m * (m + 1) * sizeof(double), s));
     for (int j = k; j < m; ++j) {
       double* vj = V + (size_t)j * n;
       double* w = V + (size_t)(j + 1) * n;
@@ -251,21 +253,24 @@ void eigsh_run(Ctx& c, int nev_req, int ncv_req, double tol, int maxitr, uint64_
       a.mode = 0;
       launch_hv(c.dev, a, s);
       ++*n_av;
-      double* hcol = Tcol + (size_t)j * (m + 1);
-      // classical Gram-Schmidt, repeated only when the DGKS test asks for it
-      dev_orthogonalize(V, n, j + 1, w, n, partial, hs, hcol, norms + j, s, dgks, nullptr, dgks + 1);
-      dev_orthogonalize(V, n, j + 1, w, n, partial, hs, hcol, norms + j, s, nullptr, dgks + 1, nullptr);
-      dev_scale_inv(w, norms + j, w, n, s);
+      dev_orthonormalize(V, n, j + 1, partial, Tcol + (size_t)j * (m + 1), norms + j, exact, s);
     }
-    EDH_HIP(hipMemcpyAsync(Tc.data(), Tcol, Tc.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-    EDH_HIP(hipMemcpyAsync(nr.data(), norms, (m + 1) * sizeof(double), hipMemcpyDeviceToHost, s));
+    EDH_HIP(hipMemcpyAsync(h_T, Tcol, nT * sizeof(double), hipMemcpyDeviceToHost, s));
     EDH_HIP(hipStreamSynchronize(s));
+    if (!exact && std::any_of(h_T + (size_t)m * (m + 1) + k, h_T + (size_t)m * (m + 1) + m,
+                              [](double x) { return std::isnan(x); })) {
+      // an invariant subspace: columns 0..k are as they were, so the cycle
+      // can be run again
+      exact = true;
+      --iter;
+      continue;
+    }
     for (int j = k; j < m; ++j)
       for (int i = 0; i <= j; ++i) {
-        T[(size_t)i * m + j] = Tc[(size_t)j * (m + 1) + i];
-        T[(size_t)j * m + i] = Tc[(size_t)j * (m + 1) + i];
+        T[(size_t)i * m + j] = h_T[(size_t)j * (m + 1) + i];
+        T[(size_t)j * m + i] = h_T[(size_t)j * (m + 1) + i];
       }
-    const double bres = nr[m - 1];
+    const double bres = h_T[(size_t)m * (m + 1) + m - 1];
     std::vector<double> A = T;
     sym_eig(m, A, theta);
     Y = A;  // columns = eigenvectors of T
@@ -280,13 +285,12 @@ void eigsh_run(Ctx& c, int nev_req, int ncv_req, double tol, int maxitr, uint64_
       // Like dsaupd/dseupd after maxitr (info = 1, Storage.h:94-129): the
       // converged Ritz pairs are returned and nconv says how many there are.
       const int nk = nconv_now;
-      std::vector<double> Cm((size_t)m * std::max(nk, 1));
       for (int q = 0; q < nk; ++q)
-        for (int i = 0; i < m; ++i) Cm[(size_t)q * m + i] = Y[(size_t)i * m + done_i[q]];
+        for (int i = 0; i < m; ++i) h_C[(size_t)q * m + i] = Y[(size_t)i * m + done_i[q]];
       if (nk > 0) {
-        EDH_HIP(hipMemcpyAsync(Cdev, Cm.data(), (size_t)m * nk * sizeof(double), hipMemcpyHostToDevice, s));
+        EDH_HIP(hipMemcpyAsync(Cdev, h_C, (size_t)m * nk * sizeof(double), hipMemcpyHostToDevice, s));
         c.evecs.ensure((size_t)nk * vbytes);
-        dev_combine(V, n, m, Cdev, nk, c.evecs.as<double>(), n, n, s);
+        dev_combine(V, n, m, Cdev, nk, c.evecs.as<double>(), false, s);
         if (evecs_host)
           EDH_HIP(hipMemcpyAsync(evecs_host, c.evecs.p, (size_t)nk * vbytes, hipMemcpyDeviceToHost, s));
       }
@@ -298,12 +302,11 @@ void eigsh_run(Ctx& c, int nev_req, int ncv_req, double tol, int maxitr, uint64_
     }
     // thick restart: keep kk lowest Ritz vectors, continue from the residual
     const int kk = restart_size(nev, m, nconv_now);
-    std::vector<double> Cm((size_t)m * kk);
+    // (the coefficients' last reader has run: the copy of T came after it)
     for (int j = 0; j < kk; ++j)
-      for (int i = 0; i < m; ++i) Cm[(size_t)j * m + i] = Y[(size_t)i * m + j];
-    EDH_HIP(hipMemcpyAsync(Cdev, Cm.data(), Cm.size() * sizeof(double), hipMemcpyHostToDevice, s));
-    dev_combine(V, n, m, Cdev, kk, Valt, n, n, s);
-    EDH_HIP(hipMemcpyAsync(Valt + (size_t)kk * n, V + (size_t)m * n, vbytes, hipMemcpyDeviceToDevice, s));
+      for (int i = 0; i < m; ++i) h_C[(size_t)j * m + i] = Y[(size_t)i * m + j];
+    EDH_HIP(hipMemcpyAsync(Cdev, h_C, (size_t)m * kk * sizeof(double), hipMemcpyHostToDevice, s));
+    dev_combine(V, n, m, Cdev, kk, Valt, true, s);
     std::swap(V, Valt);
     std::fill(T.begin(), T.end(), 0.0);
     for (int i = 0; i < kk; ++i) {

@@ -92,107 +92,249 @@ __global__ __launch_bounds__(kVecBlock) void lanczos_update_kernel(double* __res
   if (threadIdx.x == 0) share[blockIdx.x] = t;
 }
 
-// ---- Gram-Schmidt against a block of basis vectors (eigensolver) ----------
-// A pass is skipped when a gate is given and reads 0 (ARPACK dsaitr's DGKS
-// rule: the second pass runs only when the first one removed more than
-// 1 - 0.717 of the norm).
-__device__ __forceinline__ bool gated_off(const double* gate) { return gate && *gate == 0.0; }
+// ---- Gram-Schmidt of a new basis vector (eigensolver) ----------------------
+// w (column cnt of V) against columns 0..cnt-1 by classical Gram-Schmidt, a
+// second pass where ARPACK dsaitr's DGKS test asks for it (the first pass
+// left less than 0.717 of the norm), and the normalisation, in three launches:
+//   dots:    shares of h = V^T w and |w|^2
+//   update:  w -= V h, and from the same registers the shares of s = V^T w
+//            and |w|^2
+//   finish:  w = (w - V s) / nrm where the test asks for it, else w / nrm,
+//            with nrm^2 = |w|^2 - |s|^2 (exact up to rounding: |s| << |w|)
+// Where the second pass takes a good part of what the first one left (the
+// basis spans an invariant subspace and w is rounding noise) that difference
+// is no norm: *nrm is then NaN, and the caller repeats the cycle in the exact
+// form, which measures |w - V s| and scales in a fourth launch.
+// A block's shares are sums over its tiles; every block of the next launch
+// sums all of them itself, each the same numbers in the same order, so the
+// reductions take no launch of their own.  Ten launches a step (two passes of
+// dots, reduction, update, norm; scaling; H*v) became four; on 213,444 states
+// with a basis of 11 the eight of them that are not H*v took 103 us, these
+// three take 23.5 us.
+constexpr int kGsBlock = 512;   // threads
+constexpr int kGsElems = 2;     // elements per thread and tile
+constexpr int kGsTile = kGsBlock * kGsElems;
+constexpr int kGsGroup = 12;    // columns held in registers together (NCV = 11 in one group)
+constexpr int kGsWaves = kGsBlock / 64;
 
-// h_partial[blk * ld + i] = sum_e V[i][e] w[e] for i < m (m <= kMaxBasis);
-// with_nb: slot m of each block holds sum_e w[e]^2 (ld = m + 1, else m)
-__global__ void multi_dot_kernel(const double* V, int64_t ldv, int m, const double* w, int64_t n, double* partial,
-                                 int with_nb, const double* gate) {
-  __shared__ double s_acc[kMaxBasis + 1][16];
-  if (gated_off(gate)) return;
-  double acc[kMaxBasis];
-  double nb = 0.0;
-#pragma unroll
-  for (int i = 0; i < kMaxBasis; ++i) acc[i] = 0.0;
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
-    const double we = w[e];
-#pragma unroll
-    for (int i = 0; i < kMaxBasis; ++i)
-      if (i < m) acc[i] = fma(V[i * ldv + e], we, acc[i]);
-    if (with_nb) nb = fma(we, we, nb);
-  }
-  const int wid = threadIdx.x >> 6;
-#pragma unroll
-  for (int i = 0; i < kMaxBasis; ++i) {
-    if (i >= m) break;
-    double x = acc[i];
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
-    if ((threadIdx.x & 63) == 0) s_acc[i][wid] = x;
-  }
-  if (with_nb) {
-    double x = nb;
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
-    if ((threadIdx.x & 63) == 0) s_acc[m][wid] = x;
+// Sums of cnt values' shares (value i of block b at part[i * G + b]) into
+// s_h, a value per wavefront at a time.
+__device__ __forceinline__ void gs_sums(const double* __restrict__ part, int G, int cnt, double* s_h) {
+  const int lane = threadIdx.x & 63;
+  for (int i = threadIdx.x >> 6; i < cnt; i += kGsWaves) {
+    double t = 0.0;
+    for (int b = lane; b < G; b += 64) t += part[(size_t)i * G + b];
+    for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+    if (lane == 0) s_h[i] = t;
   }
   __syncthreads();
-  const int ld = m + (with_nb ? 1 : 0);
-  for (int i = threadIdx.x; i < ld; i += blockDim.x) {
+}
+
+// Block sums of acc[0..n) into part[(i0 + g) * G + block].
+template <int K>
+__device__ __forceinline__ void gs_store(const double (&acc)[K], int n, int i0, int G, double (*s_p)[K], double* part) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int g = 0; g < K; ++g) {
+    if (g >= n) break;
+    double x = acc[g];
+    for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
+    if (lane == 0) s_p[wave][g] = x;
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < n) {
     double t = 0.0;
-    for (int q = 0; q < (int)(blockDim.x >> 6); ++q) t += s_acc[i][q];
-    partial[blockIdx.x * (int64_t)ld + i] = t;
+    for (int q = 0; q < kGsWaves; ++q) t += s_p[q][threadIdx.x];
+    part[(size_t)(i0 + threadIdx.x) * G + blockIdx.x] = t;
+  }
+  __syncthreads();
+}
+
+// Columns i0 + g < cnt of V, then w itself (slot cnt), at element e.
+template <int K>
+__device__ __forceinline__ void gs_load(const double* __restrict__ V, int64_t ldv, int i0, int cnt, int64_t e,
+                                        double (&x)[K]) {
+#pragma unroll
+  for (int g = 0; g < K; ++g) x[g] = i0 + g < cnt ? V[(int64_t)(i0 + g) * ldv + e] : 0.0;
+}
+
+__global__ __launch_bounds__(kGsBlock) void gs_dots_kernel(const double* __restrict__ V, int64_t n, int cnt,
+                                                           double* __restrict__ part) {
+  __shared__ double s_p[kGsWaves][kGsGroup];
+  const int G = gridDim.x;
+  // the group's columns and, in the slot after the last one, w
+  for (int i0 = 0; i0 <= cnt; i0 += kGsGroup) {
+    double acc[kGsGroup];
+#pragma unroll
+    for (int g = 0; g < kGsGroup; ++g) acc[g] = 0.0;
+    for (int64_t e0 = (int64_t)blockIdx.x * kGsTile; e0 < n; e0 += (int64_t)G * kGsTile) {
+      double x[kGsElems][kGsGroup], we[kGsElems];
+#pragma unroll
+      for (int u = 0; u < kGsElems; ++u) {
+        const int64_t e = e0 + u * kGsBlock + threadIdx.x;
+        we[u] = e < n ? V[(int64_t)cnt * n + e] : 0.0;
+        gs_load<kGsGroup>(V, n, i0, e < n ? cnt + 1 : 0, e, x[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < kGsElems; ++u)
+#pragma unroll
+        for (int g = 0; g < kGsGroup; ++g) acc[g] = fma(x[u][g], we[u], acc[g]);
+    }
+    gs_store<kGsGroup>(acc, min(kGsGroup, cnt + 1 - i0), i0, G, s_p, part);
   }
 }
 
-// h[i] = sum over blocks of partial[blk*ld + i]; also accumulates into hsum
-// if given; with_nb: *nb = sqrt of the sum of slot m.
-__global__ void multi_reduce_kernel(const double* partial, int nblk, int m, double* h, double* hsum, int with_nb,
-                                    double* nb, const double* gate) {
-  __shared__ double s_red[16];
-  if (gated_off(gate)) return;
-  const int ld = m + (with_nb ? 1 : 0);
-  for (int i = 0; i < ld; ++i) {
-    double acc = 0.0;
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) acc += partial[b * (int64_t)ld + i];
-    double t = block_sum(acc, s_red);
-    if (threadIdx.x == 0) {
-      if (i < m) {
-        h[i] = t;
-        if (hsum) hsum[i] += t;
-      } else {
-        *nb = sqrt(t);
+// ONE: the basis fits one group, so the columns stay in registers from the
+// update to the projections; else they are read again.
+template <bool ONE>
+__global__ __launch_bounds__(kGsBlock) void gs_update_kernel(double* __restrict__ V, int64_t n, int cnt,
+                                                             const double* __restrict__ part1,
+                                                             double* __restrict__ part2, double* __restrict__ hcol) {
+  __shared__ double s_h[kMaxBasis + kGsGroup];
+  __shared__ double s_p[kGsWaves][kGsGroup + 1];
+  const int G = gridDim.x;
+  for (int i = threadIdx.x; i < kMaxBasis + kGsGroup; i += kGsBlock) s_h[i] = 0.0;
+  __syncthreads();
+  gs_sums(part1, G, cnt, s_h);
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < cnt; i += kGsBlock) hcol[i] = s_h[i];
+  double* __restrict__ w = V + (int64_t)cnt * n;
+  if (ONE) {
+    double acc[kGsGroup + 1];
+#pragma unroll
+    for (int g = 0; g <= kGsGroup; ++g) acc[g] = 0.0;
+    for (int64_t e0 = (int64_t)blockIdx.x * kGsTile; e0 < n; e0 += (int64_t)G * kGsTile) {
+      double x[kGsElems][kGsGroup], y[kGsElems];
+#pragma unroll
+      for (int u = 0; u < kGsElems; ++u) {
+        const int64_t e = e0 + u * kGsBlock + threadIdx.x;
+        y[u] = e < n ? w[e] : 0.0;
+        gs_load<kGsGroup>(V, n, 0, e < n ? cnt : 0, e, x[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < kGsElems; ++u) {
+        const int64_t e = e0 + u * kGsBlock + threadIdx.x;
+#pragma unroll
+        for (int g = 0; g < kGsGroup; ++g) y[u] = fma(-s_h[g], x[u][g], y[u]);
+        if (e < n) w[e] = y[u];
+#pragma unroll
+        for (int g = 0; g < kGsGroup; ++g) acc[g] = fma(x[u][g], y[u], acc[g]);
+        acc[kGsGroup] = fma(y[u], y[u], acc[kGsGroup]);
       }
     }
-    __syncthreads();
+    double v[kGsGroup + 1];
+#pragma unroll
+    for (int g = 0; g <= kGsGroup; ++g) v[g] = g < cnt ? acc[g < kGsGroup ? g : 0] : (g == cnt ? acc[kGsGroup] : 0.0);
+    gs_store<kGsGroup + 1>(v, cnt + 1, 0, G, s_p, part2);
+    return;
+  }
+  for (int64_t e0 = (int64_t)blockIdx.x * kGsTile; e0 < n; e0 += (int64_t)G * kGsTile)
+#pragma unroll
+    for (int u = 0; u < kGsElems; ++u) {
+      const int64_t e = e0 + u * kGsBlock + threadIdx.x;
+      if (e >= n) continue;
+      double y = w[e];
+      for (int i0 = 0; i0 < cnt; i0 += kGsGroup) {
+        double x[kGsGroup];
+        gs_load<kGsGroup>(V, n, i0, cnt, e, x);
+#pragma unroll
+        for (int g = 0; g < kGsGroup; ++g) y = fma(-s_h[i0 + g], x[g], y);
+      }
+      w[e] = y;
+    }
+  // a thread reads back only what it wrote
+  for (int i0 = 0; i0 <= cnt; i0 += kGsGroup) {
+    double acc[kGsGroup + 1];
+#pragma unroll
+    for (int g = 0; g <= kGsGroup; ++g) acc[g] = 0.0;
+    for (int64_t e0 = (int64_t)blockIdx.x * kGsTile; e0 < n; e0 += (int64_t)G * kGsTile)
+#pragma unroll
+      for (int u = 0; u < kGsElems; ++u) {
+        const int64_t e = e0 + u * kGsBlock + threadIdx.x;
+        if (e >= n) continue;
+        double x[kGsGroup];
+        const double y = w[e];
+        gs_load<kGsGroup>(V, n, i0, cnt, e, x);
+#pragma unroll
+        for (int g = 0; g < kGsGroup; ++g) acc[g] = fma(i0 + g == cnt ? y : x[g], y, acc[g]);
+      }
+    gs_store<kGsGroup + 1>(acc, min(kGsGroup, cnt + 1 - i0), i0, G, s_p, part2);
   }
 }
 
-// w -= sum_i h[i] V[i]; optional partial of |w|^2
-__global__ void multi_axpy_kernel(const double* V, int64_t ldv, int m, const double* h, double* w, int64_t n,
-                                  double* partial, const double* gate) {
-  __shared__ double s_h[kMaxBasis];
-  __shared__ double s_red[16];
-  if (gated_off(gate)) return;
-  for (int i = threadIdx.x; i < m; i += blockDim.x) s_h[i] = h[i];
+// EXACT: w = w - V s, unscaled, and the shares of its norm in part1.
+template <bool EXACT>
+__global__ __launch_bounds__(kGsBlock) void gs_finish_kernel(double* __restrict__ V, int64_t n, int cnt,
+                                                             double* part1,
+                                                             const double* __restrict__ part2,
+                                                             double* __restrict__ hcol, double* __restrict__ nrm_out) {
+  __shared__ double s_h[kMaxBasis + kGsGroup];
+  __shared__ double s_nb[1];
+  __shared__ double s_p[kGsWaves][1];
+  const int G = gridDim.x;
+  for (int i = threadIdx.x; i < kMaxBasis + kGsGroup; i += kGsBlock) s_h[i] = 0.0;
   __syncthreads();
-  double acc = 0.0;
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
-    double x = w[e];
-    for (int i = 0; i < m; ++i) x = fma(-s_h[i], V[i * ldv + e], x);
-    w[e] = x;
-    acc = fma(x, x, acc);
+  gs_sums(part2, G, cnt + 1, s_h);
+  gs_sums(part1 + (size_t)cnt * G, G, 1, s_nb);
+  const double n2 = s_h[cnt], nrm1 = sqrt(n2);
+  const bool again = nrm1 < 0.717 * sqrt(s_nb[0]);
+  double nrm = nrm1;
+  if (again) {
+    double ss = 0.0;
+    for (int i = 0; i < cnt; ++i) ss = fma(s_h[i], s_h[i], ss);
+    nrm = ss <= 0.25 * n2 ? sqrt(n2 - ss) : __builtin_nan("");
   }
-  if (partial) {
-    double t = block_sum(acc, s_red);
-    if (threadIdx.x == 0) partial[blockIdx.x] = t;
+  if (blockIdx.x == 0) {
+    if (again)
+      for (int i = threadIdx.x; i < cnt; i += kGsBlock) hcol[i] += s_h[i];
+    if (!EXACT && threadIdx.x == 0) *nrm_out = nrm;
   }
+  __syncthreads();
+  if (threadIdx.x == 0) s_h[cnt] = 0.0;  // the norm's slot is a column's coefficient below
+  __syncthreads();
+  const double f = EXACT ? 1.0 : 1.0 / nrm;
+  double acc[1] = {0.0};
+  double* __restrict__ w = V + (int64_t)cnt * n;
+  for (int64_t e0 = (int64_t)blockIdx.x * kGsTile; e0 < n; e0 += (int64_t)G * kGsTile) {
+    double y[kGsElems];
+#pragma unroll
+    for (int u = 0; u < kGsElems; ++u) {
+      const int64_t e = e0 + u * kGsBlock + threadIdx.x;
+      y[u] = e < n ? w[e] : 0.0;
+    }
+    if (again)
+      for (int i0 = 0; i0 < cnt; i0 += kGsGroup) {
+        double x[kGsElems][kGsGroup];
+#pragma unroll
+        for (int u = 0; u < kGsElems; ++u) {
+          const int64_t e = e0 + u * kGsBlock + threadIdx.x;
+          gs_load<kGsGroup>(V, n, i0, e < n ? cnt : 0, e, x[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kGsElems; ++u)
+#pragma unroll
+          for (int g = 0; g < kGsGroup; ++g) y[u] = fma(-s_h[i0 + g], x[u][g], y[u]);
+      }
+#pragma unroll
+    for (int u = 0; u < kGsElems; ++u) {
+      const int64_t e = e0 + u * kGsBlock + threadIdx.x;
+      if (e < n) w[e] = y[u] * f;
+      acc[0] = fma(y[u], y[u], acc[0]);
+    }
+  }
+  // (slot cnt of part1, which other blocks may still be reading, is not used)
+  if (EXACT) gs_store<1>(acc, 1, 0, G, s_p, part1);
 }
 
-// *nrm = sqrt(sum of the partials); gate_out: *gate_out = (*nrm < 0.717 *nb)
-__global__ void ortho_norm_kernel(const double* partial, int n, double* nrm, const double* nb, double* gate_out,
-                                  const double* gate) {
-  __shared__ double s_red[16];
-  if (gated_off(gate)) return;
-  double acc = 0.0;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) acc += partial[i];
-  double t = block_sum(acc, s_red);
-  if (threadIdx.x == 0) {
-    *nrm = sqrt(t);
-    if (gate_out) *gate_out = *nrm < 0.717 * *nb ? 1.0 : 0.0;
-  }
+// *nrm = the norm from G shares, w /= it.
+__global__ __launch_bounds__(kGsBlock) void gs_rescale_kernel(double* __restrict__ w, int64_t n,
+                                                              const double* __restrict__ part,
+                                                              double* __restrict__ nrm_out) {
+  __shared__ double s_n[1];
+  gs_sums(part, gridDim.x, 1, s_n);
+  const double nrm = sqrt(s_n[0]), f = 1.0 / nrm;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *nrm_out = nrm;
+  for (int64_t e = blockIdx.x * (int64_t)kGsBlock + threadIdx.x; e < n; e += (int64_t)gridDim.x * kGsBlock) w[e] *= f;
 }
 
 // out = x * (1 / *nrm)
@@ -202,23 +344,27 @@ __global__ void scale_inv_kernel(const double* x, const double* nrm, double* out
     out[e] = x[e] * s;
 }
 
-// Y (k columns) = V (m columns) * C (m x k, column-major, host-uploaded), per element.
-__global__ void basis_combine_kernel(const double* V, int64_t ldv, int m, const double* C, int k, double* Y,
-                                     int64_t ldy, int64_t n) {
-  __shared__ double s_c[kMaxBasis * kMaxBasis];
+// Y (k columns) = V (m columns) * C (m x k, column-major), per element, and
+// with `last` column k of Y = column m of V (the residual a thick restart
+// continues from).  K >= m: the registers it takes set the occupancy.
+template <int K>
+__global__ __launch_bounds__(kVecBlock) void basis_combine_kernel(const double* __restrict__ V, int64_t n, int m,
+                                                                  const double* __restrict__ C, int k,
+                                                                  double* __restrict__ Y, int last) {
+  __shared__ double s_c[K * K];
   for (int i = threadIdx.x; i < m * k; i += blockDim.x) s_c[i] = C[i];
   __syncthreads();
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
-    double v[kMaxBasis];
+    double v[K];
 #pragma unroll
-    for (int i = 0; i < kMaxBasis; ++i)
-      if (i < m) v[i] = V[i * ldv + e];
+    for (int i = 0; i < K; ++i) v[i] = i < m ? V[i * n + e] : 0.0;
+    if (last) Y[(int64_t)k * n + e] = V[(int64_t)m * n + e];
     for (int j = 0; j < k; ++j) {
       double y = 0.0;
 #pragma unroll
-      for (int i = 0; i < kMaxBasis; ++i)
+      for (int i = 0; i < K; ++i)
         if (i < m) y = fma(s_c[j * m + i], v[i], y);
-      Y[j * ldy + e] = y;
+      Y[j * n + e] = y;
     }
   }
 }
@@ -283,24 +429,29 @@ void dev_scale_inv(const double* x, const double* nrm, double* out, int64_t n, h
   EDH_HIP(hipGetLastError());
 }
 
-void dev_orthogonalize(const double* V, int64_t ldv, int m, double* w, int64_t n, double* partial, double* h,
-                       double* hsum, double* nrm, hipStream_t s, double* nb, const double* gate, double* gate_out) {
-  EDH_CHECK(m >= 1 && m <= kMaxBasis, EDH_ERR_LIMIT, "Krylov basis size outside the device limit");
-  EDH_CHECK(!gate_out || nb, EDH_ERR_INTERNAL, "DGKS gate needs the norm before the pass");
-  const int g = reduce_grid(n);
-  const int with_nb = nb ? 1 : 0;
-  hipLaunchKernelGGL(multi_dot_kernel, dim3(g), dim3(kVecBlock), 0, s, V, ldv, m, w, n, partial, with_nb, gate);
-  hipLaunchKernelGGL(multi_reduce_kernel, dim3(1), dim3(kVecBlock), 0, s, partial, g, m, h, hsum, with_nb, nb, gate);
-  hipLaunchKernelGGL(multi_axpy_kernel, dim3(g), dim3(kVecBlock), 0, s, V, ldv, m, h, w, n, partial, gate);
-  hipLaunchKernelGGL(ortho_norm_kernel, dim3(1), dim3(kVecBlock), 0, s, partial, g, nrm, nb, gate_out, gate);
+int gs_grid(int64_t n) {
+  return (int)std::min<int64_t>(std::max<int64_t>((n + kGsTile - 1) / kGsTile, 1), kGsShares);
+}
+
+void dev_orthonormalize(double* V, int64_t n, int cnt, double* part, double* hcol, double* nrm, bool exact,
+                        hipStream_t s) {
+  EDH_CHECK(cnt >= 1 && cnt < kMaxBasis, EDH_ERR_LIMIT, "Krylov basis size outside the device limit");
+  const int g = gs_grid(n);
+  double* part2 = part + (size_t)(cnt + 1) * g;
+  hipLaunchKernelGGL(gs_dots_kernel, dim3(g), dim3(kGsBlock), 0, s, V, n, cnt, part);
+  auto update = cnt <= kGsGroup ? gs_update_kernel<true> : gs_update_kernel<false>;
+  hipLaunchKernelGGL(update, dim3(g), dim3(kGsBlock), 0, s, V, n, cnt, part, part2, hcol);
+  auto finish = exact ? gs_finish_kernel<true> : gs_finish_kernel<false>;
+  hipLaunchKernelGGL(finish, dim3(g), dim3(kGsBlock), 0, s, V, n, cnt, part, part2, hcol, nrm);
+  if (exact)
+    hipLaunchKernelGGL(gs_rescale_kernel, dim3(g), dim3(kGsBlock), 0, s, V + (int64_t)cnt * n, n, part, nrm);
   EDH_HIP(hipGetLastError());
 }
 
-void dev_combine(const double* V, int64_t ldv, int m, const double* C, int k, double* Y, int64_t ldy, int64_t n,
-                 hipStream_t s) {
-  EDH_CHECK(m <= kMaxBasis && k <= kMaxBasis, EDH_ERR_LIMIT, "Krylov basis larger than the device limit");
-  hipLaunchKernelGGL(basis_combine_kernel, dim3(reduce_grid(n)), dim3(kVecBlock), 0, s, V, ldv, m, C, k, Y, ldy,
-                     n);
+void dev_combine(const double* V, int64_t n, int m, const double* C, int k, double* Y, bool last, hipStream_t s) {
+  EDH_CHECK(m <= kMaxBasis && k <= m, EDH_ERR_LIMIT, "Krylov basis larger than the device limit");
+  auto kern = m <= 12 ? basis_combine_kernel<12> : m <= 24 ? basis_combine_kernel<24> : basis_combine_kernel<kMaxBasis>;
+  hipLaunchKernelGGL(kern, dim3(reduce_grid(n)), dim3(kVecBlock), 0, s, V, n, m, C, k, Y, last ? 1 : 0);
   EDH_HIP(hipGetLastError());
 }
 
