@@ -27,61 +27,101 @@ constexpr int kObsMaxSites = 32;
 constexpr int kColTile = 128;  // rows per column-sum tile
 constexpr int kMomBlocks = 512;  // first-stage blocks of the moment reduction
 
-// One block per row u (grid-stride): out[u * (Ns + 2) + b] = sum_d w [bit b
-// of bits_d] for b < Ns, then sum_d w, then sum_d w^2.  MS >= Ns bit slots
-// per element (16 for up to 16 sites: half the bit tests of 32).
-template <int MS>
-__global__ __launch_bounds__(kObsBlock) void obs_rows_kernel(const double* __restrict__ v, int64_t Dup, int64_t Ddn,
-                                                             const int32_t* __restrict__ dn_bits, int Ns,
-                                                             double* __restrict__ out) {
-  constexpr int kObsMaxSites = MS;
-  __shared__ double s_part[kObsBlock / 64][kObsMaxSites + 2];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int64_t u = blockIdx.x; u < Dup; u += gridDim.x) {
-    double acc[kObsMaxSites + 2];
+// Sums of K values per lane over the wavefront, halving the values with every
+// exchange: of two lanes that exchange, one keeps the first half of the values
+// and the other the second, so K + K/2 + ... values cross lanes instead of
+// 6 K.  Each value's additions are those of the tree x_l + x_{l+32}, then
+// + 16, ... (which operand comes first does not change a sum).  Value `lo`
+// ends on this lane when `valid`.
+template <int K>
+__device__ __forceinline__ void wave_sums(double (&v)[K], int& lo, bool& valid) {
+  const int lane = threadIdx.x & 63;
+  int cnt = K;
+  lo = 0;
+  int n = K;
 #pragma unroll
-    for (int b = 0; b < kObsMaxSites + 2; ++b) acc[b] = 0.0;
-    const double* row = v + u * Ddn;
-    for (int64_t d = threadIdx.x; d < Ddn; d += kObsBlock) {
-      const double x = row[d];
-      const double w = x * x;
-      const unsigned bits = (unsigned)dn_bits[d];
+  for (int off = 32; off > 0; off >>= 1) {
+    const int h = (n + 1) / 2;
+    const bool high = (lane & off) != 0;
 #pragma unroll
-      for (int b = 0; b < kObsMaxSites; ++b)
-        if ((bits >> b) & 1u) acc[b] += w;
-      acc[kObsMaxSites] += w;
-      acc[kObsMaxSites + 1] = fma(w, w, acc[kObsMaxSites + 1]);
+    for (int i = 0; i < (K + 1) / 2; ++i) {
+      if (i >= h) break;
+      const double x = v[i], y = i + h < n ? v[i + h] : 0.0;
+      v[i] = (high ? y : x) + __shfl_xor(high ? x : y, off, 64);
     }
-    // fixed-order reduction: shuffle tree per wavefront, then the
-    // wavefronts in order
-#pragma unroll
-    for (int b = 0; b < kObsMaxSites + 2; ++b) {
-      double x = acc[b];
-      for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
-      if (lane == 0) s_part[wave][b] = x;
-    }
-    __syncthreads();
-    const int nout = Ns + 2;
-    if ((int)threadIdx.x < nout) {
-      const int b = (int)threadIdx.x < Ns ? (int)threadIdx.x : kObsMaxSites + ((int)threadIdx.x - Ns);
-      double t = 0.0;
-      for (int q = 0; q < kObsBlock / 64; ++q) t += s_part[q][b];
-      out[u * nout + threadIdx.x] = t;
-    }
-    __syncthreads();
+    lo += high ? h : 0;
+    cnt = high ? max(cnt - h, 0) : min(cnt, h);
+    n = h;
   }
+  valid = cnt >= 1;
+}
+
+// Row u: out[u * (Ns + 2) + b] = sum_d w [bit b of bits_d] for b < Ns, then
+// sum_d w, then sum_d w^2.  MS >= Ns bit slots per element (16 for up to 16
+// sites: half the bit tests of 32).
+template <int MS>
+__device__ __forceinline__ void obs_row(const double* __restrict__ row, int64_t Ddn, const int32_t* __restrict__ dn_bits,
+                                        int Ns, double* __restrict__ out, double (*s_part)[kObsMaxSites + 2]) {
+  const int wave = threadIdx.x >> 6;
+  double acc[MS + 2];
+#pragma unroll
+  for (int b = 0; b < MS + 2; ++b) acc[b] = 0.0;
+  constexpr int U = 4;  // elements in flight
+  for (int64_t d0 = threadIdx.x; d0 < Ddn; d0 += U * kObsBlock) {
+    double x[U];
+    unsigned bits[U];
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      const int64_t d = d0 + q * kObsBlock;
+      x[q] = d < Ddn ? row[d] : 0.0;
+      bits[q] = d < Ddn ? (unsigned)dn_bits[d] : 0u;
+    }
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      if (d0 + q * kObsBlock >= Ddn) break;
+      const double w = x[q] * x[q];
+#pragma unroll
+      for (int b = 0; b < MS; ++b)
+        if ((bits[q] >> b) & 1u) acc[b] += w;
+      acc[MS] += w;
+      acc[MS + 1] = fma(w, w, acc[MS + 1]);
+    }
+  }
+  // fixed-order reduction: a tree per wavefront, then the wavefronts in order
+  int b;
+  bool valid;
+  wave_sums<MS + 2>(acc, b, valid);
+  if (valid) s_part[wave][b] = acc[0];
+  __syncthreads();
+  const int nout = Ns + 2;
+  if ((int)threadIdx.x < nout) {
+    const int i = (int)threadIdx.x < Ns ? (int)threadIdx.x : MS + ((int)threadIdx.x - Ns);
+    double t = 0.0;
+    for (int q = 0; q < kObsBlock / 64; ++q) t += s_part[q][i];
+    out[threadIdx.x] = t;
+  }
+  __syncthreads();
 }
 
 // Column sums by row tiles: part[tile * Ddn + d] = sum over the tile's rows
-// of v[u][d]^2 (coalesced over d).
-__global__ __launch_bounds__(kObsBlock) void obs_cols_kernel(const double* __restrict__ v, int64_t Dup, int64_t Ddn,
-                                                             double* __restrict__ part) {
-  const int64_t d = blockIdx.x * (int64_t)kObsBlock + threadIdx.x;
-  const int64_t tile = blockIdx.y;
+// of v[u][d]^2 (coalesced over d; even and odd rows of the tile in two running
+// sums, eight rows in flight).
+__device__ __forceinline__ void obs_col_tile(const double* __restrict__ v, int64_t Dup, int64_t Ddn, int64_t d,
+                                             int64_t tile, double* __restrict__ part) {
   if (d >= Ddn) return;
   const int64_t u0 = tile * kColTile, u1 = std::min<int64_t>(Dup, u0 + kColTile);
   double s0 = 0.0, s1 = 0.0;
   int64_t u = u0;
+  for (; u + 7 < u1; u += 8) {
+    double x[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) x[q] = v[(u + q) * Ddn + d];
+#pragma unroll
+    for (int q = 0; q < 8; q += 2) {
+      s0 = fma(x[q], x[q], s0);
+      s1 = fma(x[q + 1], x[q + 1], s1);
+    }
+  }
   for (; u + 1 < u1; u += 2) {
     const double x0 = v[u * Ddn + d], x1 = v[(u + 1) * Ddn + d];
     s0 = fma(x0, x0, s0);
@@ -94,21 +134,34 @@ __global__ __launch_bounds__(kObsBlock) void obs_cols_kernel(const double* __res
   part[tile * Ddn + d] = s0 + s1;
 }
 
-// C_d = sum over the tiles in order.
-__global__ __launch_bounds__(kObsBlock) void obs_cols_sum_kernel(const double* __restrict__ part, int64_t ntile,
-                                                                 int64_t Ddn, double* __restrict__ col) {
-  const int64_t d = blockIdx.x * (int64_t)kObsBlock + threadIdx.x;
-  if (d >= Ddn) return;
-  double s = 0.0;
-  for (int64_t t = 0; t < ntile; ++t) s += part[t * Ddn + d];
-  col[d] = s;
+// The pass over the vector: blocks below nrow take rows (grid-stride), the
+// others one column tile each, in one launch so that the second reader of an
+// element finds it in cache and neither waits for the other's last blocks.
+// 14-site Kanamori sector (8,7), 82 MB: rows and columns took 43.5 + 22.4 us
+// as two launches with a full tree of exchanges per value, 42 us now.
+template <int MS>
+__global__ __launch_bounds__(kObsBlock) void obs_pass_kernel(const double* __restrict__ v, int64_t Dup, int64_t Ddn,
+                                                             const int32_t* __restrict__ dn_bits, int Ns, int nrow,
+                                                             int ncb, double* __restrict__ rows,
+                                                             double* __restrict__ part) {
+  __shared__ double s_part[kObsBlock / 64][kObsMaxSites + 2];
+  if ((int)blockIdx.x < nrow) {
+    for (int64_t u = blockIdx.x; u < Dup; u += nrow)
+      obs_row<MS>(v + u * Ddn, Ddn, dn_bits, Ns, rows + u * (Ns + 2), s_part);
+    return;
+  }
+  const int q = (int)blockIdx.x - nrow;
+  obs_col_tile(v, Dup, Ddn, (int64_t)(q % ncb) * kObsBlock + threadIdx.x, q / ncb, part);
 }
 
 // First stage of the moments: block k takes rows [k R, (k + 1) R) and
-// columns [k C, (k + 1) C); thread t = a Ns + b (a, b < Ns) sums
-// UU[a][b], UD[a][b] over its rows and DD[a][b] over its columns; thread 0
-// also sum w^2.  part[k * (3 Ns^2 + 1) + ...] = (UU, UD, DD, sumsq).
-__global__ __launch_bounds__(1024) void obs_moments_kernel(const double* __restrict__ rows, const double* __restrict__ col,
+// columns [k C, (k + 1) C), whose sums C_d over the tiles (in order) it forms
+// first; thread t = a Ns + b (a, b < Ns) sums UU[a][b], UD[a][b] over its rows
+// and DD[a][b] over its columns; thread 0 also sum w^2.
+// part[k * (3 Ns^2 + 1) + ...] = (UU, UD, DD, sumsq).
+__global__ __launch_bounds__(1024) void obs_moments_kernel(const double* __restrict__ rows,
+                                                           const double* __restrict__ colpart, int64_t ntile,
+                                                           double* __restrict__ col,
                                                            const int32_t* __restrict__ up_bits,
                                                            const int32_t* __restrict__ dn_bits, int64_t Dup,
                                                            int64_t Ddn, int Ns, double* __restrict__ part) {
@@ -116,6 +169,20 @@ __global__ __launch_bounds__(1024) void obs_moments_kernel(const double* __restr
   const int nout = Ns + 2, nm = 3 * Ns * Ns + 1;
   const int k = blockIdx.x;
   const int64_t R = (Dup + gridDim.x - 1) / gridDim.x, C = (Ddn + gridDim.x - 1) / gridDim.x;
+  for (int64_t d = k * C + t; d < min(Ddn, (k + 1) * C); d += blockDim.x) {
+    double s = 0.0;
+    int64_t q = 0;
+    for (; q + 7 < ntile; q += 8) {
+      double x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = colpart[(q + i) * Ddn + d];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s += x[i];
+    }
+    for (; q < ntile; ++q) s += colpart[q * Ddn + d];
+    col[d] = s;
+  }
+  __syncthreads();  // the block's own columns, read back below
   double* o = part + (size_t)k * nm;
   if (t < Ns * Ns) {
     const int a = t / Ns, b = t - a * Ns;
@@ -160,7 +227,13 @@ __global__ __launch_bounds__(256) void obs_moments_sum_kernel(const double* __re
 }  // namespace
 
 void static_obs_run(Ctx& c, const double* dv, int norb, double* out) {
-  static_obs_sector(c.tabs, c.dev, c.model->Ns, dv, norb, c.obs, c.stream, out);
+  const int Ns = c.model->Ns;
+  EDH_CHECK(norb >= 1 && norb <= Ns, EDH_ERR_ARG, "static observables: interacting orbitals out of range");
+  c.obs.ensure(static_obs_scratch(c.tabs, Ns) * sizeof(double));
+  double* host = c.pinned(static_obs_host(c.tabs, Ns));
+  static_obs_launch(c.tabs, c.dev, Ns, dv, c.obs.as<double>(), c.stream, host);
+  EDH_HIP(hipStreamSynchronize(c.stream));
+  static_obs_reduce(c.tabs, Ns, norb, host, out);
 }
 
 size_t static_obs_scratch(const SectorTables& st, int Ns) {
@@ -185,19 +258,13 @@ void static_obs_launch(const SectorTables& st, const DevSector& ds, int Ns, cons
   const int nm = 3 * Ns * Ns + 1;
   double* mpart = col + Ddn;
   double* mom = mpart + (size_t)kMomBlocks * nm;
-  const int grid_rows = (int)std::min<int64_t>(Dup, 4096);
-  if (Ns <= 16)
-    hipLaunchKernelGGL(obs_rows_kernel<16>, dim3(grid_rows), dim3(kObsBlock), 0, stream, dv, Dup, Ddn, ds.dn.bits, Ns,
-                       rows);
-  else
-    hipLaunchKernelGGL(obs_rows_kernel<kObsMaxSites>, dim3(grid_rows), dim3(kObsBlock), 0, stream, dv, Dup, Ddn,
-                       ds.dn.bits, Ns, rows);
-  hipLaunchKernelGGL(obs_cols_kernel, dim3((unsigned)((Ddn + kObsBlock - 1) / kObsBlock), (unsigned)ntile),
-                     dim3(kObsBlock), 0, stream, dv, Dup, Ddn, part);
-  hipLaunchKernelGGL(obs_cols_sum_kernel, dim3((unsigned)((Ddn + kObsBlock - 1) / kObsBlock)), dim3(kObsBlock), 0,
-                     stream, part, ntile, Ddn, col);
+  const int nrow = (int)std::min<int64_t>(Dup, 4096);
+  const int ncb = (int)((Ddn + kObsBlock - 1) / kObsBlock);
+  auto pass = Ns <= 16 ? obs_pass_kernel<16> : obs_pass_kernel<kObsMaxSites>;
+  hipLaunchKernelGGL(pass, dim3((unsigned)(nrow + ncb * ntile)), dim3(kObsBlock), 0, stream, dv, Dup, Ddn, ds.dn.bits,
+                     Ns, nrow, ncb, rows, part);
   hipLaunchKernelGGL(obs_moments_kernel, dim3(kMomBlocks), dim3((unsigned)std::max(64, (Ns * Ns + 63) / 64 * 64)), 0,
-                     stream, rows, col, ds.up.bits, ds.dn.bits, Dup, Ddn, Ns, mpart);
+                     stream, rows, part, ntile, col, ds.up.bits, ds.dn.bits, Dup, Ddn, Ns, mpart);
   hipLaunchKernelGGL(obs_moments_sum_kernel, dim3(nm), dim3(256), 0, stream, mpart, kMomBlocks, nm, mom);
   EDH_HIP(hipGetLastError());
   EDH_HIP(hipMemcpyAsync(host, mom, (size_t)nm * sizeof(double), hipMemcpyDeviceToHost, stream));
