@@ -139,10 +139,6 @@ struct Batch {
   hipEvent_t ev_stage[2] = {nullptr, nullptr};
   bool ev_used[2] = {false, false};
   int stage_i = 0;
-  // (sector, orbital, annihilate) -> device gather maps (four arrays, then
-  // their one allocation) and the host blob they were copied from
-  std::map<std::tuple<int, int, int>, std::vector<void*>> maps;
-  std::map<std::tuple<int, int, int>, std::vector<char>> map_blobs;
   // stream-ordered frees not yet issued: a hipFreeAsync costs tens of
   // microseconds of host time, so they are issued while the host would
   // otherwise wait for the device (the memory is no longer referenced by
@@ -151,6 +147,16 @@ struct Batch {
   void defer_free(void* p) {
     if (p) pending_free.push_back(p);
   }
+  // (sector, orbital, annihilate) -> device gather maps of c / c^+: up and
+  // down index and sign arrays in an allocation that several keys share (its
+  // deleter defers the free, so maps is cleared before the last frees are issued)
+  typedef std::tuple<int, int, int> MapKey;
+  struct GatherMaps {
+    const int32_t* m[2] = {nullptr, nullptr};
+    const int8_t* s[2] = {nullptr, nullptr};
+    std::shared_ptr<void> owner;
+  };
+  std::map<MapKey, GatherMaps> maps;
   void issue_frees_until(hipEvent_t ev);  // until ev completes (all when ev is null)
   DevBuf d_gather;
   DevBuf d_obs;  // static-observable scratch
@@ -198,7 +204,8 @@ struct Batch {
   BSector& sector(int id);
   BJob& job(int id);
   int submit_eig(int sec, int nev, int ncv, double tol, int maxitr, uint64_t seed);
-  int submit_lanczos(int sec, const double* v0_dev, int nl);
+  // init false: the caller sets the run's scalars and start vector on the device
+  int submit_lanczos(int sec, const double* v0_dev, int nl, bool init = true);
   // Green's-function start vectors and their Lanczos runs; ids[i] = -1 when
   // vector i vanishes; norms[i] = its squared norm.
   void submit_gf(const std::vector<GfRequest>& req, int nl, std::vector<int>& ids);
@@ -218,7 +225,7 @@ struct Batch {
   void issue(std::vector<OpGroup>& pre, const std::vector<std::pair<int, HvArgs>>* hv, std::vector<OpGroup>& post,
              const std::vector<BJob*>* cycles = nullptr, const std::vector<ReadReq>* reads = nullptr);
   void fill_dev(double* p, size_t n);
-  void gather_maps(int src, int orb, bool annihilate, std::vector<void*>& out);
+  void gather_maps(const std::vector<MapKey>& keys);
 };
 
 }  // namespace edh
