@@ -582,9 +582,33 @@ __host__ __device__ inline int restart_keep(int nev, int m, int nconv) {
   return kk < 1 ? 1 : kk;
 }
 
+// x of lane (lane xor 8, 4, 2, 1) within its row of sixteen, for values that
+// repeat with period 2 S: a row rotation by S reaches the same value.
+template <int S>
+__device__ __forceinline__ double row_rotate(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x120 + S, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x120 + S, 0xf, 0xf, false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// Sum over the wavefront, on every lane: the halving tree (lane distances 32,
+// 16, 8, 4, 2, 1) on the register file's own exchanges, about 150 cycles where
+// the six shuffles through LDS took about 800.
 __device__ __forceinline__ double wave_sum(double x) {
-  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-  return x;  // on every lane
+  const long long b = __double_as_longlong(x);
+  const auto l5 = __builtin_amdgcn_permlane32_swap((unsigned)b, (unsigned)b, false, false);
+  const auto h5 = __builtin_amdgcn_permlane32_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+  x = __longlong_as_double(((long long)h5[0] << 32) | l5[0]) + __longlong_as_double(((long long)h5[1] << 32) | l5[1]);
+  const long long c = __double_as_longlong(x);
+  const auto l4 = __builtin_amdgcn_permlane16_swap((unsigned)c, (unsigned)c, false, false);
+  const auto h4 = __builtin_amdgcn_permlane16_swap((unsigned)(c >> 32), (unsigned)(c >> 32), false, false);
+  x = __longlong_as_double(((long long)h4[0] << 32) | l4[0]) + __longlong_as_double(((long long)h4[1] << 32) | l4[1]);
+  x += row_rotate<8>(x);
+  x += row_rotate<4>(x);
+  x += row_rotate<2>(x);
+  x += row_rotate<1>(x);
+  return x;
 }
 
 // Value of x held by lane l (l uniform over the wavefront).
@@ -592,6 +616,14 @@ __device__ __forceinline__ double lane_value(double x, int l) {
   const long long b = __double_as_longlong(x);
   const int lo = __builtin_amdgcn_readlane((int)b, l);
   const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// x of the next lane (the last lane's is unspecified): the whole-wave shift
+__device__ __forceinline__ double wave_next(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x130, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x130, 0xf, 0xf, false);
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
@@ -617,13 +649,13 @@ __device__ __forceinline__ double rsqrt_newton(double x) {
   return y;
 }
 
-__device__ bool wave_sym_eig(int n, double* a, double* qt, double* v, double* qq, double* w, int* order) {
+__device__ bool wave_sym_eig(int n, double* a, int lda, double* qt, double* v, double* qq, double* w, int* order) {
   const int lane = threadIdx.x;
   for (int i = lane; i < n * n; i += 64) qt[i] = (i / n == i % n) ? 1.0 : 0.0;
   __syncthreads();
   for (int k = 0; k + 2 < n; ++k) {
     const int m = n - k - 1;
-    const double xi = lane < m ? a[(k + 1 + lane) * n + k] : 0.0;
+    const double xi = lane < m ? a[(k + 1 + lane) * lda + k] : 0.0;
     const double nx = sqrt(wave_sum(xi * xi));
     if (nx == 0.0) continue;
     const double x0 = lane_value(xi, 0);
@@ -634,45 +666,64 @@ __device__ bool wave_sym_eig(int n, double* a, double* qt, double* v, double* qq
     vi /= nv;
     if (lane < m) v[lane] = vi;
     __syncthreads();
-    double pi = 0.0;
-    if (lane < m) {
+    // A v (row k + 1 + lane of A) and Q v (row lane of q) in one pass; a lane
+    // past the end repeats the last row's reads
+    const double* ar = a + (k + 1 + (lane < m ? lane : m - 1)) * lda + k + 1;
+    const double* qr = qt + (k + 1) * n + (lane < n ? lane : n - 1);
+    double pi = 0.0, sum = 0.0;
 #pragma unroll 4
-      for (int j = 0; j < m; ++j) pi += a[(k + 1 + lane) * n + k + 1 + j] * v[j];
+    for (int j = 0; j < m; ++j) {
+      pi += ar[j] * v[j];
+      sum += qr[j * n] * v[j];
     }
+    if (lane >= m) pi = 0.0;
     const double K = wave_sum(vi * pi);
     const double qi = pi - K * vi;
     if (lane < m) qq[lane] = qi;
     __syncthreads();
     if (lane < m) {
 #pragma unroll 4
-      for (int j = 0; j < m; ++j) a[(k + 1 + lane) * n + k + 1 + j] -= 2.0 * (vi * qq[j] + qi * v[j]);
+      for (int j = 0; j < m; ++j) a[(k + 1 + lane) * lda + k + 1 + j] -= 2.0 * (vi * qq[j] + qi * v[j]);
     }
     if (lane == 0) {
-      a[(k + 1) * n + k] = alpha;
-      a[k * n + k + 1] = alpha;
+      a[(k + 1) * lda + k] = alpha;
+      a[k * lda + k + 1] = alpha;
     }
     if (lane >= 1 && lane < m) {
-      a[(k + 1 + lane) * n + k] = 0.0;
-      a[k * n + k + 1 + lane] = 0.0;
+      a[(k + 1 + lane) * lda + k] = 0.0;
+      a[k * lda + k + 1 + lane] = 0.0;
     }
     if (lane < n) {
-      double sum = 0.0;
-#pragma unroll 4
-      for (int j = 0; j < m; ++j) sum += qt[(k + 1 + j) * n + lane] * v[j];
 #pragma unroll 4
       for (int j = 0; j < m; ++j) qt[(k + 1 + j) * n + lane] -= 2.0 * sum * v[j];
     }
     __syncthreads();
   }
-  double dr = lane < n ? a[lane * n + lane] : 0.0;
-  double er = lane + 1 < n ? a[(lane + 1) * n + lane] : 0.0;
+  // Implicit QL.  A rotation is one wavefront's chain of some thirty FP64
+  // instructions, so what counts is the number of instructions on the way:
+  // (d_i, e_i) lie as pairs in LDS, where one uniform access reads or writes
+  // both; lanes past the end repeat the last row of q instead of being masked;
+  // the next rotation's pair and q row are read while this one runs; the exit
+  // for a vanished rotation is tested off the chain; and two rotations follow
+  // each other without a jump.  (365 cycles a rotation where shuffled (d, e)
+  // and masked rows took 530; a decomposition of order 12 takes 62 us, of
+  // order 20 144 us, against 72 and 172; a nine-site three-orbital solve, whose
+  // sweeps wait for it, 129 -> 126 ms.)
+  const int ql = lane < n ? lane : n - 1;
+  double* de = v;  // v and qq are free now
+  if (lane < n) {
+    de[2 * lane] = a[lane * lda + lane];
+    de[2 * lane + 1] = lane + 1 < n ? a[(lane + 1) * lda + lane] : 0.0;
+  }
   const double eps = 2.220446049250313e-16;
   for (int l = 0; l < n; ++l) {
     int iter = 0;
     for (;;) {
+      __syncthreads();
+      const double dr = de[2 * ql], er = de[2 * ql + 1];
       // m = the first index >= l whose off-diagonal is negligible (else
       // n - 1): every lane tests its own, one ballot
-      const double dnext = __shfl_down(dr, 1, 64);
+      const double dnext = wave_next(dr);
       const bool split = lane < n - 1 && fabs(er) <= eps * (fabs(dr) + fabs(dnext));
       const unsigned long long hits = __ballot(split) & (~0ull << l);
       const int m = hits ? __ffsll((long long)hits) - 1 : n - 1;
@@ -683,54 +734,62 @@ __device__ bool wave_sym_eig(int n, double* a, double* qt, double* v, double* qq
       double r = sqrt(fma(g, g, 1.0));
       g = lane_value(dr, m) - dl + el / (g + copysign(r, g));
       double sn = 1.0, c = 1.0, pp = 0.0;
-      bool early = false;
       // the eigenvector rows: rotation i turns rows i and i + 1, and row
       // i + 1 is the row that rotation i + 1 produced, so it is carried in a
       // register instead of being read back
-      double carry = lane < n ? qt[m * n + lane] : 0.0;
-      for (int i = m - 1; i >= l; --i) {
-        const double ei = lane_value(er, i);
+      double carry = qt[m * n + ql];
+      double* pq = qt + (m - 1) * n + ql;
+      double* pd = de + 2 * (m - 1);
+      double dhi = pd[2], di = pd[0], ei = pd[1], qi = pq[0];
+      int left = m - l;
+      bool early = false;
+      // Rotation i = l + left - 1 of this sweep; false (and no change) when it
+      // vanishes.  What it reads ahead at i = 0 lies before the arrays, still
+      // in this block's LDS, and is not used.
+      auto rotate = [&]() {
+        const double dn = pd[-2], en = pd[-1], qn = pq[-n];
         const double f = sn * ei;
         const double b = c * ei;
         // the entries are moderate (Ritz values and couplings of H), so
         // f^2 + g^2 cannot overflow; r and 1/r from one reciprocal square
         // root (the rotation's latency chain is the QL sweep's cost)
         const double x2 = fma(f, f, g * g);
-        if (x2 == 0.0) {
-          if (lane == i + 1) {
-            er = 0.0;
-            dr -= pp;
-          }
-          if (lane == m) er = 0.0;
-          if (lane < n) qt[(i + 1) * n + lane] = carry;
-          early = true;
-          break;
-        }
-        const double rinv = rsqrt_newton(x2);
-        r = x2 * rinv;
-        if (lane == i + 1) er = r;
+        double rinv = rsqrt_newton(x2);
+        asm volatile("" : "+v"(rinv));  // computed before the exit is decided
+        if (__ballot(x2 == 0.0) != 0) return false;  // the same on every lane
         sn = f * rinv;
         c = g * rinv;
-        g = lane_value(dr, i + 1) - pp;
-        r = (lane_value(dr, i) - g) * sn + 2.0 * c * b;
-        pp = sn * r;
-        if (lane == i + 1) dr = g + pp;
-        g = c * r - b;
-        if (lane < n) {
-          const double q0 = qt[i * n + lane];
-          qt[(i + 1) * n + lane] = sn * q0 + c * carry;
-          carry = c * q0 - sn * carry;
-        }
+        g = dhi - pp;
+        const double t = fma(b, 2.0 * c, sn * (di - g));
+        pp = sn * t;
+        pd[2] = fma(sn, t, g);
+        pd[3] = x2 * rinv;
+        g = fma(c, t, -b);
+        pq[n] = fma(c, carry, sn * qi);
+        carry = fma(c, qi, -(sn * carry));
+        dhi = di;
+        di = dn;
+        ei = en;
+        qi = qn;
+        pq -= n;
+        pd -= 2;
+        return true;
+      };
+      for (;;) {
+        if (!rotate()) { early = true; break; }
+        if (--left == 0) break;
+        if (!rotate()) { early = true; break; }
+        if (--left == 0) break;
       }
-      if (early) continue;
-      if (lane < n) qt[l * n + lane] = carry;
-      if (lane == l) {
-        dr -= pp;
-        er = g;
-      }
-      if (lane == m) er = 0.0;
+      // row and pair i + 1: after a whole sweep i + 1 = l
+      pq[n] = carry;
+      pd[2] = dhi - pp;
+      pd[3] = early ? 0.0 : g;
+      de[2 * m + 1] = 0.0;
     }
   }
+  const double dr = de[2 * ql];
+  __syncthreads();
   // stable ascending order: lane i's rank among (d, index)
   if (lane < n) {
     int rk = 0;
@@ -745,11 +804,14 @@ __device__ bool wave_sym_eig(int n, double* a, double* qt, double* v, double* qq
   if (lane < n) {
     w[lane] = qq[order[lane]];
 #pragma unroll 4
-    for (int j = 0; j < n; ++j) a[lane * n + j] = qt[order[j] * n + lane];
+    for (int j = 0; j < n; ++j) a[lane * lda + j] = qt[order[j] * n + lane];
   }
   __syncthreads();
   return true;
 }
+
+// odd rows keep a column of the cycle's matrix off the same LDS banks
+__host__ __device__ inline int cycle_lda(int m) { return m | 1; }
 
 struct BCyc {
   double* sc;
@@ -778,7 +840,8 @@ __device__ void cycle_end(const BCyc& o, double* s_e, int* s_done, int* s_nconv_
   const int k = (int)ctl[C_K];
   const int phase = (int)ctl[kCtlPhase];
   double* a = s_e;
-  double* qt = a + m * m;
+  const int lda = cycle_lda(m);
+  double* qt = a + m * lda;
   double* v = qt + m * m;
   double* qq = v + m;
   double* w = qq + m;
@@ -788,10 +851,10 @@ __device__ void cycle_end(const BCyc& o, double* s_e, int* s_done, int* s_nconv_
   for (int i = lane; i < m * m; i += 64) {
     const int r = i / m, c = i % m;
     const int hi = r > c ? r : c, lo = r > c ? c : r;
-    a[i] = (hi < k) ? (r == c ? theta_kept[r] : 0.0) : Tcol[(size_t)hi * (m + 1) + lo];
+    a[r * lda + c] = (hi < k) ? (r == c ? theta_kept[r] : 0.0) : Tcol[(size_t)hi * (m + 1) + lo];
   }
   __syncthreads();
-  if (!wave_sym_eig(m, a, qt, v, qq, w, order)) {
+  if (!wave_sym_eig(m, a, lda, qt, v, qq, w, order)) {
     if (lane == 0) ctl[kCtlState] = 2.0;
     return;
   }
@@ -800,7 +863,7 @@ __device__ void cycle_end(const BCyc& o, double* s_e, int* s_done, int* s_nconv_
     const double eps23 = 3.666852862501036e-11;  // eps^(2/3)
     int nc = 0;
     for (int i = 0; i < o.nev; ++i) {
-      const double bound = fabs(bres * a[(m - 1) * m + i]);
+      const double bound = fabs(bres * a[(m - 1) * lda + i]);
       if (bound <= o.tol * fmax(fabs(w[i]), eps23)) s_done[nc++] = i;
     }
     s_nconv = nc;
@@ -814,7 +877,7 @@ __device__ void cycle_end(const BCyc& o, double* s_e, int* s_done, int* s_nconv_
     // the converged Ritz pairs are the result (after maxitr: dseupd with info = 1)
     if (lane < nc) ctl[C_HDR + lane] = w[s_done[lane]];
     if (lane < m)
-      for (int c = 0; c < nc; ++c) C[c * m + lane] = a[lane * m + s_done[c]];
+      for (int c = 0; c < nc; ++c) C[c * m + lane] = a[lane * lda + s_done[c]];
     __syncthreads();
     if (lane == 0) {
       ctl[C_ITER] = iter;
@@ -830,7 +893,7 @@ __device__ void cycle_end(const BCyc& o, double* s_e, int* s_done, int* s_nconv_
   // thick restart: new basis column c < kk = sum_i A[i][c] V_i, column kk = V_m
   const int kk = restart_keep(o.nev, m, nc);
   if (lane <= m) {
-    for (int c = 0; c < kk; ++c) C[c * (m + 1) + lane] = lane < m ? a[lane * m + c] : 0.0;
+    for (int c = 0; c < kk; ++c) C[c * (m + 1) + lane] = lane < m ? a[lane * lda + c] : 0.0;
     C[kk * (m + 1) + lane] = lane == m ? 1.0 : 0.0;
   }
   if (lane < kk) ctl[ctl_theta(m) + lane] = w[lane];
@@ -1815,7 +1878,7 @@ void Batch::issue(std::vector<OpGroup>& pre, const std::vector<std::pair<int, Hv
     }
     launch(pl_post);
     if (ncyc) {
-      const size_t smem = (size_t)(2 * max_m * max_m + 3 * max_m) * sizeof(double) + (size_t)max_m * sizeof(int);
+      const size_t smem = (size_t)(max_m * (cycle_lda(max_m) + max_m) + 3 * max_m) * sizeof(double) + (size_t)max_m * sizeof(int);
       hipLaunchKernelGGL(bcycle_kernel, dim3(ncyc), dim3(64), smem, stream, (const BCyc*)(db + cyc_off));
       // the combination reads at most max_m + 1 basis vectors per element:
       // registers for twelve of them when that suffices (occupancy)
