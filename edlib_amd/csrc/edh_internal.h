@@ -159,8 +159,9 @@ void build_sector(const Model& m, int nup, int ndn, SectorTables& st, bool need_
 
 // H*v variants: single pass (rows, up-spin term from the cache hierarchy) or
 // two passes: whole columns, then whole rows gathered in LDS (hv_lines.hip)
-// where several of each fit, else rows without the up-spin term, then
-// XCD-aware column slabs for it.  HV_AUTO picks the sector's faster one.
+// where several of each fit, else rows without the up-spin term, then tiles
+// of rows and columns for it (hv_tiles.hip).  HV_AUTO picks the sector's
+// faster one.
 enum HvVariant { HV_SINGLE = 0, HV_TWO_PASS = 1, HV_AUTO = -1 };
 
 // Device mirror of one sector.
@@ -213,7 +214,11 @@ struct DevSector {
   double* kan_tc = nullptr;
   int32_t* row_order = nullptr;  // processing order of up rows
   int variant = HV_SINGLE;       // chosen H*v variant
-  int* counters = nullptr;       // work queues of the slab pass (8 ints)
+  // the up spin's entries for the tile pass (up_tile_tables), where the line
+  // passes do not apply
+  int32_t* up_slices = nullptr;
+  uint32_t* up_in = nullptr;
+  uint32_t* up_out = nullptr;
   int64_t table_bytes = 0;
   std::vector<void*> allocs;
   hipStream_t astream = nullptr;  // stream the tables were allocated on (stream-ordered pool)
@@ -303,7 +308,7 @@ constexpr int kCtlCol = 0, kCtlPhase = 1, kCtlState = 2;
 
 void launch_hv(const DevSector& ds, const HvArgs& a, hipStream_t s, int variant = HV_AUTO);
 int hv_num_blocks(const DevSector& ds);
-int hv_autotune(DevSector& ds, hipStream_t s);
+int hv_choose(const DevSector& ds);
 
 // Two passes of LDS gathers over whole lines (hv_lines.hip): rows and columns
 // per work-group, work-group sizes and LDS of each pass, fixed by the sector
@@ -314,6 +319,9 @@ struct HvLinesPlan {
   bool ok;
 };
 HvLinesPlan hv_lines_plan(const DevSector& ds);
+// Host tables of the tile pass (hv_tiles.hip).
+void up_tile_tables(const SpinTables& sp, std::vector<int32_t>& slices, std::vector<uint32_t>& in,
+                    std::vector<uint32_t>& out);
 int hv_lines_threads(int64_t D);
 int hv_lines_partials(const DevSector& ds);  // shares of <v, w> per operand
 bool hv_lines_faster(const DevSector& ds);   // than the single pass, for one operand alone

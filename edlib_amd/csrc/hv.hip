@@ -21,10 +21,9 @@
 // its value set are small, 16-bit entries are packed by slot quads.  Either
 // way all quads of a column group are loaded at once, one group ahead.
 //
-// Up-spin slab kernel (two-pass variant): the rows kernel runs without the
-// up-spin term, then each XCD sweeps all rows over its own column slab of 16
-// columns, so the slab (D_up x 128 B) stays in that XCD's L2 while every
-// neighbour row segment is re-read from it.
+// Two-pass variant: whole columns, then whole rows gathered in LDS
+// (hv_lines.hip) where they fit; else the rows kernel without the up-spin
+// term, then that term over tiles of rows and columns (hv_tiles.hip).
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
@@ -596,103 +595,6 @@ __global__ __launch_bounds__(1024) void hv_rows_multi_kernel(HvParams p, HvMulti
   }
 }
 
-// Up-spin term over column slabs of 16 (one 128-byte line per row segment):
-// w[u][c] += sum_k Hup[u][k] v[k][c].  Persistent work-groups read the XCD
-// they run on (HW_REG_XCC_ID) and claim (slab, row block) items from that
-// XCD's queue: XCD x owns slabs x, x+8, x+16, ... and its work-groups sweep
-// all row blocks of one slab before the next, so the slab (D_up x 128 B)
-// stays in that XCD's L2 while the ~17 neighbour segments of each row are
-// re-read from it.  A work-group that finds its queue empty takes items from
-// the other XCDs' queues, so every item is processed whatever XCD ids are
-// reported.  The CSR entries of an item's rows are staged in LDS as (row
-// offset, value) pairs; a wavefront covers four rows of the slab.
-constexpr int kSlabW = 16;
-constexpr int kSlabWG = 256;
-constexpr int kSlabRows = 64;
-constexpr int kSlabEnt = 2048;
-constexpr int kXcd = 8;
-
-__global__ void zero_counters_kernel(int* c, int n) {
-  if ((int)threadIdx.x < n) c[threadIdx.x] = 0;
-}
-
-__global__ __launch_bounds__(kSlabWG) void hv_upslab_kernel(HvParams p, int* counters) {
-  __shared__ double s_red[16];
-  __shared__ int s_item;
-  __shared__ uint32_t s_off[kSlabEnt];
-  __shared__ double s_val[kSlabEnt];
-  double vscale, wscale;
-  if (!hv_scales(p, s_red, false, vscale, wscale)) return;
-  unsigned xcc;
-  asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
-  const int home = (int)(xcc & (kXcd - 1));
-  const int Ddn = p.Ddn;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int quarter = lane >> 4;
-  const int wave = tid >> 6;
-  const double* __restrict__ V = p.v;
-  double dsum = 0.0;
-  for (int t = 0; t < kXcd; ++t) {
-    const int x = (home + t) & (kXcd - 1);
-    const int nsl_x = p.nslabs > x ? (p.nslabs - x + kXcd - 1) / kXcd : 0;
-    const int items = nsl_x * p.nrb;
-    for (;;) {
-      if (tid == 0) s_item = atomicAdd(counters + x, 1);
-      __syncthreads();  // also: the previous item's readers of s_off/s_val are done
-      const int item = s_item;
-      if (item >= items) {
-        __syncthreads();  // everyone has read s_item before it is rewritten
-        break;
-      }
-      const int slab = x + kXcd * (item / p.nrb);
-      const int rb = item - (item / p.nrb) * p.nrb;
-      const int c = slab * kSlabW + (lane & 15);
-      const int r0 = rb * p.rows_per_wg;
-      const int r1 = min(r0 + p.rows_per_wg, p.Dup);
-      const int e0 = p.up_rowp[r0], ne = p.up_rowp[r1] - e0;
-      const bool staged = p.off32 && ne <= kSlabEnt;
-      if (staged)
-        for (int i = tid; i < ne; i += kSlabWG) {
-          const uint32_t e = p.up_packed[e0 + i];
-          s_off[i] = (e & kColMask) * (uint32_t)Ddn;
-          s_val[i] = p.values[e >> kColBits];
-        }
-      __syncthreads();
-      for (int r = r0 + wave * 4 + quarter; r < r1; r += (kSlabWG / 64) * 4) {
-        if (c >= Ddn) continue;
-        const int hb = p.up_rowp[r], he = p.up_rowp[r + 1];
-        double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-        if (staged) {
-          int q = hb - e0;
-          const int qe = he - e0;
-          for (; q + 3 < qe; q += 4) {
-            const double x0 = V[s_off[q] + c], x1 = V[s_off[q + 1] + c];
-            const double x2 = V[s_off[q + 2] + c], x3 = V[s_off[q + 3] + c];
-            a0 = fma(s_val[q], x0, a0);
-            a1 = fma(s_val[q + 1], x1, a1);
-            a2 = fma(s_val[q + 2], x2, a2);
-            a3 = fma(s_val[q + 3], x3, a3);
-          }
-          for (; q < qe; ++q) a0 = fma(s_val[q], V[s_off[q] + c], a0);
-        } else {
-          for (int q = hb; q < he; ++q) {
-            const uint32_t e = p.up_packed[q];
-            a0 = fma(p.values[e >> kColBits], V[(size_t)(e & kColMask) * Ddn + c], a0);
-          }
-        }
-        const double acc = (a0 + a1) + (a2 + a3);
-        const size_t o = (size_t)r * Ddn + c;
-        const double wn = __builtin_nontemporal_load(p.w + o) + acc * vscale;
-        __builtin_nontemporal_store(wn, p.w + o);
-        if (p.dot_partial) dsum = fma(V[o] * vscale, wn, dsum);
-      }
-    }
-  }
-  if (p.dot_partial) block_reduce_store(dsum, s_red, p.dot_partial + blockIdx.x);
-}
-
-
 // ---------------------------------------------------------------------------
 // Grouped H*v: every operand of a batch in one launch.  The up-rows of all
 // operands are cut into work units (operand, first row, row count; about
@@ -963,15 +865,6 @@ void launch_j(const HvParams& p, const Launch& L, int cross, bool kan, bool up, 
   }
 }
 
-// Slab pass geometry; returns its (persistent) grid size.
-int slab_geometry(const DevSector& ds, int& nslabs, int& rows_per_wg, int& nrb) {
-  nslabs = (int)((ds.dn.D + kSlabW - 1) / kSlabW);
-  rows_per_wg = kSlabRows;
-  nrb = (int)((ds.up.D + rows_per_wg - 1) / rows_per_wg);
-  const int64_t items = (int64_t)nslabs * nrb;
-  return (int)std::min<int64_t>(items, 2048);
-}
-
 HvParams make_params(const DevSector& ds, const HvArgs& a) {
   HvParams p;
   std::memset(&p, 0, sizeof(p));  // padding too: batched sweeps compare descriptor bytes
@@ -1022,8 +915,9 @@ HvParams make_params(const DevSector& ds, const HvArgs& a) {
   p.dscale = a.dscale;
   p.done = a.done;
   p.lz = a.step;
-  slab_geometry(ds, p.nslabs, p.rows_per_wg, p.nrb);
-  p.off32 = (uint64_t)ds.N < (uint64_t(1) << 32);
+  p.up_slices = ds.up_slices;
+  p.up_in = ds.up_in;
+  p.up_out = ds.up_out;
   p.row_t = hv_lines_threads(ds.dn.D);
   p.col_t = hv_lines_threads(ds.up.D);
   p.xcd_rows = 1;
@@ -1037,8 +931,7 @@ HvParams make_params(const DevSector& ds, const HvArgs& a) {
 int hv_num_blocks(const DevSector& ds) {
   if (ds.variant != HV_TWO_PASS) return plan(ds).grid;
   if (hv_lines_plan(ds).ok) return hv_lines_partials(ds);
-  int nslabs, rpw, nrb;
-  return slab_geometry(ds, nslabs, rpw, nrb);
+  return hv_up_tiles_blocks(ds);
 }
 
 void launch_hv(const DevSector& ds, const HvArgs& a, hipStream_t s, int variant) {
@@ -1055,63 +948,26 @@ void launch_hv(const DevSector& ds, const HvArgs& a, hipStream_t s, int variant)
     default: launch_j<4>(p, L, ds.cross_mode, kan, up, s); break;
   }
   if (!up) {
-    // the rows pass wrote the partial result; the slab pass adds the up-spin
+    // the rows pass wrote the partial result; the tile pass adds the up-spin
     // term and produces the dot partials (the rows pass skips them)
-    int nslabs, rpw, nrb;
-    const int grid = slab_geometry(ds, nslabs, rpw, nrb);
-    hipLaunchKernelGGL(zero_counters_kernel, dim3(1), dim3(64), 0, s, ds.counters, kXcd);
-    hipLaunchKernelGGL(hv_upslab_kernel, dim3(grid), dim3(kSlabWG), 0, s, p, ds.counters);
-    EDH_HIP(hipGetLastError());
+    launch_hv_up_tiles(ds, p, s);
   }
 }
 
-// Where the line passes apply the choice is a rule (hv_lines_faster); else
-// both variants are timed on scratch vectors and the faster one is kept (an
-// environment override EDH_HV_VARIANT=0/1 fixes the choice).
-int hv_autotune(DevSector& ds, hipStream_t s) {
+// The variant of a single sector (an environment override EDH_HV_VARIANT=0/1
+// fixes it): the line passes by their own rule, else the tile pass from 4 M
+// states on.  Measured there (MI355X, us per H*v, single pass : two passes):
+//   16 sites, 12870 x 12870: 4x4 torus 4820 : 3470, ring 2973 : 2539, Anderson
+//     2802 : 2835, Kanamori 6329 : 5631; 12870 x 11440 all-to-all 9192 : 7498
+//   rectangular: 12870 x 1820 torus 580 : 454, ring 364 : 338; 1820 x 12870
+//     534 : 432, 334 : 335; 12870 x 4368 Anderson 1219 : 903; 4368 x 12870
+//     Kanamori 1986 : 1877; 12870 x 560 torus 213 : 199
+//   17 sites, 24310 x 19448: Anderson 8198 : 7792.
+int hv_choose(const DevSector& ds) {
   const char* env = getenv("EDH_HV_VARIANT");
   if (env && (env[0] == '0' || env[0] == '1')) return env[0] - '0';
   if (hv_lines_plan(ds).ok) return hv_lines_faster(ds) ? HV_TWO_PASS : HV_SINGLE;
-  if (ds.N < (1 << 22)) return HV_SINGLE;  // short rows: the slab pass never pays
-  double *v = nullptr, *w = nullptr;
-  if (hipMalloc(&v, ds.N * sizeof(double)) != hipSuccess) return HV_SINGLE;
-  if (hipMalloc(&w, ds.N * sizeof(double)) != hipSuccess) {
-    (void)hipFree(v);
-    return HV_SINGLE;
-  }
-  EDH_HIP(hipMemsetAsync(v, 0, ds.N * sizeof(double), s));
-  EDH_HIP(hipMemsetAsync(w, 0, ds.N * sizeof(double), s));
-  HvArgs a{};
-  a.v = v;
-  a.w = w;
-  a.wprev = w;
-  a.vscale = 1.0;
-  a.wscale = 1.0;
-  a.mode = 1;
-  hipEvent_t e0, e1;
-  EDH_HIP(hipEventCreate(&e0));
-  EDH_HIP(hipEventCreate(&e1));
-  float best = 1e30f;
-  int choice = HV_SINGLE;
-  for (int var = HV_SINGLE; var <= HV_TWO_PASS; ++var) {
-    launch_hv(ds, a, s, var);  // warm-up
-    EDH_HIP(hipEventRecord(e0, s));
-    for (int r = 0; r < 2; ++r) launch_hv(ds, a, s, var);
-    EDH_HIP(hipEventRecord(e1, s));
-    EDH_HIP(hipEventSynchronize(e1));
-    float ms = 0.f;
-    EDH_HIP(hipEventElapsedTime(&ms, e0, e1));
-    if (ms < best) {
-      best = ms;
-      choice = var;
-    }
-  }
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  EDH_HIP(hipStreamSynchronize(s));
-  (void)hipFree(v);
-  (void)hipFree(w);
-  return choice;
+  return ds.N >= (1 << 22) ? HV_TWO_PASS : HV_SINGLE;
 }
 
 }  // namespace edh

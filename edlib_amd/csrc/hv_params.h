@@ -55,8 +55,11 @@ struct HvParams {
   const double* dscale;
   const int* done;
   LzStep lz;
-  // slab kernel geometry; off32: every element offset fits 32 bits
-  int nslabs, rows_per_wg, nrb, off32;
+  // tile pass: per slice of two up rows (start, length) of its entries within
+  // the tile and outside it
+  const int32_t* up_slices;
+  const uint32_t* up_in;
+  const uint32_t* up_out;
   int row_t, col_t;  // line passes: threads that share a row, a column (hv_lines_threads)
   int xcd_rows;  // rows kernel: XCD-grouped row assignment (measured 2 % faster on the 16-site sector)
   // rows kernel in a batch: an eigensolver run's control block (v and w are
@@ -162,6 +165,11 @@ struct HvBatchJob {
   double* tdot;         // per-task shares of <v, w>, or null
   const double* lzk;    // Lanczos run's step counter (buffers in rotation) or null
 };
+
+// The up-spin term in tiles (hv_tiles.hip): w += Hup v and the shares of
+// <v, w>, hv_up_tiles_blocks of them.
+int hv_up_tiles_blocks(const DevSector& ds);
+void launch_hv_up_tiles(const DevSector& ds, const HvParams& p, hipStream_t s);
 
 // Fills the descriptor of one operand (hv.hip).
 HvBatchJob make_job(const DevSector& ds, const HvArgs& a);

@@ -285,12 +285,21 @@ void upload_sector(const SectorTables& st, int Ns, DevSector& ds, hipStream_t s,
     ds.nkan = (int)kc.size();
     if (ds.lines) add_row_tiles(pk, st, kc, ds);
   }
-  pk.add(ds.counters, std::vector<int32_t>(64, 0));
   pk.add(ds.row_order, rcm_order(st.up.rowp, st.up.col, st.up.D));
   pk.commit(ds, s, stage);
   if (stage) return;
+  Packer tiles;
+  if (ds.N > 0 && !hv_lines_plan(ds).ok) {
+    std::vector<int32_t> slices;
+    std::vector<uint32_t> in, out;
+    up_tile_tables(st.up, slices, in, out);
+    tiles.add(ds.up_slices, slices);
+    tiles.add(ds.up_in, in);
+    tiles.add(ds.up_out, out);
+    tiles.commit(ds, s, nullptr);
+  }
   EDH_HIP(hipStreamSynchronize(s));
-  ds.variant = hv_autotune(ds, s);
+  ds.variant = hv_choose(ds);
 }
 
 }  // namespace edh

@@ -34,7 +34,7 @@ def main():
     ap.add_argument("--copy-mib", type=int, default=1024)
     ap.add_argument("--sites", type=int, default=16, choices=(12, 14, 16))
     ap.add_argument("--variant", type=int, default=-1, choices=(-1, 0, 1),
-                    help="H*v variant: -1 = autotuned, 0 = single pass, 1 = two passes")
+                    help="H*v variant: -1 = the sector's own choice, 0 = single pass, 1 = two passes")
     a = ap.parse_args()
     import edlib_amd as ea
     from edlib_amd import _lib

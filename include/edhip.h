@@ -171,9 +171,9 @@ int edh_static_observables(edh_ctx* ctx, const double* v, int64_t n, int mem, in
 
 /* H*v kernel variant of the current sector: 0 = single pass (rows), 1 = two
  * passes (whole columns, then whole rows gathered in LDS where several of each
- * fit; else rows, then column slabs for the up-spin term).  The sector set-up
- * takes the faster one, by a rule on the sector where lines fit LDS, else by
- * timing both; edh_set_hv_variant fixes one of them (-1: choose again). */
+ * fit; else rows, then tiles of rows and columns for the up-spin term).  The
+ * sector set-up takes the faster one by a rule on the sector;
+ * edh_set_hv_variant fixes one of them (-1: choose again). */
 int edh_get_hv_variant(edh_ctx* ctx, int* variant);
 int edh_set_hv_variant(edh_ctx* ctx, int variant);
 
