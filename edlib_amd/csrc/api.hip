@@ -536,11 +536,14 @@ int lanczos_device(Ctx& c, int nl, double* alpha, double* beta, double* step_ms)
   }
   // One Lanczos step = H*v with the shares of alpha, then the update with
   // the shares of |w|^2; the scalars stay on the device, and the host issues
-  // every step without waiting (kernels of a stopped run return at once).
+  // every step without waiting (kernels of a stopped run return at once).  A
+  // sector that fits one work-group takes the whole run in one launch.
   double* cur = c.lz[0].as<double>();
   double* prev = c.lz[1].as<double>();
   double* out = c.lz[2].as<double>();
-  for (int k = 1; k <= nl; ++k) {
+  const bool whole = lanczos_run_fits(c.dev);
+  if (whole) dev_lanczos_run(c.dev, cur, nl, res, s);
+  for (int k = 1; !whole && k <= nl; ++k) {
     HvArgs a{};
     a.v = cur;
     a.w = out;

@@ -175,6 +175,7 @@ struct DevSpin {
   int32_t* sl_len = nullptr;
   uint32_t* ell = nullptr;
   uint32_t* lell = nullptr;  // ell's slots as line-pass entries
+  int max_hops = 0;          // entries of the longest row
   double vt16[4] = {0, 0, 0, 0};
   int nvt16 = 0;
   int32_t* q4_ptr = nullptr;
@@ -309,6 +310,10 @@ constexpr int kCtlCol = 0, kCtlPhase = 1, kCtlState = 2;
 void launch_hv(const DevSector& ds, const HvArgs& a, hipStream_t s, int variant = HV_AUTO);
 int hv_num_blocks(const DevSector& ds);
 int hv_choose(const DevSector& ds);
+// A whole Lanczos run in one launch, for sectors that fit one work-group
+// (lanczos_run.hip): res = {steps taken, stopped | alpha[nl] | beta[nl + 1]}.
+bool lanczos_run_fits(const DevSector& ds);
+void dev_lanczos_run(const DevSector& ds, const double* v0, int nl, double* res, hipStream_t s);
 
 // Two passes of LDS gathers over whole lines (hv_lines.hip): rows and columns
 // per work-group, work-group sizes and LDS of each pass, fixed by the sector

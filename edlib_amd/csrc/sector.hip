@@ -76,6 +76,8 @@ void upload_spin(Packer& pk, const SpinTables& sp, DevSpin& d, bool lines) {
   pk.add(d.ell_q4, sp.ell_q4);
   pk.add(d.ell_s4, sp.ell_s4);
   d.s4_scale = sp.s4_scale;
+  d.max_hops = 0;
+  for (size_t r = 0; r + 1 < sp.rowp.size(); ++r) d.max_hops = std::max(d.max_hops, sp.rowp[r + 1] - sp.rowp[r]);
 }
 
 // Reverse Cuthill-McKee order of the graph whose adjacency is the CSR
