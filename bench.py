@@ -400,7 +400,7 @@ def main():
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": load_traffic(chosen, kern_ms),
                      "kernel": {0: "edh::hv_rows_kernel (single pass)",
-                                1: "edh::hv_rows_kernel (no up term) + edh::hv_upslab_kernel (two passes)"}[chosen],
+                                1: "edh::hv_rows_kernel (no up term) + edh::hv_up_tiles_kernel (two passes)"}[chosen],
                      "kernel_ms": round(kern_ms, 4), "variants": per_variant},
     }
     out["pcie_inclusive_gbs"] = round(pcie_gbs, 2)

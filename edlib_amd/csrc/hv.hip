@@ -57,10 +57,13 @@ constexpr int kStage = 8;
 // of each chunk c0; a wavefront therefore covers exactly one ELL slice per j,
 // so slot counts are wavefront-uniform and the slot loops need no padding
 // beyond their own slice.
-// CTL: the operands are resolved from an eigensolver run's control block
-// (batch sweeps only; a separate instantiation keeps the other launches'
-// register allocation as it is).
-template <int J, int CROSS, bool KAN, bool LDS, int EF, bool UP, bool CTL>
+// RUN: the operands of an eigensolver run are resolved from its control block
+// (kRunCtl, batch sweeps only), the scales of a step of a single-sector Lanczos
+// run from the shares of its last norm (kRunLanczos; with lz.k = 0 as without).
+// Separate instantiations keep the other launches' register allocation as it
+// is (what a Lanczos step keeps to the kernel's end costs the signed form 2 %).
+enum { kRunNone = 0, kRunCtl = 1, kRunLanczos = 2 };
+template <int J, int CROSS, bool KAN, bool LDS, int EF, bool UP, int RUN>
 __global__ __launch_bounds__(1024) void hv_rows_kernel(HvParams p) {
   extern __shared__ double s_v[];
   __shared__ double s_red[16];
@@ -68,11 +71,22 @@ __global__ __launch_bounds__(1024) void hv_rows_kernel(HvParams p) {
   const int tid = threadIdx.x;
   const int Ddn = p.Ddn;
   const int na = 1 << (p.Ns - p.nb);
-  double vscale, wscale;
-  if (!hv_scales(p, s_red, blockIdx.x == 0, vscale, wscale)) return;
+  double vscale, wscale, beta = 0.0;
+  int rows = p.Dup;
+  if (RUN == kRunLanczos) {
+    const HvScales sc(p, s_red);
+    vscale = sc.v;
+    wscale = sc.w;
+    beta = sc.beta;
+    if (!sc.live) rows = 0;  // (no early exit: see HvScales::record)
+  } else {
+    if (p.done && *p.done) return;
+    vscale = p.dscale ? p.dscale[0] : p.vscale;
+    wscale = p.dscale ? p.dscale[1] : p.wscale;
+  }
   const double* __restrict__ V = p.v;
   double* __restrict__ W = p.w;
-  if (CTL) {
+  if (RUN == kRunCtl) {
     if (p.ctl[kCtlState] != 0.0) return;  // uniform over the grid
     const int64_t N = (int64_t)p.Dup * p.Ddn;
     const double* base = p.ctl[kCtlPhase] != 0.0 ? p.v_alt : p.v;
@@ -88,7 +102,7 @@ __global__ __launch_bounds__(1024) void hv_rows_kernel(HvParams p) {
   if (EF == 4)
     for (int i = tid; i < p.nvals; i += T) s_vals[i] = vals[i];
 
-  for (int slot0 = blockIdx.x; slot0 < p.Dup; slot0 += gridDim.x) {
+  for (int slot0 = blockIdx.x; slot0 < rows; slot0 += gridDim.x) {
     // work-groups go to the XCDs in turn (b mod 8): within each window of
     // 256 consecutive work-groups, XCD x takes 32 consecutive rows of the
     // order, so the rows in flight on one XCD share neighbour rows in its L2
@@ -375,7 +389,8 @@ __global__ __launch_bounds__(1024) void hv_rows_kernel(HvParams p) {
     }
     if (LDS) __syncthreads();
   }
-  if (UP && p.dot_partial) block_reduce_store(dsum, s_red, p.dot_partial + blockIdx.x);
+  if (UP && p.dot_partial && rows > 0) block_reduce_store(dsum, s_red, p.dot_partial + blockIdx.x);
+  if (RUN == kRunLanczos && blockIdx.x == 0) HvScales::record(p, vscale, beta, rows > 0);
 }
 
 // Several Lanczos operands of one sector in one launch (the batch's
@@ -827,9 +842,10 @@ Launch plan(const DevSector& ds) {
 
 template <int J, int CROSS, bool KAN, bool LDS, int EF>
 void launch_t(const HvParams& p, const Launch& L, bool up, hipStream_t s) {
-  auto k = !up     ? hv_rows_kernel<J, CROSS, KAN, LDS, EF, false, false>
-           : p.ctl ? hv_rows_kernel<J, CROSS, KAN, LDS, EF, true, true>
-                   : hv_rows_kernel<J, CROSS, KAN, LDS, EF, true, false>;
+  auto k = !up      ? hv_rows_kernel<J, CROSS, KAN, LDS, EF, false, kRunLanczos>
+           : p.ctl  ? hv_rows_kernel<J, CROSS, KAN, LDS, EF, true, kRunCtl>
+           : p.lz.k ? hv_rows_kernel<J, CROSS, KAN, LDS, EF, true, kRunLanczos>
+                    : hv_rows_kernel<J, CROSS, KAN, LDS, EF, true, kRunNone>;
   if (L.smem > 64 * 1024)
     EDH_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)L.smem));
   hipLaunchKernelGGL(k, dim3(L.grid), dim3(L.block), L.smem, s, p);
@@ -956,18 +972,21 @@ void launch_hv(const DevSector& ds, const HvArgs& a, hipStream_t s, int variant)
 
 // The variant of a single sector (an environment override EDH_HV_VARIANT=0/1
 // fixes it): the line passes by their own rule, else the tile pass from 4 M
-// states on.  Measured there (MI355X, us per H*v, single pass : two passes):
-//   16 sites, 12870 x 12870: 4x4 torus 4820 : 3470, ring 2973 : 2539, Anderson
-//     2802 : 2835, Kanamori 6329 : 5631; 12870 x 11440 all-to-all 9192 : 7498
-//   rectangular: 12870 x 1820 torus 580 : 454, ring 364 : 338; 1820 x 12870
-//     534 : 432, 334 : 335; 12870 x 4368 Anderson 1219 : 903; 4368 x 12870
-//     Kanamori 1986 : 1877; 12870 x 560 torus 213 : 199
-//   17 sites, 24310 x 19448: Anderson 8198 : 7792.
+// states on, with signed uniform hopping (whose single pass decodes an entry in
+// half the instructions) from 32 hops per state of both spins on.  Measured
+// (MI355X, us per H*v, single pass : two passes; hops):
+//   signed, 16 sites: 4x4 torus 12870 x 12870 (34) 3765 : 3291 (4806 : 3464
+//     back to back for seconds), 12870 x 1820 (30) 423 : 433; ring 12870 x
+//     12870 (17) 2098 : 2372, 12870 x 1820 252 : 318, 1820 x 12870 239 : 313
+//   other, 16 sites: Anderson 12870 x 12870 (16) 2796 : 2824, 12870 x 4368 1219
+//     : 903; Kanamori 12870 x 12870 6329 : 5631, 4368 x 12870 1986 : 1877;
+//     all-to-all 12870 x 11440 9192 : 7498; 17 sites, 24310 x 19448: Anderson
+//     8198 : 7792.
 int hv_choose(const DevSector& ds) {
   const char* env = getenv("EDH_HV_VARIANT");
   if (env && (env[0] == '0' || env[0] == '1')) return env[0] - '0';
   if (hv_lines_plan(ds).ok) return hv_lines_faster(ds) ? HV_TWO_PASS : HV_SINGLE;
-  return ds.N >= (1 << 22) ? HV_TWO_PASS : HV_SINGLE;
+  return ds.N >= (1 << 22) && (!ds.dn_signed || ds.hops >= 32) ? HV_TWO_PASS : HV_SINGLE;
 }
 
 }  // namespace edh

@@ -45,14 +45,16 @@ struct View {
   bool accum, live;
 };
 
-__device__ __forceinline__ View resolve_view(const HvBatchJob& J, double* s_red, bool first) {
+__device__ __forceinline__ View resolve_view(const HvBatchJob& J, const HvScales& sc) {
   const HvParams& p = J.p;
   View o;
   o.V = p.v;
   o.W = p.w;
   o.Wp = p.wprev;
   o.accum = p.accumulate != 0;
-  o.live = hv_scales(p, s_red, first, o.vs, o.ws);
+  o.live = sc.live;
+  o.vs = sc.v;
+  o.ws = sc.w;
   if (J.ctl) {  // eigensolver run: its basis column and buffer
     if (J.ctl[kCtlState] != 0.0) o.live = false;
     const int64_t N = (int64_t)p.Dup * p.Ddn;
@@ -464,7 +466,7 @@ __global__ __launch_bounds__(1024) void hv_row_lines_kernel(LinesArgs a, int nti
   extern __shared__ double s_line[];
   __shared__ double s_red[16];
   const HvBatchJob& j = a.j[blockIdx.y];
-  const View o = resolve_view(j, s_red, false);
+  const View o = resolve_view(j, HvScales(j.p, s_red));
   if (!o.live) return;
   Ahead<B, NI> f;
   int t = blockIdx.x;
@@ -484,10 +486,10 @@ __global__ __launch_bounds__(1024) void hv_col_lines_kernel(LinesArgs a, int nti
   extern __shared__ double s_line[];
   __shared__ double s_red[16];
   const HvBatchJob& j = a.j[blockIdx.y];
-  const View o = resolve_view(j, s_red, blockIdx.x == 0);
-  if (!o.live) return;
+  const HvScales sc(j.p, s_red);
+  const View o = resolve_view(j, sc);
   const int x = blockIdx.x & 7, step = gridDim.x >> 3;
-  const int t1 = min(ntiles, (x + 1) * per);  // this XCD's tiles: [x per, t1)
+  const int t1 = o.live ? min(ntiles, (x + 1) * per) : 0;  // this XCD's tiles: [x per, t1)
   Ahead<B, NI> f;
   int t = x * per + (blockIdx.x >> 3);
   if (t < t1) col_fetch<B, NI>(j, o, t * B, f, 0, NI);
@@ -496,6 +498,7 @@ __global__ __launch_bounds__(1024) void hv_col_lines_kernel(LinesArgs a, int nti
     col_tile<B, NI>(j, o, t * B, first, n < t1, n * B, f, s_line);
     t = n;
   }
+  if (blockIdx.x == 0) HvScales::record(j.p, sc.v, sc.beta, sc.live);
 }
 
 // Work-groups that stay on the chip for a launch: as many as the CUs hold at
@@ -567,7 +570,7 @@ int hv_lines_partials(const DevSector& ds) {
 //   13 sites, 2.9 M: Kanamori (32) 100 : 61, Anderson (13) 45.6 : 40.9, ring
 //     (14, signed uniform hopping) 37.6 : 43.2
 //   14 sites, 11.8 M: Kanamori (36) 378 : 203, Anderson (14) 175 : 125, 2x7
-//     torus (23, signed) 185 : 158, ring (15, signed) 141 : 139
+//     torus (23, signed) 178 : 156, ring (15, signed) 135 : 134
 //   15 sites, 41.4 M, two lines at a time: Kanamori (38) 1443 : 1134, Anderson
 //     (15) 651 : 711; 11 sites, 213,444: Kanamori (26) 10.9 : 14.8.
 // Two launches cost about 8 us before they gain, and the single pass's signed

@@ -18,7 +18,8 @@
 // of 16 columns in L2 took 3.5 ms.  Narrower slabs fit L2 but touch more lines
 // (a row of 12,870 elements is no multiple of a line) and take more address
 // work: 16 columns x 1024 rows 2.4 ms, 32 x 512 2.2 ms, 64 x 256 2.0 ms, 128 x
-// 128 2.4 ms.  The whole H*v of that sector: 4.9 -> 3.5 ms.
+// 128 2.4 ms.  The whole H*v of that sector, one after the other for seconds: 4.8
+// -> 3.5 ms (alone 3.8 -> 3.3: the single pass's 25 GB of gathers cost clock).
 #include <algorithm>
 
 #include "hv_params.h"
@@ -50,8 +51,9 @@ template <bool VEC>
 __global__ __launch_bounds__(kTileWG) void hv_up_tiles_kernel(HvParams p, int ntiles, int nslabs, int per) {
   extern __shared__ double s_tile[];  // the tile, a zero row, the value table
   __shared__ double s_red[16];
-  double vs, ws;
-  if (!hv_scales(p, s_red, false, vs, ws)) return;
+  const HvScales sc(p, s_red);
+  if (!sc.live) return;
+  const double vs = sc.v;
   const int Dup = p.Dup, Ddn = p.Ddn;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
