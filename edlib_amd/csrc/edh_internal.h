@@ -360,8 +360,10 @@ void launch_hv_batch(const void* djobs, const HvBatchUnit* dunits, int nunits, i
 bool hv_batch_routed(int64_t dup, int64_t ddn);
 // The same for Lanczos operands (Green's-function runs): also sectors of at
 // least 256 rows of 512..4608 elements whose format has the multi-operand
-// kernel, so that their runs share launches (the decision depends on the
-// sector only, so a run's arithmetic does not depend on the other runs).
+// kernel, so that their runs share launches, and sectors of kLinesLanczos
+// states and more where the line passes beat the single pass (the decision
+// depends on the sector only, so a run's arithmetic does not depend on the
+// other runs).
 bool hv_batch_routed_lanczos(const DevSector& ds);
 int64_t hv_batch_rows_partials(const DevSector& ds);
 void launch_hv_batch_rows(const DevSector& ds, const HvArgs& a, hipStream_t s);
