@@ -164,6 +164,20 @@ void build_sector(const Model& m, int nup, int ndn, SectorTables& st, bool need_
 // faster one.
 enum HvVariant { HV_SINGLE = 0, HV_TWO_PASS = 1, HV_AUTO = -1 };
 
+// Impurity terms by target and the row tiles they need (DevSector::row_tiles);
+// empty where the terms have no such form.
+constexpr int kOwnState = 4;  // kan_td of no state offset and no row offset
+struct RowTileTables {
+  int t = 0;
+  std::vector<int32_t> tiles, td;
+  std::vector<double> tc;
+};
+RowTileTables row_tile_tables(const SectorTables& st, int Ns);
+// The kan_td entry that slot r of a row tile with n rows follows: a slot past
+// the rows stands for the tile's first row, whose row offsets lead past the
+// tile from there, so it stays on its own (zero) state.
+__host__ __device__ inline int row_tile_entry(int r, int n, int td) { return r < n ? td : kOwnState; }
+
 // Device mirror of one sector.
 struct DevSpin {
   int64_t D = 0;
@@ -207,7 +221,7 @@ struct DevSector {
   // rows sharing their bath bits (row_tiles: four rows per tile, -1 = none):
   // up pattern a leads to at most kan_t up patterns; a down pattern b has at
   // most one term to target j, coefficient kan_tc (0: none) and kan_td =
-  // 8 * (state offset) + 4 + (row offset) at (a kan_t + j) 2^ml + b.
+  // 8 * (state offset) + kOwnState + (row offset) at (a kan_t + j) 2^ml + b.
   // row_tiles null: the terms have no such form, or more than three orbitals.
   int kan_t = 0, n_row_tiles = 0;
   int32_t* row_tiles = nullptr;

@@ -196,11 +196,11 @@ __device__ __forceinline__ void kan_targets(const HvParams& p, const double* tc,
     for (int r = 0; r < B; ++r) {
       const int q = (a[r] * p.kan_t + j) * na + b;
       c[r] = r < n ? tc[q] : 0.0;
-      at[r] = td[q];  // 8 * (state offset) + 4 + (row offset)
+      at[r] = row_tile_entry(r, n, td[q]);  // 8 * (state offset) + kOwnState + (row offset)
     }
 #pragma unroll
     for (int r = 0; r < B; ++r) {
-      const int rr = r + (at[r] & 7) - 4;  // the partner's row in the tile
+      const int rr = r + (at[r] & 7) - kOwnState;  // the partner's row in the tile
       x[r] = s[((size_t)(rr >> 1) * ld + d + (at[r] >> 3)) * 2 + (rr & 1)];
     }
     // (a state without this term must not pick up 0 * infinity)

@@ -114,13 +114,15 @@ std::vector<int32_t> rcm_order(const std::vector<int32_t>& rowp, const std::vect
   return order;
 }
 
-// Impurity terms by target and the row tiles they need (DevSector::row_tiles).
+}  // namespace
+
 // A run of rows sharing their bath bits has C(ml, k) <= 3 rows for up to
 // three orbitals; a tile takes a run of several rows and fills up with single
 // ones.
-void add_row_tiles(Packer& pk, const SectorTables& st, const std::vector<double>& kc, DevSector& ds) {
-  const int ml = st.kan_ml, na = 1 << ml, nb = ds.Ns - ml;
-  if (ml > 3) return;
+RowTileTables row_tile_tables(const SectorTables& st, int Ns) {
+  RowTileTables out;
+  const int ml = st.kan_ml, na = 1 << ml, nb = Ns - ml;
+  if (ml < 1 || ml > 3) return out;
   std::vector<std::vector<int>> tgt(na);
   int nt = 0;
   for (int a = 0; a < na; ++a) {
@@ -128,22 +130,22 @@ void add_row_tiles(Packer& pk, const SectorTables& st, const std::vector<double>
       if (std::find(tgt[a].begin(), tgt[a].end(), st.kan[q].new_a) == tgt[a].end()) tgt[a].push_back(st.kan[q].new_a);
     nt = std::max(nt, (int)tgt[a].size());
   }
-  if (nt == 0) return;
-  std::vector<int32_t> td((size_t)na * nt * na, 4);
+  if (nt == 0) return out;
+  std::vector<int32_t> td((size_t)na * nt * na, kOwnState);
   std::vector<double> tc(td.size(), 0.0);
   for (int a = 0; a < na; ++a)
     for (int b = 0; b < na; ++b)
       for (int q = st.kan_ptr[a * na + b]; q < st.kan_ptr[a * na + b + 1]; ++q) {
         const size_t j = std::find(tgt[a].begin(), tgt[a].end(), st.kan[q].new_a) - tgt[a].begin();
         const size_t at = ((size_t)a * nt + j) * na + b;
-        if (tc[at] != 0.0) return;  // two terms of (a, b) lead to this up pattern
+        if (tc[at] != 0.0) return out;  // two terms of (a, b) lead to this up pattern
         const int32_t lu = (int32_t)((1ll << (st.nup - __builtin_popcount(a))) - 1);
         const int32_t ld = (int32_t)((1ll << (st.ndn - __builtin_popcount(b))) - 1);
         const int du = st.up.rank[lu | (st.kan[q].new_a << nb)] - st.up.rank[lu | (a << nb)];
         const int dd = st.dn.rank[ld | (st.kan[q].new_b << nb)] - st.dn.rank[ld | (b << nb)];
-        if (du < -2 || du > 2) return;
-        td[at] = 8 * dd + 4 + du;
-        tc[at] = kc[q];
+        if (du < -2 || du > 2) return out;
+        td[at] = 8 * dd + kOwnState + du;
+        tc[at] = st.kan[q].coef;
       }
   // runs of rows with the same bath bits
   const int32_t bath = (int32_t)((1ll << nb) - 1);
@@ -151,7 +153,7 @@ void add_row_tiles(Packer& pk, const SectorTables& st, const std::vector<double>
   for (int64_t u = 0; u < st.up.D;) {
     int64_t e = u + 1;
     while (e < st.up.D && (st.up.bits[e] & bath) == (st.up.bits[u] & bath)) ++e;
-    if (e - u > 4) return;
+    if (e - u > 4) return out;
     if (e - u == 1) {
       single.push_back((int32_t)u);
     } else {
@@ -164,14 +166,12 @@ void add_row_tiles(Packer& pk, const SectorTables& st, const std::vector<double>
     if (t < 0 && next < single.size()) t = single[next++];
   while (next < single.size())
     for (int k = 0; k < 4; ++k) tiles.push_back(next < single.size() ? single[next++] : -1);
-  ds.kan_t = nt;
-  ds.n_row_tiles = (int)(tiles.size() / 4);
-  pk.add(ds.row_tiles, tiles);
-  pk.add(ds.kan_td, td);
-  pk.add(ds.kan_tc, tc);
+  out.t = nt;
+  out.tiles = std::move(tiles);
+  out.td = std::move(td);
+  out.tc = std::move(tc);
+  return out;
 }
-
-}  // namespace
 
 void DevSector::release() {
   for (void* p : allocs) (void)hipFreeAsync(p, astream);
@@ -285,7 +285,14 @@ void upload_sector(const SectorTables& st, int Ns, DevSector& ds, hipStream_t s,
     pk.add(ds.kan_off, koff);
     pk.add(ds.kan_c, kc);
     ds.nkan = (int)kc.size();
-    if (ds.lines) add_row_tiles(pk, st, kc, ds);
+    if (ds.lines) {
+      const RowTileTables r = row_tile_tables(st, Ns);
+      ds.kan_t = r.t;
+      ds.n_row_tiles = (int)(r.tiles.size() / 4);
+      pk.add(ds.row_tiles, r.tiles);
+      pk.add(ds.kan_td, r.td);
+      pk.add(ds.kan_tc, r.tc);
+    }
   }
   pk.add(ds.row_order, rcm_order(st.up.rowp, st.up.col, st.up.D));
   pk.commit(ds, s, stage);
