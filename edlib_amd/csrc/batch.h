@@ -216,6 +216,11 @@ struct Batch {
                int64_t* elements);
 
  private:
+  template <class F>
+  int add_job(F fill);
+  void fill_eig(BJob& j, int sec, int nev, int ncv, double tol, int maxitr, uint64_t seed);
+  void fill_lanczos(BJob& j, int sec, const double* v0_dev, int nl, bool init);
+  void start_gf(const std::vector<GfRequest>& req, int nl, std::vector<int>& ids, std::vector<int>& made, void*& d);
   double* dalloc(BJob& j, size_t count);
   void release_job(BJob& j);
   bool drain_slab(bool wait);

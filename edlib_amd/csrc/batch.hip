@@ -1255,23 +1255,38 @@ void Batch::finish_dense(BJob& j) {
   j.state = JOB_DONE;
 }
 
-int Batch::submit_eig(int sec, int nev_req, int ncv_req, double tol, int maxitr, uint64_t seed) {
-  BSector& s = sector(sec);
-  EDH_CHECK(nev_req >= 1 && ncv_req >= 2, EDH_ERR_ARG, "batch: bad nev/ncv");
+// A process joins the batch once it is complete: a sweep never sees one whose
+// memory or scalars are missing, and a submission that fails leaves nothing.
+template <class F>
+int Batch::add_job(F fill) {
   auto jp = std::make_unique<BJob>();
-  BJob& j = *jp;
+  try {
+    fill(*jp);
+    jobs.push_back(std::move(jp));
+  } catch (...) {
+    if (jp) release_job(*jp);
+    throw;
+  }
+  return (int)jobs.size() - 1;
+}
+
+int Batch::submit_eig(int sec, int nev_req, int ncv_req, double tol, int maxitr, uint64_t seed) {
+  EDH_CHECK(nev_req >= 1 && ncv_req >= 2, EDH_ERR_ARG, "batch: bad nev/ncv");
+  return add_job([&](BJob& j) { fill_eig(j, sec, nev_req, ncv_req, tol, maxitr, seed); });
+}
+
+void Batch::fill_eig(BJob& j, int sec, int nev_req, int ncv_req, double tol, int maxitr, uint64_t seed) {
+  BSector& s = sector(sec);
   j.kind = JOB_EIG;
   j.sec = sec;
   j.n = s.tabs.N;
   j.tol = tol;
   j.maxitr = maxitr;
-  jobs.push_back(std::move(jp));
-  const int id = (int)jobs.size() - 1;
   const int64_t n = j.n;
   if (n == 0) {
     j.nev = 0;
     j.state = JOB_DONE;
-    return id;
+    return;
   }
   if (n == 1) {  // Storage.h:49-52 and the one-state eigenpair (SpinResolvedStorage.h:52-56)
     j.nev = 1;
@@ -1282,13 +1297,13 @@ int Batch::submit_eig(int sec, int nev_req, int ncv_req, double tol, int maxitr,
     EDH_HIP(hipStreamSynchronize(stream));
     j.nconv = 1;
     j.state = JOB_DONE;
-    return id;
+    return;
   }
   const int ncv = (int)std::min<int64_t>(ncv_req, n);
   j.nev = std::min(nev_req, ncv - 1);
   if (ncv >= n || n <= 64) {
     finish_dense(j);
-    return id;
+    return;
   }
   j.m = std::min(ncv, kMaxBasis - 1);
   EDH_CHECK(j.nev < j.m - 1, EDH_ERR_LIMIT, "batch: NEV too large for the device Krylov basis (max 46)");
@@ -1305,25 +1320,24 @@ int Batch::submit_eig(int sec, int nev_req, int ncv_req, double tol, int maxitr,
   dev_random_uniform(j.V, n, seed, stream);
   j.pending_start_norm = true;  // normalised by the next sweep
   j.state = JOB_ACTIVE;
-  return id;
 }
 
 int Batch::submit_lanczos(int sec, const double* v0_dev, int nl, bool init) {
-  BSector& s = sector(sec);
   EDH_CHECK(nl >= 1, EDH_ERR_ARG, "batch: nl must be >= 1");
-  auto jp = std::make_unique<BJob>();
-  BJob& j = *jp;
+  return add_job([&](BJob& j) { fill_lanczos(j, sec, v0_dev, nl, init); });
+}
+
+void Batch::fill_lanczos(BJob& j, int sec, const double* v0_dev, int nl, bool init) {
+  BSector& s = sector(sec);
   j.kind = JOB_LZ;
   j.sec = sec;
   j.n = s.tabs.N;
   j.nl = nl;
   j.alpha.assign(nl, 0.0);
   j.beta.assign(nl + 1, 0.0);
-  jobs.push_back(std::move(jp));
-  const int id = (int)jobs.size() - 1;
   if (j.n == 0) {
     j.state = JOB_DONE;
-    return id;
+    return;
   }
   // one allocation per run (one stream-ordered free when it ends): the
   // three vectors, the scalars (alpha history (nl), beta history (nl + 1),
@@ -1350,7 +1364,6 @@ int Batch::submit_lanczos(int sec, const double* v0_dev, int nl, bool init) {
     EDH_HIP(hipMemcpyAsync(j.lz[0], v0_dev, (size_t)j.n * sizeof(double), hipMemcpyDeviceToDevice, stream));
   j.step = 1;
   j.state = JOB_ACTIVE;
-  return id;
 }
 
 // Device gather maps of c / c^+ on `orb` out of sector src (the single-sector
@@ -1391,6 +1404,7 @@ void Batch::gather_maps(const std::vector<MapKey>& keys) {
   std::shared_ptr<void> owner(base, [this](void* p) { defer_free(p); });
   int c = -1;
   char* h = uploads.take(tot, c);
+  std::map<MapKey, GatherMaps> made;  // known to later submissions once their copy is on its way
   for (const Piece& p : fresh) {
     GatherMaps g;
     g.owner = owner;
@@ -1400,10 +1414,11 @@ void Batch::gather_maps(const std::vector<MapKey>& keys) {
       g.m[q] = reinterpret_cast<const int32_t*>(static_cast<char*>(base) + p.off[q]);
       g.s[q] = reinterpret_cast<const int8_t*>(static_cast<char*>(base) + p.off[2 + q]);
     }
-    maps[p.key] = g;
+    made[p.key] = g;
   }
   EDH_HIP(hipMemcpyAsync(base, h, tot, hipMemcpyHostToDevice, stream));
   uploads.mark(c, stream);
+  maps.merge(made);
 }
 
 // Green's-function start vectors c(+)_orb |psi> (GreensFunction.h:395-416,
@@ -1417,7 +1432,6 @@ void Batch::gather_maps(const std::vector<MapKey>& keys) {
 void Batch::submit_gf(const std::vector<GfRequest>& req, int nl, std::vector<int>& ids) {
   EDH_CHECK(nl >= 1, EDH_ERR_ARG, "batch: nl must be >= 1");
   ids.assign(req.size(), -1);
-  OpGroup g{G_NORM, {}};
   std::vector<MapKey> keys;
   for (const GfRequest& q : req) {
     BJob& e = job(q.eig_job);
@@ -1439,13 +1453,37 @@ void Batch::submit_gf(const std::vector<GfRequest>& req, int nl, std::vector<int
     if (q.orb2 >= 0) keys.push_back({e.sec, q.orb2, q.annihilate ? 1 : 0});
   }
   gather_maps(keys);
+  std::vector<int> made;
+  void* d = nullptr;  // descriptors of the start launch
+  try {
+    start_gf(req, nl, ids, made, d);
+  } catch (...) {
+    // the runs have no scalars or start vectors yet, and nobody knows them
+    for (int id : made) {
+      release_job(*jobs[id]);
+      jobs[id].reset();
+    }
+    defer_free(d);
+    ids.assign(req.size(), -1);
+    throw;
+  }
+  defer_free(d);  // stream-ordered: freed after the kernel
+}
+
+// The runs of a checked submission, their start vectors and norms; made lists
+// the runs created so far.
+void Batch::start_gf(const std::vector<GfRequest>& req, int nl, std::vector<int>& ids, std::vector<int>& made,
+                     void*& d) {
+  OpGroup g{G_NORM, {}};
   std::vector<GfStart> runs;
   std::vector<int2> work;
+  made.reserve(req.size());
   for (size_t r = 0; r < req.size(); ++r) {
     const GfRequest& q = req[r];
     const BSector& b = sector(q.dst_sec);
     if (b.tabs.N == 0) continue;
     const int id = submit_lanczos(q.dst_sec, nullptr, nl, false);
+    made.push_back(id);
     BJob& j = job(id);
     const BJob& e = job(q.eig_job);
     const GatherMaps& m = maps.at({e.sec, q.orb, q.annihilate ? 1 : 0});
@@ -1484,7 +1522,6 @@ void Batch::submit_gf(const std::vector<GfRequest>& req, int nl, std::vector<int
   }
   if (!runs.empty()) {
     const size_t rb = align16(runs.size() * sizeof(GfStart)), wb = work.size() * sizeof(int2);
-    void* d = nullptr;
     EDH_HIP(hipMallocAsync(&d, rb + wb, stream));
     int c = -1;
     char* h = uploads.take(rb + wb, c);
@@ -1495,7 +1532,6 @@ void Batch::submit_gf(const std::vector<GfRequest>& req, int nl, std::vector<int
     hipLaunchKernelGGL(bgf_start_kernel, dim3((unsigned)work.size()), dim3(kOpBlock), 0, stream,
                        (const GfStart*)d, (const int2*)(static_cast<char*>(d) + rb));
     EDH_HIP(hipGetLastError());
-    defer_free(d);  // stream-ordered: freed after the kernel
   }
   std::vector<OpGroup> pre{g}, post;
   issue(pre, nullptr, post);
