@@ -347,8 +347,7 @@ int edh_alloc(edh_ctx* ctx, size_t bytes, void** dptr) {
   require_ctx(ctx);
   EDH_CHECK(dptr, EDH_ERR_ARG, "null argument");
   use_device(ctx->c);
-  hipError_t e = hipMalloc(dptr, bytes);
-  EDH_CHECK(e == hipSuccess, EDH_ERR_NOMEM, std::string("hipMalloc failed: ") + hipGetErrorString(e));
+  check_alloc(hipMalloc(dptr, bytes), "hipMalloc");
   API_END
 }
 

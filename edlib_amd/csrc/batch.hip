@@ -1039,8 +1039,7 @@ double* Batch::dalloc(BJob& j, size_t count) {
   const size_t bytes = std::max<size_t>(count, 1) * sizeof(double);
   // stream-ordered: every reader and writer of a job's memory runs on the
   // batch stream, so the memory can return to the pool in stream order
-  hipError_t e = hipMallocAsync(&p, bytes, stream);
-  if (e != hipSuccess) throw Error(EDH_ERR_NOMEM, std::string("batch: hipMallocAsync failed: ") + hipGetErrorString(e));
+  check_alloc(hipMallocAsync(&p, bytes, stream), "batch: hipMallocAsync");
   j.allocs.push_back(p);
   j.bytes += bytes;
   bytes_in_use += bytes;
@@ -2162,7 +2161,10 @@ int Batch::autotune(const std::vector<int>& sec_ids) {
   int64_t tot = 0;
   for (int id : ids) tot += secs[id]->tabs.N;
   double* scratch = nullptr;
-  if (hipMalloc(&scratch, (size_t)2 * tot * sizeof(double)) != hipSuccess) return hv_block;
+  if (hipMalloc(&scratch, (size_t)2 * tot * sizeof(double)) != hipSuccess) {
+    (void)hipGetLastError();  // not an error of the next launch
+    return hv_block;
+  }
   hipLaunchKernelGGL(bfill_kernel, dim3(1024), dim3(256), 0, stream, scratch, 2 * tot, 0.0);
   std::vector<std::pair<int, HvArgs>> hv;
   int64_t off = 0;

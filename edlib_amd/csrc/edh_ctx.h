@@ -16,8 +16,7 @@ struct DevBuf {
     p = nullptr;
     bytes = 0;
     if (b == 0) return;
-    hipError_t e = hipMalloc(&p, b);
-    if (e != hipSuccess) throw Error(EDH_ERR_NOMEM, std::string("hipMalloc failed: ") + hipGetErrorString(e));
+    check_alloc(hipMalloc(&p, b), "hipMalloc");
     bytes = b;
   }
   void release() {

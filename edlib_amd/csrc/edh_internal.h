@@ -23,12 +23,23 @@ struct Error : public std::runtime_error {
   Error(int c, const std::string& m) : std::runtime_error(m), code(c) {}
 };
 
+// A reported error is taken off the runtime's record, which keeps it until it
+// is asked for: the next check of a launch would report it again.
 #define EDH_HIP(call)                                                                              \
   do {                                                                                             \
     hipError_t e_ = (call);                                                                        \
-    if (e_ != hipSuccess)                                                                          \
+    if (e_ != hipSuccess) {                                                                        \
+      (void)hipGetLastError();                                                                     \
       throw ::edh::Error(EDH_ERR_HIP, std::string(#call) + ": " + hipGetErrorString(e_));          \
+    }                                                                                              \
   } while (0)
+
+// The same for an allocation.
+inline void check_alloc(hipError_t e, const char* what) {
+  if (e == hipSuccess) return;
+  (void)hipGetLastError();
+  throw Error(EDH_ERR_NOMEM, std::string(what) + " failed: " + hipGetErrorString(e));
+}
 
 #define EDH_CHECK(cond, code, msg)                 \
   do {                                             \

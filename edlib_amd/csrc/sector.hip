@@ -30,8 +30,7 @@ class Packer {
   void commit(DevSector& ds, hipStream_t s, UploadStage* stage) {
     if (blob_.empty()) return;
     void* p = nullptr;
-    hipError_t e = hipMallocAsync(&p, blob_.size(), s);
-    if (e != hipSuccess) throw Error(EDH_ERR_NOMEM, std::string("hipMallocAsync failed: ") + hipGetErrorString(e));
+    check_alloc(hipMallocAsync(&p, blob_.size(), s), "hipMallocAsync");
     ds.allocs.push_back(p);
     if (stage) {
       int c = -1;

@@ -37,3 +37,20 @@ def test_failed_submission_leaves_nothing(tmp_path, what):
     print(failed)
     """ % what)
     assert int(out) >= 1
+
+
+def test_next_submission_does_not_report_the_error_again(tmp_path):
+    """The runtime keeps an error until it is asked for; a failed submission
+    must not show up in the check of another request's launch."""
+    fake_device.run(tmp_path, SETUP + """
+    for submit in (lambda: b.submit_gf(reqs, 10), lambda: b.submit_eig(sid[3, 3], 2, 8),
+                   lambda: b.submit_lanczos(sid[3, 3], np.ones(400), 10), lambda: b.add_sector(m, 4, 4)):
+        fake.fake_fail_alloc(1)
+        try:
+            submit()
+            raise SystemExit("the submission did not fail")
+        except ea.EdhError:
+            pass
+        fake.fake_fail_alloc(0)
+        b.submit_gf(reqs, 10)
+    """)
