@@ -57,11 +57,11 @@ Ctx::~Ctx() {
   small.release();
   gtab.release();
   obs.release();
-  if (pin) (void)hipHostFree(pin);
   if (stream) {
     (void)hipStreamSynchronize(stream);  // the tables return to the pool in stream order
     (void)hipStreamDestroy(stream);
   }
+  release_pinned();
 }
 
 namespace {
@@ -279,6 +279,7 @@ int edh_create(edh_ctx** out, int device) {
   c->c.device = device;
   EDH_HIP(hipSetDevice(device));
   EDH_HIP(hipStreamCreate(&c->c.stream));
+  c->c.pin = edh::pinned_take(Ctx::kPinned, c->c.pin_count);
   edh::configure_mem_pool(device);
   edh::noalloc_register_device(device);
   *out = c.release();

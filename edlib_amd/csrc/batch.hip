@@ -29,7 +29,6 @@
 #include <cstdio>
 #include <cstring>
 #include <memory>
-#include <mutex>
 #include <numeric>
 #include <thread>
 
@@ -969,39 +968,6 @@ int chunk_of(int64_t n) {
 int nchunks(int64_t n) { return (int)((n + chunk_of(n) - 1) / chunk_of(n)); }
 
 size_t align16(size_t x) { return (x + 15) & ~size_t(15); }
-
-// Pinned status read-back buffers outlive their batch: a released buffer
-// is kept for the next batch of the process, since allocating and freeing
-// pinned memory costs about a millisecond per call.
-std::mutex g_pinned_mu;
-std::vector<std::pair<double*, size_t>> g_pinned_free;  // (buffer, capacity in doubles)
-
-double* pinned_take(size_t need, size_t& cap) {
-  {
-    std::lock_guard<std::mutex> lk(g_pinned_mu);
-    size_t best = g_pinned_free.size();
-    for (size_t q = 0; q < g_pinned_free.size(); ++q)
-      if (g_pinned_free[q].second >= need &&
-          (best == g_pinned_free.size() || g_pinned_free[q].second < g_pinned_free[best].second))
-        best = q;
-    if (best < g_pinned_free.size()) {
-      const auto r = g_pinned_free[best];
-      g_pinned_free.erase(g_pinned_free.begin() + (std::ptrdiff_t)best);
-      cap = r.second;
-      return r.first;
-    }
-  }
-  double* h = nullptr;
-  EDH_HIP(hipHostMalloc((void**)&h, need * sizeof(double)));
-  cap = need;
-  return h;
-}
-
-// Only once no copy into the buffer is pending.
-void pinned_give(double* h, size_t cap) {
-  std::lock_guard<std::mutex> lk(g_pinned_mu);
-  g_pinned_free.push_back({h, cap});
-}
 
 }  // namespace
 

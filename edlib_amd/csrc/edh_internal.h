@@ -268,6 +268,14 @@ struct UploadStage {
   void release();  // after the stream has finished every copy
 };
 
+// Pinned host buffers for small reads and writes outlive the batch or context
+// that took them: a returned one is kept (at most 64) for the next, since
+// allocating and freeing pinned memory costs about a millisecond per call.
+// cap: the buffer's capacity in doubles, at least `need`.  A buffer is returned
+// once no copy into or out of it is pending.
+double* pinned_take(size_t need, size_t& cap);
+void pinned_give(double* h, size_t cap);
+
 // Uploads a sector's tables in one allocation and one copy.  Without a
 // stage the call waits for the copy (and then times the H*v variants);
 // with one it returns at once and the variants are not timed.

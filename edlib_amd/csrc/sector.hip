@@ -3,6 +3,7 @@
 #include <cstdint>
 #include <cstring>
 #include <functional>
+#include <mutex>
 
 #include "edh_internal.h"
 
@@ -186,6 +187,44 @@ void configure_mem_pool(int device) {
   uint64_t keep = UINT64_MAX;
   EDH_HIP(hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep));
   done[device] = true;
+}
+
+namespace {
+std::mutex g_pinned_mu;
+std::vector<std::pair<double*, size_t>> g_pinned_free;  // (buffer, capacity in doubles)
+constexpr size_t kPinnedKept = 64;
+}  // namespace
+
+double* pinned_take(size_t need, size_t& cap) {
+  {
+    std::lock_guard<std::mutex> lk(g_pinned_mu);
+    size_t best = g_pinned_free.size();
+    for (size_t q = 0; q < g_pinned_free.size(); ++q)
+      if (g_pinned_free[q].second >= need &&
+          (best == g_pinned_free.size() || g_pinned_free[q].second < g_pinned_free[best].second))
+        best = q;
+    if (best < g_pinned_free.size()) {
+      const auto r = g_pinned_free[best];
+      g_pinned_free.erase(g_pinned_free.begin() + (std::ptrdiff_t)best);
+      cap = r.second;
+      return r.first;
+    }
+  }
+  double* h = nullptr;
+  EDH_HIP(hipHostMalloc((void**)&h, need * sizeof(double)));
+  cap = need;
+  return h;
+}
+
+void pinned_give(double* h, size_t cap) {
+  {
+    std::lock_guard<std::mutex> lk(g_pinned_mu);
+    if (g_pinned_free.size() < kPinnedKept) {
+      g_pinned_free.push_back({h, cap});
+      return;
+    }
+  }
+  (void)hipHostFree(h);
 }
 
 char* UploadStage::take(size_t bytes, int& c) {
