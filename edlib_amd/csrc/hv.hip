@@ -389,7 +389,12 @@ __global__ __launch_bounds__(1024) void hv_rows_kernel(HvParams p) {
     }
     if (LDS) __syncthreads();
   }
-  if (UP && p.dot_partial && rows > 0) block_reduce_store(dsum, s_red, p.dot_partial + blockIdx.x);
+  if (UP && p.dot_partial && rows > 0) {
+    // (a slower wavefront may still be reading the scales' shares in s_red;
+    // with rows in LDS their barriers lie in between)
+    if (!LDS && RUN == kRunLanczos) __syncthreads();
+    block_reduce_store(dsum, s_red, p.dot_partial + blockIdx.x);
+  }
   if (RUN == kRunLanczos && blockIdx.x == 0) HvScales::record(p, vscale, beta, rows > 0);
 }
 
