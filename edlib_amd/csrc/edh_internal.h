@@ -216,7 +216,8 @@ struct DevSector {
   double* values = nullptr;
   int nvalues = 0;  // entries of values
   int nkan = 0;     // impurity terms (entries of kan_off and kan_c)
-  bool lines = false;      // the line passes' tables are there
+  bool lines = false;      // the line passes' entries can hold the sector's columns
+  bool two_pass = false;   // the two passes' tables are there
   bool dn_signed = false;  // the down spin has the signed byte-offset form (ell_s4)
   double hops = 0;  // mean hopping entries per state, both spins
   int imp_ml = 0;
@@ -277,9 +278,14 @@ double* pinned_take(size_t need, size_t& cap);
 void pinned_give(double* h, size_t cap);
 
 // Uploads a sector's tables in one allocation and one copy.  Without a
-// stage the call waits for the copy (and then times the H*v variants);
-// with one it returns at once and the variants are not timed.
+// stage the call waits for the copy and sets the variant that hv_choose gives
+// by rule; with one it returns at once.  The two passes' tables are among them
+// only where they are taken (half filled ring of 8 sites: 23.6 KB instead of
+// 29.7; 11-site three-orbital impurity 141 KB instead of 216).
 void upload_sector(const SectorTables& st, int Ns, DevSector& ds, hipStream_t s, UploadStage* stage = nullptr);
+
+// The two passes' tables of a sector that was uploaded without them.
+void hv_two_pass_tables(const SectorTables& st, DevSector& ds, hipStream_t s);
 
 // Keeps freed stream-ordered allocations in the device's default pool (no
 // return to the driver at synchronisations), so that allocation in the
@@ -364,6 +370,7 @@ int hv_lines_threads(int64_t D);
 int hv_lines_partials(const DevSector& ds);  // shares of <v, w> per operand
 bool hv_lines_faster(const DevSector& ds);   // than the single pass, for one operand alone
 constexpr int kLinesMax = 4;  // operands per launch
+constexpr int64_t kLinesMin = 400000;  // smallest sector for which the line passes are taken
 constexpr int64_t kLinesLanczos = 2500000;  // smallest sector whose Lanczos operands take them in a batch
 void launch_hv_lines(const DevSector& ds, const HvArgs* ops, int count, hipStream_t s);
 

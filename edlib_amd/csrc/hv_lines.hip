@@ -518,7 +518,7 @@ size_t pair_up(size_t n) { return (n + 1) & ~size_t(1); }
 
 size_t row_smem(const DevSector& ds, int B) {
   size_t d = (size_t)B * (ds.dn.D + 1) + (size_t)ds.nvalues;
-  if (ds.row_tiles && B == 4) {
+  if (ds.n_row_tiles > 0 && B == 4) {
     const size_t nk = ((size_t)1 << (2 * ds.kan_ml)) * ds.kan_t;
     d += nk + (nk + 1) / 2;
   }
@@ -541,7 +541,7 @@ int hv_lines_threads(int64_t D) {
 
 namespace {
 int row_tiles(const DevSector& ds, const HvLinesPlan& L) {
-  return L.row_b == 4 && ds.row_tiles ? ds.n_row_tiles : (int)((ds.up.D + L.row_b - 1) / L.row_b);
+  return L.row_b == 4 && ds.n_row_tiles > 0 ? ds.n_row_tiles : (int)((ds.up.D + L.row_b - 1) / L.row_b);
 }
 }  // namespace
 
@@ -576,8 +576,9 @@ int hv_lines_partials(const DevSector& ds) {
 // Two launches cost about 8 us before they gain, and the single pass's signed
 // form decodes an entry in half the instructions.
 bool hv_lines_faster(const DevSector& ds) {
+  if (ds.N < kLinesMin) return false;
   const HvLinesPlan L = hv_lines_plan(ds);
-  if (!L.ok || ds.N < 400000) return false;
+  if (!L.ok) return false;
   if (L.row_b < 4 || L.col_b < 4) return ds.hops >= 30;
   if (ds.N < 2500000) return ds.hops >= 28;
   return ds.hops >= (ds.dn_signed ? 20 : 12);
@@ -585,7 +586,7 @@ bool hv_lines_faster(const DevSector& ds) {
 
 void launch_hv_lines(const DevSector& ds, const HvArgs* ops, int count, hipStream_t s) {
   const HvLinesPlan L = hv_lines_plan(ds);
-  EDH_CHECK(L.ok, EDH_ERR_INTERNAL, "H*v lines: the sector's lines do not fit LDS");
+  EDH_CHECK(L.ok && ds.two_pass, EDH_ERR_INTERNAL, "H*v lines: the sector has no tables for them");
   EDH_CHECK(count >= 1 && count <= kLinesMax, EDH_ERR_INTERNAL, "H*v lines: operand count");
   LinesArgs a;
   for (int q = 0; q < count; ++q) {

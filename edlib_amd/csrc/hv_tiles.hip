@@ -225,7 +225,7 @@ void up_tile_tables(const SpinTables& sp, std::vector<int32_t>& slices, std::vec
 int hv_up_tiles_blocks(const DevSector& ds) { return tile_grid(ds).grid; }
 
 void launch_hv_up_tiles(const DevSector& ds, const HvParams& p, hipStream_t s) {
-  EDH_CHECK(ds.up_slices, EDH_ERR_INTERNAL, "H*v tiles: the sector has no tables for them");
+  EDH_CHECK(ds.two_pass && ds.up_slices, EDH_ERR_INTERNAL, "H*v tiles: the sector has no tables for them");
   const TileGrid g = tile_grid(ds);
   const size_t smem = ((size_t)(kTileRows + 1) * kTileW + ds.nvalues) * sizeof(double);
   const bool vec = ds.dn.D % 2 == 0 && ((uintptr_t)p.v | (uintptr_t)p.w) % 16 == 0;

@@ -60,7 +60,7 @@ std::vector<uint32_t> line_entries(const SpinTables& sp) {
   return out;
 }
 
-void upload_spin(Packer& pk, const SpinTables& sp, DevSpin& d, bool lines) {
+void upload_spin(Packer& pk, const SpinTables& sp, DevSpin& d) {
   d.D = sp.D;
   pk.add(d.bits, sp.bits);
   pk.add(d.ediag, sp.ediag);
@@ -69,7 +69,6 @@ void upload_spin(Packer& pk, const SpinTables& sp, DevSpin& d, bool lines) {
   pk.add(d.sl_ptr, sp.sl_ptr);
   pk.add(d.sl_len, sp.sl_len);
   pk.add(d.ell, sp.ell);
-  if (lines) pk.add(d.lell, line_entries(sp));
   for (int q = 0; q < 4; ++q) d.vt16[q] = sp.vt16[q];
   d.nvt16 = sp.nvt16;
   pk.add(d.q4_ptr, sp.q4_ptr);
@@ -262,6 +261,38 @@ void UploadStage::release() {
   chunks.clear();
 }
 
+namespace {
+
+// Geometry of the impurity terms' row tiles (their tables are returned).
+RowTileTables set_row_tiles(const SectorTables& st, DevSector& ds) {
+  RowTileTables r;
+  if (ds.lines && st.kan_ml > 0) r = row_tile_tables(st, ds.Ns);
+  ds.kan_t = r.t;
+  ds.n_row_tiles = (int)(r.tiles.size() / 4);
+  return r;
+}
+
+// Tables of the line passes, or of the tile pass where lines do not fit.
+void add_two_pass(Packer& pk, const SectorTables& st, DevSector& ds) {
+  const RowTileTables r = set_row_tiles(st, ds);
+  if (hv_lines_plan(ds).ok) {
+    pk.add(ds.up.lell, line_entries(st.up));
+    pk.add(ds.dn.lell, line_entries(st.dn));
+    pk.add(ds.row_tiles, r.tiles);
+    pk.add(ds.kan_td, r.td);
+    pk.add(ds.kan_tc, r.tc);
+    return;
+  }
+  std::vector<int32_t> slices;
+  std::vector<uint32_t> in, out;
+  up_tile_tables(st.up, slices, in, out);
+  pk.add(ds.up_slices, slices);
+  pk.add(ds.up_in, in);
+  pk.add(ds.up_out, out);
+}
+
+}  // namespace
+
 void upload_sector(const SectorTables& st, int Ns, DevSector& ds, hipStream_t s, UploadStage* stage) {
   ds.release();
   ds.astream = s;
@@ -278,13 +309,9 @@ void upload_sector(const SectorTables& st, int Ns, DevSector& ds, hipStream_t s,
   ds.up.D = st.up.D;
   ds.dn.D = st.dn.D;
   ds.dn_signed = !st.dn.ell_s4.empty();
-  // the line passes' tables: in a batch where its Lanczos operands take them,
-  // for a single sector (no stage) wherever they apply, since the caller may
-  // ask for that variant
   ds.lines = std::max(st.up.D, st.dn.D) < (1 << (kLineOff - 4)) - 1;
-  if (stage) ds.lines = st.N >= kLinesLanczos && hv_lines_faster(ds);
-  upload_spin(pk, st.up, ds.up, ds.lines);
-  upload_spin(pk, st.dn, ds.dn, ds.lines);
+  upload_spin(pk, st.up, ds.up);
+  upload_spin(pk, st.dn, ds.dn);
   pk.add(ds.values, st.values);
   ds.cross_mode = st.cross_mode;
   ds.cross_u = st.cross_u;
@@ -323,30 +350,29 @@ void upload_sector(const SectorTables& st, int Ns, DevSector& ds, hipStream_t s,
     pk.add(ds.kan_off, koff);
     pk.add(ds.kan_c, kc);
     ds.nkan = (int)kc.size();
-    if (ds.lines) {
-      const RowTileTables r = row_tile_tables(st, Ns);
-      ds.kan_t = r.t;
-      ds.n_row_tiles = (int)(r.tiles.size() / 4);
-      pk.add(ds.row_tiles, r.tiles);
-      pk.add(ds.kan_td, r.td);
-      pk.add(ds.kan_tc, r.tc);
-    }
+    if (st.N >= kLinesMin) (void)set_row_tiles(st, ds);  // the choice below depends on their LDS
   }
   pk.add(ds.row_order, rcm_order(st.up.rowp, st.up.col, st.up.D));
+  // the two passes' tables where they are taken by themselves: in a batch by
+  // its Lanczos operands, else by the sector's own choice
+  const int variant = stage ? HV_SINGLE : hv_choose(ds);
+  const bool two_pass =
+      ds.N > 0 && (stage ? st.N >= kLinesLanczos && hv_lines_faster(ds) : variant == HV_TWO_PASS);
+  if (two_pass) add_two_pass(pk, st, ds);
   pk.commit(ds, s, stage);
+  ds.two_pass = two_pass;
   if (stage) return;
-  Packer tiles;
-  if (ds.N > 0 && !hv_lines_plan(ds).ok) {
-    std::vector<int32_t> slices;
-    std::vector<uint32_t> in, out;
-    up_tile_tables(st.up, slices, in, out);
-    tiles.add(ds.up_slices, slices);
-    tiles.add(ds.up_in, in);
-    tiles.add(ds.up_out, out);
-    tiles.commit(ds, s, nullptr);
-  }
   EDH_HIP(hipStreamSynchronize(s));
-  ds.variant = hv_choose(ds);
+  ds.variant = variant;
+}
+
+void hv_two_pass_tables(const SectorTables& st, DevSector& ds, hipStream_t s) {
+  if (ds.two_pass || ds.N == 0) return;
+  Packer pk;
+  add_two_pass(pk, st, ds);
+  pk.commit(ds, s, nullptr);
+  EDH_HIP(hipStreamSynchronize(s));
+  ds.two_pass = true;
 }
 
 }  // namespace edh
