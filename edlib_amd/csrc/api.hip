@@ -440,9 +440,11 @@ int edh_set_hv_variant(edh_ctx* ctx, int variant) {
   require_sector(c);
   use_device(c);
   EDH_CHECK(variant >= -1 && variant <= 1, EDH_ERR_ARG, "variant must be -1, 0 or 1");
-  const int take = variant < 0 ? hv_choose(c.dev) : variant;
-  if (take == HV_TWO_PASS) hv_two_pass_tables(c.tabs, c.dev, c.stream);
+  const int take = variant < 0 ? hv_choose(c.dev, false) : variant;
+  const int in_place = variant < 0 ? hv_choose(c.dev, true) : variant;
+  if (take == HV_TWO_PASS || in_place == HV_TWO_PASS) hv_two_pass_tables(c.tabs, c.dev, c.stream);
   c.dev.variant = take;
+  c.dev.variant_in_place = in_place;
   API_END
 }
 

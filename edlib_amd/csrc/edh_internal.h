@@ -218,7 +218,7 @@ struct DevSector {
   int nkan = 0;     // impurity terms (entries of kan_off and kan_c)
   bool lines = false;      // the line passes' entries can hold the sector's columns
   bool two_pass = false;   // the two passes' tables are there
-  bool dn_signed = false;  // the down spin has the signed byte-offset form (ell_s4)
+  int dn_form = 2;  // the down spin's entries in the single pass: 0 signed (ell_s4), 1 compact (ell_q4), 2 plain
   double hops = 0;  // mean hopping entries per state, both spins
   int imp_ml = 0;
   int cross_mode = 0;
@@ -241,6 +241,7 @@ struct DevSector {
   double* kan_tc = nullptr;
   int32_t* row_order = nullptr;  // processing order of up rows
   int variant = HV_SINGLE;       // chosen H*v variant
+  int variant_in_place = HV_SINGLE;  // the same for w = H v + w in place (edh_av's accumulated form)
   // the up spin's entries for the tile pass (up_tile_tables), where the line
   // passes do not apply
   int32_t* up_slices = nullptr;
@@ -348,7 +349,7 @@ constexpr int kCtlCol = 0, kCtlPhase = 1, kCtlState = 2;
 
 void launch_hv(const DevSector& ds, const HvArgs& a, hipStream_t s, int variant = HV_AUTO);
 int hv_num_blocks(const DevSector& ds);
-int hv_choose(const DevSector& ds);
+int hv_choose(const DevSector& ds, bool in_place);
 // A whole Lanczos run in one launch, for sectors that fit one work-group
 // (lanczos_run.hip): res = {steps taken, stopped | alpha[nl] | beta[nl + 1]}.
 bool lanczos_run_fits(const DevSector& ds);
@@ -368,9 +369,10 @@ void up_tile_tables(const SpinTables& sp, std::vector<int32_t>& slices, std::vec
                     std::vector<uint32_t>& out);
 int hv_lines_threads(int64_t D);
 int hv_lines_partials(const DevSector& ds);  // shares of <v, w> per operand
-bool hv_lines_faster(const DevSector& ds);   // than the single pass, for one operand alone
+// than the single pass, for one operand alone; in_place: w = H v + w
+bool hv_lines_faster(const DevSector& ds, bool in_place = false);
 constexpr int kLinesMax = 4;  // operands per launch
-constexpr int64_t kLinesMin = 400000;  // smallest sector for which the line passes are taken
+constexpr int64_t kLinesMin = 500000;  // smallest sector for which the line passes are taken
 constexpr int64_t kLinesLanczos = 2500000;  // smallest sector whose Lanczos operands take them in a batch
 void launch_hv_lines(const DevSector& ds, const HvArgs* ops, int count, hipStream_t s);
 

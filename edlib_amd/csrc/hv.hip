@@ -960,7 +960,7 @@ int hv_num_blocks(const DevSector& ds) {
 
 void launch_hv(const DevSector& ds, const HvArgs& a, hipStream_t s, int variant) {
   if (ds.N == 0) return;
-  if (variant == HV_AUTO) variant = ds.variant;
+  if (variant == HV_AUTO) variant = a.mode && a.wprev == a.w ? ds.variant_in_place : ds.variant;
   if (variant == HV_TWO_PASS && hv_lines_plan(ds).ok) return launch_hv_lines(ds, &a, 1, s);
   Launch L = plan(ds);
   HvParams p = make_params(ds, a);
@@ -979,22 +979,39 @@ void launch_hv(const DevSector& ds, const HvArgs& a, hipStream_t s, int variant)
 }
 
 // The variant of a single sector (an environment override EDH_HV_VARIANT=0/1
-// fixes it): the line passes by their own rule, else the tile pass from 4 M
-// states on, with signed uniform hopping (whose single pass decodes an entry in
-// half the instructions) from 32 hops per state of both spins on.  Measured
-// (MI355X, us per H*v, single pass : two passes; hops):
-//   signed, 16 sites: 4x4 torus 12870 x 12870 (34) 3765 : 3291 (4806 : 3464
-//     back to back for seconds), 12870 x 1820 (30) 423 : 433; ring 12870 x
-//     12870 (17) 2098 : 2372, 12870 x 1820 252 : 318, 1820 x 12870 239 : 313
-//   other, 16 sites: Anderson 12870 x 12870 (16) 2796 : 2824, 12870 x 4368 1219
-//     : 903; Kanamori 12870 x 12870 6329 : 5631, 4368 x 12870 1986 : 1877;
-//     all-to-all 12870 x 11440 9192 : 7498; 17 sites, 24310 x 19448: Anderson
-//     8198 : 7792.
-int hv_choose(const DevSector& ds) {
+// fixes it): where lines fit LDS by their own rule, else the tile pass from 4 M
+// states on where the hops of both spins per state are enough of them.  What is
+// enough depends on how cheaply the single pass decodes an entry (signed,
+// compact, plain) and on the shape: the up-spin gathers that the tiles save grow
+// with D_up, while a long row's other work is the single pass's anyway.  Measured
+// (MI355X, single pass / two passes at hops; rings of one to four neighbours,
+// tori, impurities of one to three orbitals, disordered; 12870 x 4368 also
+// stands for 24310 x 2380, 4368 x 12870 for 2380 x 24310):
+//   signed   0.92 at 17, 1.17 at 34 (12870 x 12870 1.15); wide 0.84 at 16, 1.06
+//     at 32; 12870 x 4368 1.02 at 16, 1.24 at 32; 1820 x 12870 0.99 at 30, 1.11
+//     at 45
+//   compact  0.92 at 33, 1.01..1.07 at 49, 1.08..1.14 at 66; 12870 x 4368 1.07
+//     at 32, 12870 x 1820 0.93 at 30 and 1.06 at 45; 4368 x 12870 0.94 at 48,
+//     1.01 at 63; 1820 x 12870 0.95 at 60
+//   plain    0.94..1.04 at 15, 1.03..1.09 at 29..34; 12870 x 4368 1.27 at 15
+//     (12870 x 1820 0.92, 1.07 at 30); 4368 x 12870 0.88 at 15, 1.00 at 28, 1.04
+//     at 48, Kanamori 1.06 at 39; 1820 x 12870 0.99 at 45, 1.01 at 60
+// In place the ratios are 0.01 to 0.05 lower.
+int hv_choose(const DevSector& ds, bool in_place) {
   const char* env = getenv("EDH_HV_VARIANT");
   if (env && (env[0] == '0' || env[0] == '1')) return env[0] - '0';
-  if (hv_lines_plan(ds).ok) return hv_lines_faster(ds) ? HV_TWO_PASS : HV_SINGLE;
-  return ds.N >= (1 << 22) && (!ds.dn_signed || ds.hops >= 32) ? HV_TWO_PASS : HV_SINGLE;
+  if (hv_lines_plan(ds).ok) return hv_lines_faster(ds, in_place) ? HV_TWO_PASS : HV_SINGLE;
+  if (ds.N < (1 << 22)) return HV_SINGLE;
+  const int64_t up = ds.up.D, dn = ds.dn.D;
+  double need = 32;  // hops per state
+  if (ds.dn_form != 0) {
+    if (dn > 4 * up) return HV_SINGLE;
+    const bool compact = ds.dn_form == 1;
+    if (dn > 2 * up) need = compact ? 62 : ds.kan_ml > 0 ? 37 : 45;
+    else if (up >= 2 * dn) need = compact ? 40 : dn >= 2048 ? 14 : 28;
+    else need = compact ? 48 : 28;
+  }
+  return ds.hops >= need ? HV_TWO_PASS : HV_SINGLE;
 }
 
 }  // namespace edh

@@ -563,25 +563,47 @@ int hv_lines_partials(const DevSector& ds) {
   return L.ok ? row_tiles(ds, L) : 0;
 }
 
-// The two passes against the single pass for one operand (MI355X, us per H*v,
-// single pass : lines; hops = mean entries per state of both spins):
-//   12 sites, 853,776 states: 3x4 torus t, t' (52 hops) 29.9 : 21.3, Kanamori
-//     (30) 27.8 : 21.2, 3x4 torus (26) 18.4 : 18.1, Anderson (12) 13.0 : 15.7
-//   13 sites, 2.9 M: Kanamori (32) 100 : 61, Anderson (13) 45.6 : 40.9, ring
-//     (14, signed uniform hopping) 37.6 : 43.2
-//   14 sites, 11.8 M: Kanamori (36) 378 : 203, Anderson (14) 175 : 125, 2x7
-//     torus (23, signed) 178 : 156, ring (15, signed) 135 : 134
-//   15 sites, 41.4 M, two lines at a time: Kanamori (38) 1443 : 1134, Anderson
-//     (15) 651 : 711; 11 sites, 213,444: Kanamori (26) 10.9 : 14.8.
-// Two launches cost about 8 us before they gain, and the single pass's signed
-// form decodes an entry in half the instructions.
-bool hv_lines_faster(const DevSector& ds) {
+// The two passes against the single pass for one operand: the hops of both
+// spins per state from which on they are faster, by what the single pass's
+// entry costs to decode (signed, compact, plain).  In place (w = H v + w) the
+// column pass reads w in pieces of 32 bytes, so it takes more.  Measured
+// (MI355X, single pass / two passes at hops, in place behind the comma; rings
+// of one to four neighbours, tori, impurities of one to three orbitals,
+// disordered):
+//   four lines at a time, 0.6 to 2.5 M states: signed 924 x 924 1.02, 0.87 at 39
+//     and 1.22, 1.05 at 66; compact 0.89, 0.76 at 26, 1.10, 0.94 at 39, 1.26,
+//     1.08 at 52; plain 1.11, 0.92 at 26, 1.29, 1.07 at 39, Kanamori 1.23, 1.04
+//     at 30, disordered 1.47, 1.24 at 29
+//   below that two launches are most of the time: 495 x 924 and 924 x 495 0.74
+//     to 1.03, in place 0.56 to 0.97 at any hops; 715 x 715 signed 0.96, compact
+//     1.05, plain 1.16 at 48, disordered (general cross term) 1.31, 1.16 at 29
+//   from 2.5 M on: signed 2002 x 2002 1.00, 0.84 at 21, 1.14, 0.96 at 28, 1.38,
+//     1.17 at 42 (3432 x 3432 1.14, 0.95 at 23, 1.31, 1.10 at 30); compact 0.87,
+//     0.72 at 14, 1.24, 1.04 at 28; plain 1.08, 0.89 at 14, 1.42, 1.17 at 28
+//     (3003 x 3003 and 3432 x 3432 1.42 to 1.6, 1.11 to 1.24 at 14)
+//   one spin two lines at a time (3003 x 6435, 6435 x 3003): signed 0.96 to
+//     1.00, 0.84 to 0.89 at 30, 1.16, 1.03 at 45; compact 1.13, 0.97 at 30, 1.30,
+//     1.13 at 45; plain 1.37, 1.18 at 30
+//   both spins (5005 .. 8008): signed 0.83 to 0.94, 0.68 to 0.82 at 32, 1.04 to
+//     1.12, 0.89 to 0.99 at 48, 1.02 to 1.12 in place at 63; compact 0.96, 0.78 at
+//     32, 1.12, 0.95 at 47, 1.21, 1.08 at 63; plain 1.14, 0.94 at 31, 1.31, 1.11
+//     at 47
+bool hv_lines_faster(const DevSector& ds, bool in_place) {
   if (ds.N < kLinesMin) return false;
   const HvLinesPlan L = hv_lines_plan(ds);
   if (!L.ok) return false;
-  if (L.row_b < 4 || L.col_b < 4) return ds.hops >= 30;
-  if (ds.N < 2500000) return ds.hops >= 28;
-  return ds.hops >= (ds.dn_signed ? 20 : 12);
+  static const double small[2][3] = {{39, 36, 28}, {56, 45, 34}};
+  static const double large[2][3] = {{21, 20, 12}, {34, 28, 22}};
+  static const double mixed[2][3] = {{36, 30, 30}, {45, 36, 30}};
+  static const double pairs[2][3] = {{46, 40, 30}, {62, 54, 40}};
+  const int q = in_place ? 1 : 0, f = ds.dn_form;
+  const bool general = f == 2 && ds.cross_mode == CROSS_GENERAL;
+  if (L.row_b < 4 && L.col_b < 4) return ds.hops >= pairs[q][f];
+  if (L.row_b < 4 || L.col_b < 4) return ds.hops >= mixed[q][f];
+  if (ds.N >= 2500000) return ds.hops >= (in_place && f == 2 && ds.N >= 9000000 ? 12 : large[q][f]);
+  if (ds.N < 600000) return general && ds.hops >= 28;
+  // (the single pass's terms beyond the hopping make up for six hops)
+  return ds.hops >= (in_place && f == 2 && (general || ds.kan_ml > 0) ? 28 : small[q][f]);
 }
 
 void launch_hv_lines(const DevSector& ds, const HvArgs* ops, int count, hipStream_t s) {

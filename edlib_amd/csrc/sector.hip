@@ -308,7 +308,7 @@ void upload_sector(const SectorTables& st, int Ns, DevSector& ds, hipStream_t s,
             (double)st.dn.col.size() / (double)std::max<int64_t>(st.dn.D, 1);
   ds.up.D = st.up.D;
   ds.dn.D = st.dn.D;
-  ds.dn_signed = !st.dn.ell_s4.empty();
+  ds.dn_form = !st.dn.ell_s4.empty() ? 0 : !st.dn.ell_q4.empty() ? 1 : 2;
   ds.lines = std::max(st.up.D, st.dn.D) < (1 << (kLineOff - 4)) - 1;
   upload_spin(pk, st.up, ds.up);
   upload_spin(pk, st.dn, ds.dn);
@@ -355,15 +355,16 @@ void upload_sector(const SectorTables& st, int Ns, DevSector& ds, hipStream_t s,
   pk.add(ds.row_order, rcm_order(st.up.rowp, st.up.col, st.up.D));
   // the two passes' tables where they are taken by themselves: in a batch by
   // its Lanczos operands, else by the sector's own choice
-  const int variant = stage ? HV_SINGLE : hv_choose(ds);
-  const bool two_pass =
-      ds.N > 0 && (stage ? st.N >= kLinesLanczos && hv_lines_faster(ds) : variant == HV_TWO_PASS);
+  const int variant = stage ? HV_SINGLE : hv_choose(ds, false), in_place = stage ? HV_SINGLE : hv_choose(ds, true);
+  const bool two_pass = ds.N > 0 && (stage ? st.N >= kLinesLanczos && hv_lines_faster(ds)
+                                           : variant == HV_TWO_PASS || in_place == HV_TWO_PASS);
   if (two_pass) add_two_pass(pk, st, ds);
   pk.commit(ds, s, stage);
   ds.two_pass = two_pass;
   if (stage) return;
   EDH_HIP(hipStreamSynchronize(s));
   ds.variant = variant;
+  ds.variant_in_place = in_place;
 }
 
 void hv_two_pass_tables(const SectorTables& st, DevSector& ds, hipStream_t s) {

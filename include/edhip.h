@@ -172,8 +172,9 @@ int edh_static_observables(edh_ctx* ctx, const double* v, int64_t n, int mem, in
 /* H*v kernel variant of the current sector: 0 = single pass (rows), 1 = two
  * passes (whole columns, then whole rows gathered in LDS where several of each
  * fit; else rows, then tiles of rows and columns for the up-spin term).  The
- * sector set-up takes the faster one by a rule on the sector;
- * edh_set_hv_variant fixes one of them (-1: choose again). */
+ * sector set-up takes the faster one by a rule on the sector, and by another
+ * for w = H v + w (clear = 0), which may take the single pass where w = H v takes
+ * two; edh_set_hv_variant fixes one of them for both (-1: choose again). */
 int edh_get_hv_variant(edh_ctx* ctx, int* variant);
 int edh_set_hv_variant(edh_ctx* ctx, int variant);
 
