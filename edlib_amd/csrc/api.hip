@@ -521,17 +521,29 @@ int lanczos_device(Ctx& c, int nl, double* alpha, double* beta, double* step_ms)
     return 1;
   }
   const int ndot = hv_num_blocks(c.dev), nshare = lanczos_update_grid(n);
-  c.partial.ensure((size_t)(ndot + nshare) * sizeof(double));
+  // The sums that work-groups repeat are taken once, in a launch of their own,
+  // where there are many.  MI355X, us a step of a ring, single pass (four
+  // launches with a captured graph : two launches : scales once : shares folded
+  // : both): 2002 rows, 4.0 M states 78 : 70.8 : 69.0 : 70.8 : 69.3; 3432 rows,
+  // 11.8 M 218 : 223 : 206 : 222 : 205, 48 k 23.8 : 16.0 : 17.9 : 15.3 : 17.0;
+  // 6435 rows, 19.3 M 376 : 387 : 357 : 383 : 353, 0.68 M 42.1 : 35.6 : 33.6 :
+  // 31.2 : 29.5; 24310 rows, 57.9 M 1343 : 1406 : 1303 : 1378 : 1275; 184756 rows,
+  // 3.7 M 428 : 500 : 428 : 323 : 252.
+  const int groups = hv_num_groups(c.dev);
+  const bool scale_once = groups >= 6000 || (groups >= 2000 && n >= 1000000), fold = ndot >= 3000;
+  c.partial.ensure((size_t)(ndot + nshare + kLzFold) * sizeof(double));
   double* dot = c.partial.as<double>();
   double* share = dot + ndot;
-  // {stop state, alpha[nl], beta[nl + 1]} (read back in one copy), scale[nl + 1]
+  double* folded = share + nshare;
+  // {stop state, alpha[nl], beta[nl + 1]} (read back in one copy), scale[nl + 1], scale pair
   const size_t nres = 1 + (size_t)nl + (size_t)nl + 1;
-  c.scal.ensure((nres + (size_t)nl + 1) * sizeof(double));
+  c.scal.ensure((nres + (size_t)nl + 3) * sizeof(double));
   double* res = c.scal.as<double>();
   int* st = (int*)res;
   double* dalpha = res + 1;
   double* dbeta = dalpha + nl;
   double* scale = dbeta + nl + 1;
+  double* pair = scale + nl + 1;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (step_ms) {
     EDH_HIP(hipEventCreate(&e0));
@@ -562,8 +574,15 @@ int lanczos_device(Ctx& c, int nl, double* alpha, double* beta, double* step_ms)
     a.step.scale = scale;
     a.step.beta = dbeta;
     a.step.st = st;
+    if (scale_once) {
+      dev_lanczos_scale(a.step, pair, s);
+      a.step = LzStep();
+      a.dscale = pair;
+      a.done = st + 1;
+    }
     launch_hv(c.dev, a, s);
-    dev_lanczos_update(out, cur, n, dot, ndot, scale, dalpha, st, k, share, s);
+    if (fold) dev_lanczos_fold(dot, ndot, st, folded, s);
+    dev_lanczos_update(out, cur, n, fold ? folded : dot, fold ? kLzFold : ndot, scale, dalpha, st, k, share, s);
     double* t = prev;
     prev = cur;
     cur = out;

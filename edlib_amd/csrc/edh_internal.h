@@ -349,6 +349,7 @@ constexpr int kCtlCol = 0, kCtlPhase = 1, kCtlState = 2;
 
 void launch_hv(const DevSector& ds, const HvArgs& a, hipStream_t s, int variant = HV_AUTO);
 int hv_num_blocks(const DevSector& ds);
+int hv_num_groups(const DevSector& ds);  // work-groups of its first launch that form a Lanczos step's scales
 int hv_choose(const DevSector& ds, bool in_place);
 // A whole Lanczos run in one launch, for sectors that fit one work-group
 // (lanczos_run.hip): res = {steps taken, stopped | alpha[nl] | beta[nl + 1]}.

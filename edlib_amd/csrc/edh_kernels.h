@@ -33,6 +33,12 @@ void dev_combine(const double* V, int64_t n, int m, const double* C, int k, doub
 // shares of |w|^2.  w and x 16-byte aligned.
 constexpr int kLzShares = 512;
 int lanczos_update_grid(int64_t n);
+// The same sums taken once, for sectors of many rows: the step's scales into
+// pair (then the H*v takes them as dscale, and st[1] as done), the H*v's shares
+// into kLzFold.
+constexpr int kLzFold = 256;
+void dev_lanczos_scale(const LzStep& step, double* pair, hipStream_t s);
+void dev_lanczos_fold(const double* dot, int ndot, const int* st, double* out, hipStream_t s);
 void dev_lanczos_update(double* w, const double* x, int64_t n, const double* dot, int ndot, const double* scale,
                         double* alpha, const int* st, int k, double* share, hipStream_t s);
 

@@ -958,6 +958,10 @@ int hv_num_blocks(const DevSector& ds) {
   return hv_up_tiles_blocks(ds);
 }
 
+int hv_num_groups(const DevSector& ds) {
+  return ds.variant == HV_TWO_PASS && hv_lines_plan(ds).ok ? 0 : plan(ds).grid;  // (the line passes' stay: few)
+}
+
 void launch_hv(const DevSector& ds, const HvArgs& a, hipStream_t s, int variant) {
   if (ds.N == 0) return;
   if (variant == HV_AUTO) variant = a.mode && a.wprev == a.w ? ds.variant_in_place : ds.variant;

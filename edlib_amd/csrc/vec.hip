@@ -92,6 +92,33 @@ __global__ __launch_bounds__(kVecBlock) void lanczos_update_kernel(double* __res
   if (threadIdx.x == 0) share[blockIdx.x] = t;
 }
 
+// A step of a sector with many rows: what every work-group of its H*v and every
+// block of its update would sum again is summed once, in two launches of their
+// own.
+//   scale: the sums of HvScales, left as {scale of v_k, of v_{k-1}} for the H*v
+//   fold:  the H*v's shares of <v, w> into kLzFold
+__global__ __launch_bounds__(kVecBlock) void lanczos_scale_kernel(LzStep lz, double* __restrict__ pair) {
+  __shared__ double s_red[16];
+  HvParams p;
+  p.lz = lz;
+  const HvScales sc(p, s_red);
+  if (threadIdx.x != 0) return;
+  pair[0] = sc.v;
+  pair[1] = sc.w;
+  HvScales::record(p, sc.v, sc.beta, sc.live);
+}
+
+__global__ __launch_bounds__(64) void lanczos_fold_kernel(const double* __restrict__ dot, int ndot,
+                                                          const int* __restrict__ st, double* __restrict__ out) {
+  if (st[1]) return;
+  const int per = (ndot + gridDim.x - 1) / gridDim.x;
+  const int e1 = min(ndot, ((int)blockIdx.x + 1) * per);
+  double x = 0.0;
+  for (int i = blockIdx.x * per + threadIdx.x; i < e1; i += 64) x += dot[i];
+  for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
+  if (threadIdx.x == 0) out[blockIdx.x] = x;
+}
+
 // ---- Gram-Schmidt of a new basis vector (eigensolver) ----------------------
 // w (column cnt of V) against columns 0..cnt-1 by classical Gram-Schmidt, a
 // second pass where ARPACK dsaitr's DGKS test asks for it (the first pass
@@ -459,6 +486,16 @@ int lanczos_update_grid(int64_t n) {
   // four elements a thread, at most 512 blocks (their shares are summed by
   // every work-group of the next H*v)
   return (int)std::min<int64_t>(std::max<int64_t>((n + 4 * kVecBlock - 1) / (4 * kVecBlock), 1), kLzShares);
+}
+
+void dev_lanczos_scale(const LzStep& step, double* pair, hipStream_t s) {
+  hipLaunchKernelGGL(lanczos_scale_kernel, dim3(1), dim3(kVecBlock), 0, s, step, pair);
+  EDH_HIP(hipGetLastError());
+}
+
+void dev_lanczos_fold(const double* dot, int ndot, const int* st, double* out, hipStream_t s) {
+  hipLaunchKernelGGL(lanczos_fold_kernel, dim3(kLzFold), dim3(64), 0, s, dot, ndot, st, out);
+  EDH_HIP(hipGetLastError());
 }
 
 void dev_lanczos_update(double* w, const double* x, int64_t n, const double* dot, int ndot, const double* scale,
