@@ -61,52 +61,64 @@ __device__ __forceinline__ bool exceeds(cplx d, double big) {
   return m > 0.5 * big && hypot(d.re, d.im) > big;
 }
 
-// Lanczos.h:201-224 at the point z.
-__device__ __forceinline__ cplx fraction(cplx z, int n, int isign, double weight, const double* alpha,
-                                         const double* beta) {
+// Coefficients staged in LDS, kCfLds steps at a time from the last one down,
+// and a step's pair read while the one before is computed: the recurrence is a
+// serial chain, and a global read per step was the longest part of it (256
+// points, whole call: 500 steps 146 us with every read global, 107 staged, 100
+// with the pair read ahead; 1500 steps 343, 364 with blocks of one wavefront and
+// nothing staged beyond 1024, 250 now).
+constexpr int kCfLds = 1024;
+
+// Lanczos.h:201-224 at the point z; all threads of the block take part, those
+// that are not live compute nothing.
+__device__ __forceinline__ cplx fraction(bool live, cplx z, int n, int isign, double weight, const double* alpha,
+                                         const double* beta, double2* s_ab) {
   const double big = (double)FLT_MAX / 2.0;
   const double shift = 1.0 / ((double)FLT_MAX / 1000.0);
   if (n == 1) return cdiv({weight, 0.0}, {z.re - alpha[0] * isign, z.im});
-  const cplx dl1 = {z.re - alpha[n - 1] * isign, z.im};
-  const cplx dl2 = {z.re - alpha[n - 2] * isign, z.im};
-  cplx dA = dl1;                                                    // det[i+2]
-  cplx dB = csub(cmul(dl2, dl1), {beta[n - 1] * beta[n - 1], 0.0});  // det[i+1]
-  for (int i = n - 3; i >= 0; --i) {
-    const cplx dli = {z.re - alpha[i] * isign, z.im};
-    const double b2 = beta[i + 1] * beta[i + 1];
-    cplx d = csub(cmul(dli, dB), cscale(dA, b2));
-    if (exceeds(d, big) && i != 0) {
-      d = cscale(d, shift);
-      dB = cscale(dB, shift);
+  cplx dA = z, dB = z;
+  for (int hi = n; hi > 0; hi -= kCfLds) {
+    const int lo = hi > kCfLds ? hi - kCfLds : 0;
+    if (hi < n) __syncthreads();  // the steps above are done with
+    // s_ab[i - lo] = {alpha_i, beta_{i+1}}
+    for (int i = lo + threadIdx.x; i < hi; i += blockDim.x)
+      s_ab[i - lo] = make_double2(alpha[i], i + 1 < n ? beta[i + 1] : 0.0);
+    __syncthreads();
+    if (!live) continue;
+    int k = hi - lo - 1;
+    if (hi == n) {
+      const double b = s_ab[k - 1].y;
+      const cplx dl1 = {z.re - s_ab[k].x * isign, z.im};
+      const cplx dl2 = {z.re - s_ab[k - 1].x * isign, z.im};
+      dA = dl1;                                 // det[i+2]
+      dB = csub(cmul(dl2, dl1), {b * b, 0.0});  // det[i+1]
+      k -= 2;
     }
-    dA = dB;
-    dB = d;
+    double2 c = s_ab[max(k, 0)];
+    for (; k >= 0; --k) {
+      const double2 ab = c;
+      c = s_ab[max(k - 1, 0)];
+      const cplx dli = {z.re - ab.x * isign, z.im};
+      const double b2 = ab.y * ab.y;
+      cplx d = csub(cmul(dli, dB), cscale(dA, b2));
+      if (exceeds(d, big) && k + lo != 0) {
+        d = cscale(d, shift);
+        dB = cscale(dB, shift);
+      }
+      dA = dB;
+      dB = d;
+    }
   }
-  return cdiv(cscale(dA, weight), dB);
-}
-
-// Coefficients of up to kCfLds steps are staged in LDS: the recurrence is a
-// serial chain, and a global read per step was the longest part of it.
-constexpr int kCfLds = 1024;
-
-__device__ __forceinline__ cplx fraction_staged(bool live, cplx z, int n, int isign, double weight,
-                                                const double* alpha, const double* beta, double* s_ab) {
-  if (n > kCfLds) return live ? fraction(z, n, isign, weight, alpha, beta) : z;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    s_ab[i] = alpha[i];
-    s_ab[n + i] = beta[i];
-  }
-  __syncthreads();
-  return live ? fraction(z, n, isign, weight, s_ab, s_ab + n) : z;
+  return live ? cdiv(cscale(dA, weight), dB) : z;
 }
 
 __global__ __launch_bounds__(64) void cf_kernel(int nz, const double* zre, const double* zim, double ev, int nlanc,
                                                 int isign, double expb, const double* alpha, const double* beta,
                                                 double* out_re, double* out_im) {
-  __shared__ double s_ab[2 * kCfLds];
+  __shared__ double2 s_ab[kCfLds];
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   const int at = min(q, nz - 1);
-  const cplx res = fraction_staged(q < nz, {zre[at], zim[at]}, nlanc, isign, ev * expb, alpha, beta, s_ab);
+  const cplx res = fraction(q < nz, {zre[at], zim[at]}, nlanc, isign, ev * expb, alpha, beta, s_ab);
   if (q >= nz) return;
   out_re[q] = res.re;
   out_im[q] = res.im;
@@ -116,14 +128,14 @@ __global__ __launch_bounds__(64) void cf_kernel(int nz, const double* zre, const
 // points z = excited_j * isign_j + i wn[q].
 __global__ __launch_bounds__(64) void cf_batch_kernel(int nz, const double* wr, const double* wn, const CfJob* jobs,
                                                       double* out_re, double* out_im) {
-  __shared__ double s_ab[2 * kCfLds];
+  __shared__ double2 s_ab[kCfLds];
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   const int at = min(q, nz - 1);
   const CfJob& J = jobs[blockIdx.y];
   // z = freq_point + isign * E (Lanczos.h:146-148): i w_n on the Matsubara
   // mesh (wr null), w + i pi/beta on the real axis
   const cplx z = {(wr ? wr[at] : 0.0) + J.excited * J.isign, wn[at]};
-  const cplx res = fraction_staged(q < nz, z, J.nlanc, J.isign, J.ev * J.expb, J.alpha, J.beta, s_ab);
+  const cplx res = fraction(q < nz, z, J.nlanc, J.isign, J.ev * J.expb, J.alpha, J.beta, s_ab);
   if (q >= nz) return;
   out_re[(size_t)blockIdx.y * nz + q] = res.re;
   out_im[(size_t)blockIdx.y * nz + q] = res.im;
