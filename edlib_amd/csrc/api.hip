@@ -61,7 +61,6 @@ Ctx::~Ctx() {
     (void)hipStreamSynchronize(stream);  // the tables return to the pool in stream order
     (void)hipStreamDestroy(stream);
   }
-  release_pinned();
 }
 
 namespace {
@@ -279,7 +278,7 @@ int edh_create(edh_ctx** out, int device) {
   c->c.device = device;
   EDH_HIP(hipSetDevice(device));
   EDH_HIP(hipStreamCreate(&c->c.stream));
-  c->c.pin = edh::pinned_take(Ctx::kPinned, c->c.pin_count);
+  (void)PinnedLease(1, c->c.stream);  // the process's first one is allocated here, not in a call
   edh::configure_mem_pool(device);
   edh::noalloc_register_device(device);
   *out = c.release();
@@ -597,7 +596,8 @@ int lanczos_device(Ctx& c, int nl, double* alpha, double* beta, double* step_ms)
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
   }
-  double* h = c.pinned(nres);
+  const PinnedLease lease(nres, s);
+  double* h = lease.get();
   EDH_HIP(hipMemcpyAsync(h, res, nres * sizeof(double), hipMemcpyDeviceToHost, s));
   EDH_HIP(hipStreamSynchronize(s));
   int host_st[2];
@@ -744,7 +744,8 @@ int edh_cf_eval(edh_ctx* ctx, int nz, const double* zre, const double* zim, doub
   double* dz = c.small.as<double>();
   double* da = dz + 2 * (size_t)nz;
   double* dr = dz + nin;
-  double* h = c.pinned(nin + nout);
+  const PinnedLease lease(nin + nout, c.stream);
+  double* h = lease.get();
   std::copy(zre, zre + nz, h);
   std::copy(zim, zim + nz, h + nz);
   std::copy(alpha, alpha + nlanc, h + 2 * (size_t)nz);

@@ -47,32 +47,6 @@ struct Ctx {
   DevBuf gtab;              // gather tables for a_adag / operators
   DevBuf obs;               // static-observable row sums and column tiles
   int n_evecs = 0;
-  // Pinned host memory for small reads and writes (one call at a time uses it):
-  // taken when the context is created, so that no call pays for the usual
-  // sizes; a longer run or mesh replaces it by a larger one.
-  static constexpr size_t kPinned = 16384;  // doubles: a basis of 47, 4096 points, 8000 steps
-  double* pin = nullptr;
-  size_t pin_count = 0;
-  bool pin_grown = false;  // not one of pinned_take's
-  double* pinned(size_t count) {
-    if (count > pin_count) {
-      size_t cap = kPinned;
-      while (cap < count) cap *= 2;
-      double* p = nullptr;
-      EDH_HIP(hipHostMalloc((void**)&p, cap * sizeof(double)));
-      release_pinned();
-      pin = p;
-      pin_count = cap;
-      pin_grown = true;
-    }
-    return pin;
-  }
-  void release_pinned() {  // no copy pending
-    if (pin && pin_grown) (void)hipHostFree(pin);
-    else if (pin) pinned_give(pin, pin_count);
-    pin = nullptr;
-    pin_count = 0;
-  }
   ~Ctx();
 };
 

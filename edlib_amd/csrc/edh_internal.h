@@ -5,6 +5,7 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <exception>
 #include <map>
 #include <memory>
 #include <stdexcept>
@@ -270,13 +271,36 @@ struct UploadStage {
   void release();  // after the stream has finished every copy
 };
 
-// Pinned host buffers for small reads and writes outlive the batch or context
-// that took them: a returned one is kept (at most 64) for the next, since
-// allocating and freeing pinned memory costs about a millisecond per call.
-// cap: the buffer's capacity in doubles, at least `need`.  A buffer is returned
-// once no copy into or out of it is pending.
+// Pinned host buffers for small reads and writes are kept (at most 64, none of
+// more than 32 MB) for the next user, since allocating and freeing pinned memory
+// costs up to a millisecond.  cap: the buffer's capacity in doubles, at least
+// `need`.  A buffer is returned once no copy into or out of it is pending.
 double* pinned_take(size_t need, size_t& cap);
 void pinned_give(double* h, size_t cap);
+
+// A pinned buffer for one call that waits for its copies: contexts hold none of
+// their own, so many of them cost no more than one.  A call that ends by an
+// exception waits before the buffer goes to another one.
+class PinnedLease {
+ public:
+  PinnedLease(size_t need, hipStream_t s) : stream_(s) {
+    size_t cap = 16384;  // a basis of 47, 4096 points, 8000 steps
+    while (cap < need) cap *= 2;
+    h_ = pinned_take(cap, cap_);
+  }
+  ~PinnedLease() {
+    if (std::uncaught_exceptions() > 0) (void)hipStreamSynchronize(stream_);
+    pinned_give(h_, cap_);
+  }
+  PinnedLease(const PinnedLease&) = delete;
+  PinnedLease& operator=(const PinnedLease&) = delete;
+  double* get() const { return h_; }
+
+ private:
+  hipStream_t stream_;
+  double* h_ = nullptr;
+  size_t cap_ = 0;
+};
 
 // Uploads a sector's tables in one allocation and one copy.  Without a
 // stage the call waits for the copy and sets the variant that hv_choose gives

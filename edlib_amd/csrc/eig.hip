@@ -226,7 +226,8 @@ void eigsh_run(Ctx& c, int nev_req, int ncv_req, double tol, int maxitr, uint64_
   double* Tcol = c.small.as<double>();             // column j at Tcol + j*(m+1)
   double* norms = Tcol + (size_t)m * (m + 1);      // norm after orthogonalising column j
   double* Cdev = Tcol + nT;                        // combine coefficients
-  double* const h_T = c.pinned(nT + (size_t)kMaxBasis * kMaxBasis);
+  const PinnedLease lease(nT + (size_t)kMaxBasis * kMaxBasis, s);
+  double* const h_T = lease.get();
   double* const h_C = h_T + nT;
   double* V = c.krylov[0].as<double>();
   double* Valt = c.krylov[1].as<double>();

@@ -230,7 +230,8 @@ void static_obs_run(Ctx& c, const double* dv, int norb, double* out) {
   const int Ns = c.model->Ns;
   EDH_CHECK(norb >= 1 && norb <= Ns, EDH_ERR_ARG, "static observables: interacting orbitals out of range");
   c.obs.ensure(static_obs_scratch(c.tabs, Ns) * sizeof(double));
-  double* host = c.pinned(static_obs_host(c.tabs, Ns));
+  const PinnedLease lease(static_obs_host(c.tabs, Ns), c.stream);
+  double* host = lease.get();
   static_obs_launch(c.tabs, c.dev, Ns, dv, c.obs.as<double>(), c.stream, host);
   EDH_HIP(hipStreamSynchronize(c.stream));
   static_obs_reduce(c.tabs, Ns, norb, host, out);

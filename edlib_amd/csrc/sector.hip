@@ -191,7 +191,7 @@ void configure_mem_pool(int device) {
 namespace {
 std::mutex g_pinned_mu;
 std::vector<std::pair<double*, size_t>> g_pinned_free;  // (buffer, capacity in doubles)
-constexpr size_t kPinnedKept = 64;
+constexpr size_t kPinnedKept = 64, kPinnedLargest = size_t(1) << 22;  // buffers, doubles
 }  // namespace
 
 double* pinned_take(size_t need, size_t& cap) {
@@ -216,7 +216,7 @@ double* pinned_take(size_t need, size_t& cap) {
 }
 
 void pinned_give(double* h, size_t cap) {
-  {
+  if (cap <= kPinnedLargest) {
     std::lock_guard<std::mutex> lk(g_pinned_mu);
     if (g_pinned_free.size() < kPinnedKept) {
       g_pinned_free.push_back({h, cap});

@@ -6,6 +6,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <mutex>
 
 namespace {
 const int kOk = 0, kOutOfMemory = 2;
@@ -15,8 +16,11 @@ struct Counts {
 long g_fail_at = 0;  // the n-th stream-ordered allocation from now on fails
 int g_last = kOk;    // kept until it is asked for
 std::map<void*, size_t> g_mem;
+std::mutex g_mu;
 
-int take(void** p, size_t n) {
+int take(void** p, size_t n, long& count) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  ++count;
   *p = nullptr;
   if (g_fail_at > 0 && --g_fail_at == 0) return g_last = kOutOfMemory;
   *p = malloc(n ? n : 1);
@@ -27,6 +31,7 @@ int take(void** p, size_t n) {
 }
 int give(void* p) {
   if (!p) return kOk;
+  std::lock_guard<std::mutex> lk(g_mu);
   if (g_mem.erase(p)) --g.live;
   free(p);
   return kOk;
@@ -53,9 +58,9 @@ int hipGetLastError() {
   return e;
 }
 const char* hipGetErrorString(int e) { return e == kOutOfMemory ? "out of memory" : "error"; }
-int hipMalloc(void** p, size_t n) { return ++g.allocs, g.alloc_bytes += (long)n, take(p, n); }
-int hipMallocAsync(void** p, size_t n, void*) { return ++g.allocs, g.alloc_bytes += (long)n, take(p, n); }
-int hipHostMalloc(void** p, size_t n, unsigned) { return ++g.host_allocs, take(p, n); }
+int hipMalloc(void** p, size_t n) { return g.alloc_bytes += (long)n, take(p, n, g.allocs); }
+int hipMallocAsync(void** p, size_t n, void*) { return g.alloc_bytes += (long)n, take(p, n, g.allocs); }
+int hipHostMalloc(void** p, size_t n, unsigned) { return take(p, n, g.host_allocs); }
 int hipFree(void* p) { return give(p); }
 int hipFreeAsync(void* p, void*) { return give(p); }
 int hipHostFree(void* p) { return give(p); }
