@@ -392,7 +392,6 @@ HvLinesPlan hv_lines_plan(const DevSector& ds);
 // Host tables of the tile pass (hv_tiles.hip).
 void up_tile_tables(const SpinTables& sp, std::vector<int32_t>& slices, std::vector<uint32_t>& in,
                     std::vector<uint32_t>& out);
-int hv_lines_threads(int64_t D);
 int hv_lines_partials(const DevSector& ds);  // shares of <v, w> per operand
 // than the single pass, for one operand alone; in_place: w = H v + w
 bool hv_lines_faster(const DevSector& ds, bool in_place = false);

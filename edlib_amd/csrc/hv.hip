@@ -942,8 +942,6 @@ HvParams make_params(const DevSector& ds, const HvArgs& a) {
   p.up_slices = ds.up_slices;
   p.up_in = ds.up_in;
   p.up_out = ds.up_out;
-  p.row_t = hv_lines_threads(ds.dn.D);
-  p.col_t = hv_lines_threads(ds.up.D);
   p.xcd_rows = 1;
   p.ctl = a.ctl;
   p.v_alt = a.v_alt;
@@ -1159,6 +1157,9 @@ void launch_multi_c(const HvParams& p, const HvMulti& m, const Launch& L, size_t
 void launch_hv_batch_rows_multi(const DevSector& ds, const HvArgs* a, int count, hipStream_t s) {
   const int fit = hv_batch_rows_multi_fit(ds);
   EDH_CHECK(count >= 2 && count <= fit, EDH_ERR_INTERNAL, "grouped H*v: operand count does not fit one launch");
+  for (int k = 0; k < count; ++k)
+    EDH_CHECK(a[k].dscale && a[k].tdot && !a[k].lzk && !a[k].ctl, EDH_ERR_INTERNAL,
+              "grouped H*v: multi-operand launch takes Lanczos operands with device scales");
   if (lines_lanczos(ds)) {
     HvArgs b[kLinesMax];
     for (int k = 0; k < count; ++k) {
@@ -1172,8 +1173,6 @@ void launch_hv_batch_rows_multi(const DevSector& ds, const HvArgs* a, int count,
   HvMulti m;
   std::memset(&m, 0, sizeof(m));
   for (int k = 0; k < count; ++k) {
-    EDH_CHECK(a[k].dscale && a[k].tdot && !a[k].lzk && !a[k].ctl, EDH_ERR_INTERNAL,
-              "grouped H*v: multi-operand launch takes Lanczos operands with device scales");
     m.v[k] = a[k].v;
     m.w[k] = a[k].w;
     m.wprev[k] = a[k].wprev;

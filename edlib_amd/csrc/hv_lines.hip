@@ -36,7 +36,7 @@ namespace edh {
 
 namespace {
 
-// The operand of a job as the device resolves it.
+// The operand of a job with the scales of this launch.
 struct View {
   const double* V;
   double* W;
@@ -45,33 +45,8 @@ struct View {
   bool accum, live;
 };
 
-__device__ __forceinline__ View resolve_view(const HvBatchJob& J, const HvScales& sc) {
-  const HvParams& p = J.p;
-  View o;
-  o.V = p.v;
-  o.W = p.w;
-  o.Wp = p.wprev;
-  o.accum = p.accumulate != 0;
-  o.live = sc.live;
-  o.vs = sc.v;
-  o.ws = sc.w;
-  if (J.ctl) {  // eigensolver run: its basis column and buffer
-    if (J.ctl[kCtlState] != 0.0) o.live = false;
-    const int64_t N = (int64_t)p.Dup * p.Ddn;
-    const double* base = J.ctl[kCtlPhase] != 0.0 ? J.v_alt : p.v;
-    const int64_t col = (int64_t)J.ctl[kCtlCol];
-    o.V = base + col * N;
-    o.W = const_cast<double*>(base) + (col + 1) * N;
-  } else if (J.lzk) {  // Lanczos run: its buffers in rotation by the step counter
-    const int k = (int)*J.lzk;
-    const double* b[3] = {p.v, p.wprev, p.w};
-    const int r0 = lz_buffer(k, 0), r1 = lz_buffer(k, 1), r2 = lz_buffer(k, 2);
-    o.V = r0 == 0 ? b[0] : (r0 == 1 ? b[1] : b[2]);
-    o.Wp = r1 == 0 ? b[0] : (r1 == 1 ? b[1] : b[2]);
-    o.W = const_cast<double*>(r2 == 0 ? b[0] : (r2 == 1 ? b[1] : b[2]));
-    o.accum = k > 1;
-  }
-  return o;
+__device__ __forceinline__ View view_of(const HvParams& p, const HvScales& sc) {
+  return View{p.v, p.w, p.wprev, sc.v, sc.w, p.accumulate != 0, sc.live};
 }
 
 // LDS image of B lines of D elements: planes of two lines, the pair of a
@@ -255,10 +230,9 @@ __device__ __forceinline__ void row_fetch(const HvBatchJob& J, const View& o, in
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     if (i < i0 || i >= i1) continue;
-    const int d = threadIdx.x + i * p.row_t;
+    const int d = threadIdx.x + i * blockDim.x;
 #pragma unroll
-    for (int r = 0; r < B; ++r)
-      f.x[i][r] = (int)threadIdx.x < p.row_t && d < D && r < R.n ? o.V[(size_t)R.u[r] * D + d] : 0.0;
+    for (int r = 0; r < B; ++r) f.x[i][r] = d < D && r < R.n ? o.V[(size_t)R.u[r] * D + d] : 0.0;
   }
 }
 
@@ -290,8 +264,8 @@ __device__ __forceinline__ void row_tile(const HvBatchJob& J, const View& o, int
       t.ct[i] = p.cross_rowtab[(size_t)row_of(R, i % B) * p.Ns + i / B];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int d = tid + i * p.row_t;
-    if (tid < p.row_t && d < D) {
+    const int d = tid + i * T;
+    if (d < D) {
 #pragma unroll
       for (int r = 0; r < B; ++r) f.x[i][r] *= o.vs;
       put_state<B>(s, ld, d, f.x[i]);
@@ -307,12 +281,10 @@ __device__ __forceinline__ void row_tile(const HvBatchJob& J, const View& o, int
     eu[r] = p.up_e[R.u[r]];
   }
   double dsum = 0.0;
-  // row_t threads of the work-group take the basis states in turn (the
-  // sector's own number, whatever the launch's work-group size)
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int d = tid + i * p.row_t;
-    if (tid < p.row_t && d < D) {
+    const int d = tid + i * T;
+    if (d < D) {
       double acc[B], x[B], cr[B], wv[B];
       // the column pass's part and the accumulated input: added last, so that
       // the gathers do not wait for them
@@ -376,7 +348,7 @@ __device__ __forceinline__ void col_fetch(const HvBatchJob& J, const View& o, in
                                           int i1) {
   const HvParams& p = J.p;
   const int nc = min(B, p.Ddn - c0);
-  const int c = threadIdx.x % B, row0 = threadIdx.x / B, rstep = p.col_t / B;
+  const int c = threadIdx.x % B, row0 = threadIdx.x / B, rstep = blockDim.x / B;
   const double* __restrict__ src = o.V + c0;
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
@@ -384,7 +356,7 @@ __device__ __forceinline__ void col_fetch(const HvBatchJob& J, const View& o, in
 #pragma unroll
     for (int r = 0; r < B; ++r) {
       const int d = row0 + (i * B + r) * rstep;
-      f.x[i][r] = (int)threadIdx.x < p.col_t && d < p.Dup && c < nc ? src[(size_t)d * p.Ddn + c] : 0.0;
+      f.x[i][r] = d < p.Dup && c < nc ? src[(size_t)d * p.Ddn + c] : 0.0;
     }
   }
 }
@@ -406,14 +378,14 @@ __device__ __forceinline__ void col_tile(const HvBatchJob& J, const View& o, int
   const int c = tid % B;
   if (tid < B) s[((size_t)(tid >> 1) * ld + D) * 2 + (tid & 1)] = 0.0;  // the padding entries' state
   {
-    const int row0 = tid / B, rstep = p.col_t / B;
+    const int row0 = tid / B, rstep = T / B;
     double* const sc = s + ((size_t)(c >> 1) * ld * 2 + (c & 1));
 #pragma unroll
     for (int i = 0; i < NI; ++i)
 #pragma unroll
       for (int r = 0; r < B; ++r) {
         const int d = row0 + (i * B + r) * rstep;
-        if (tid < p.col_t && d < D) sc[(size_t)d * 2] = f.x[i][r] * o.vs;
+        if (d < D) sc[(size_t)d * 2] = f.x[i][r] * o.vs;
       }
   }
   __syncthreads();
@@ -422,8 +394,8 @@ __device__ __forceinline__ void col_tile(const HvBatchJob& J, const View& o, int
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     // whole wavefronts: lanes past the last row work on it again
-    const int d1 = tid + i * p.col_t;
-    if (tid < p.col_t && d1 - lane < D) {
+    const int d1 = tid + i * T;
+    if (d1 - lane < D) {
       const int d = min(d1, D - 1);
       double acc[B];
 #pragma unroll
@@ -466,7 +438,7 @@ __global__ __launch_bounds__(1024) void hv_row_lines_kernel(LinesArgs a, int nti
   extern __shared__ double s_line[];
   __shared__ double s_red[16];
   const HvBatchJob& j = a.j[blockIdx.y];
-  const View o = resolve_view(j, HvScales(j.p, s_red));
+  const View o = view_of(j.p, HvScales(j.p, s_red));
   if (!o.live) return;
   Ahead<B, NI> f;
   int t = blockIdx.x;
@@ -487,7 +459,7 @@ __global__ __launch_bounds__(1024) void hv_col_lines_kernel(LinesArgs a, int nti
   __shared__ double s_red[16];
   const HvBatchJob& j = a.j[blockIdx.y];
   const HvScales sc(j.p, s_red);
-  const View o = resolve_view(j, sc);
+  const View o = view_of(j.p, sc);
   const int x = blockIdx.x & 7, step = gridDim.x >> 3;
   const int t1 = o.live ? min(ntiles, (x + 1) * per) : 0;  // this XCD's tiles: [x per, t1)
   Ahead<B, NI> f;
@@ -530,16 +502,13 @@ size_t col_smem(const DevSector& ds, int B, int block) {
   return ((size_t)B * (ds.up.D + 1) + pair_up(ds.nvalues) + (size_t)block * B) * sizeof(double);
 }
 
-}  // namespace
-
-// Threads that share a line of D states: as few rounds as 1024 threads
+// Threads of a work-group for lines of D states: as few rounds as 1024 threads
 // allow, split evenly.
 int hv_lines_threads(int64_t D) {
   const int64_t it = (D + 1023) / 1024;
   return (int)std::max<int64_t>(64, ((D + it - 1) / std::max<int64_t>(it, 1) + 63) / 64 * 64);
 }
 
-namespace {
 int row_tiles(const DevSector& ds, const HvLinesPlan& L) {
   return L.row_b == 4 && ds.n_row_tiles > 0 ? ds.n_row_tiles : (int)((ds.up.D + L.row_b - 1) / L.row_b);
 }

@@ -60,7 +60,6 @@ struct HvParams {
   const int32_t* up_slices;
   const uint32_t* up_in;
   const uint32_t* up_out;
-  int row_t, col_t;  // line passes: threads that share a row, a column (hv_lines_threads)
   int xcd_rows;  // rows kernel: XCD-grouped row assignment (measured 2 % faster on the 16-site sector)
   // rows kernel in a batch: an eigensolver run's control block (v and w are
   // then columns col and col + 1 of the basis in v or v_alt; a run whose
