@@ -63,8 +63,16 @@ constexpr int kStage = 8;
 // Separate instantiations keep the other launches' register allocation as it
 // is (what a Lanczos step keeps to the kernel's end costs the signed form 2 %).
 enum { kRunNone = 0, kRunCtl = 1, kRunLanczos = 2 };
+template <int RUN>
+struct RowParams {
+  typedef HvParams type;
+};
+template <>
+struct RowParams<kRunLanczos> {
+  typedef HvStepParams type;
+};
 template <int J, int CROSS, bool KAN, bool LDS, int EF, bool UP, int RUN>
-__global__ __launch_bounds__(1024) void hv_rows_kernel(HvParams p) {
+__global__ __launch_bounds__(1024) void hv_rows_kernel(typename RowParams<RUN>::type p) {
   extern __shared__ double s_v[];
   __shared__ double s_red[16];
   const int T = blockDim.x;
@@ -73,7 +81,7 @@ __global__ __launch_bounds__(1024) void hv_rows_kernel(HvParams p) {
   const int na = 1 << (p.Ns - p.nb);
   double vscale, wscale, beta = 0.0;
   int rows = p.Dup;
-  if (RUN == kRunLanczos) {
+  if constexpr (RUN == kRunLanczos) {
     const HvScales sc(p, s_red);
     vscale = sc.v;
     wscale = sc.w;
@@ -398,7 +406,8 @@ __global__ __launch_bounds__(1024) void hv_rows_kernel(HvParams p) {
     if (!LDS && RUN == kRunLanczos) __syncthreads();
     block_reduce_store(dsum, s_red, p.dot_partial + blockIdx.x);
   }
-  if (RUN == kRunLanczos && blockIdx.x == 0) HvScales::record(p, vscale, beta, rows > 0);
+  if constexpr (RUN == kRunLanczos)
+    if (blockIdx.x == 0) HvScales::record(p, vscale, beta, rows > 0);
 }
 
 // Several Lanczos operands of one sector in one launch (the batch's
@@ -848,46 +857,56 @@ Launch plan(const DevSector& ds) {
   return L;
 }
 
-template <int J, int CROSS, bool KAN, bool LDS, int EF>
-void launch_t(const HvParams& p, const Launch& L, bool up, hipStream_t s) {
-  auto k = !up      ? hv_rows_kernel<J, CROSS, KAN, LDS, EF, false, kRunLanczos>
-           : p.ctl  ? hv_rows_kernel<J, CROSS, KAN, LDS, EF, true, kRunCtl>
-           : p.lz.k ? hv_rows_kernel<J, CROSS, KAN, LDS, EF, true, kRunLanczos>
-                    : hv_rows_kernel<J, CROSS, KAN, LDS, EF, true, kRunNone>;
+template <class P>
+void launch_rows(void (*k)(P), const P& p, const Launch& L, hipStream_t s) {
   if (L.smem > 64 * 1024)
     EDH_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)L.smem));
   hipLaunchKernelGGL(k, dim3(L.grid), dim3(L.block), L.smem, s, p);
   EDH_HIP(hipGetLastError());
 }
 
+template <int J, int CROSS, bool KAN, bool LDS, int EF>
+void launch_t(const HvParams& p, const LzStep& lz, const Launch& L, bool up, hipStream_t s) {
+  if (up && lz.k == 0)
+    return launch_rows(p.ctl ? hv_rows_kernel<J, CROSS, KAN, LDS, EF, true, kRunCtl>
+                             : hv_rows_kernel<J, CROSS, KAN, LDS, EF, true, kRunNone>, p, L, s);
+  HvStepParams q;
+  static_cast<HvParams&>(q) = p;
+  q.lz = lz;
+  launch_rows(up ? hv_rows_kernel<J, CROSS, KAN, LDS, EF, true, kRunLanczos>
+                 : hv_rows_kernel<J, CROSS, KAN, LDS, EF, false, kRunLanczos>, q, L, s);
+}
+
 template <int J, int CROSS>
-void launch_c(const HvParams& p, const Launch& L, bool kan, bool up, hipStream_t s) {
+void launch_c(const HvParams& p, const LzStep& lz, const Launch& L, bool kan, bool up, hipStream_t s) {
   if (kan) {
-    if (L.ef == 4) launch_t<J, CROSS, true, true, 4>(p, L, up, s);
-    else if (L.ef == 3) launch_t<J, CROSS, true, true, 3>(p, L, up, s);
-    else if (L.ef == 2) launch_t<J, CROSS, true, true, 2>(p, L, up, s);
-    else if (L.ef == 1) launch_t<J, CROSS, true, true, 1>(p, L, up, s);
-    else if (L.lds) launch_t<J, CROSS, true, true, 0>(p, L, up, s);
-    else launch_t<J, CROSS, true, false, 0>(p, L, up, s);
+    if (L.ef == 4) launch_t<J, CROSS, true, true, 4>(p, lz, L, up, s);
+    else if (L.ef == 3) launch_t<J, CROSS, true, true, 3>(p, lz, L, up, s);
+    else if (L.ef == 2) launch_t<J, CROSS, true, true, 2>(p, lz, L, up, s);
+    else if (L.ef == 1) launch_t<J, CROSS, true, true, 1>(p, lz, L, up, s);
+    else if (L.lds) launch_t<J, CROSS, true, true, 0>(p, lz, L, up, s);
+    else launch_t<J, CROSS, true, false, 0>(p, lz, L, up, s);
   } else {
-    if (L.ef == 4) launch_t<J, CROSS, false, true, 4>(p, L, up, s);
-    else if (L.ef == 3) launch_t<J, CROSS, false, true, 3>(p, L, up, s);
-    else if (L.ef == 2) launch_t<J, CROSS, false, true, 2>(p, L, up, s);
-    else if (L.ef == 1) launch_t<J, CROSS, false, true, 1>(p, L, up, s);
-    else if (L.lds) launch_t<J, CROSS, false, true, 0>(p, L, up, s);
-    else launch_t<J, CROSS, false, false, 0>(p, L, up, s);
+    if (L.ef == 4) launch_t<J, CROSS, false, true, 4>(p, lz, L, up, s);
+    else if (L.ef == 3) launch_t<J, CROSS, false, true, 3>(p, lz, L, up, s);
+    else if (L.ef == 2) launch_t<J, CROSS, false, true, 2>(p, lz, L, up, s);
+    else if (L.ef == 1) launch_t<J, CROSS, false, true, 1>(p, lz, L, up, s);
+    else if (L.lds) launch_t<J, CROSS, false, true, 0>(p, lz, L, up, s);
+    else launch_t<J, CROSS, false, false, 0>(p, lz, L, up, s);
   }
 }
 
 template <int J>
-void launch_j(const HvParams& p, const Launch& L, int cross, bool kan, bool up, hipStream_t s) {
+void launch_j(const HvParams& p, const LzStep& lz, const Launch& L, int cross, bool kan, bool up, hipStream_t s) {
   switch (cross) {
-    case CROSS_NONE: launch_c<J, CROSS_NONE>(p, L, kan, up, s); break;
-    case CROSS_POPC: launch_c<J, CROSS_POPC>(p, L, kan, up, s); break;
-    case CROSS_IMP: launch_c<J, CROSS_IMP>(p, L, kan, up, s); break;
-    default: launch_c<J, CROSS_GENERAL>(p, L, kan, up, s); break;
+    case CROSS_NONE: launch_c<J, CROSS_NONE>(p, lz, L, kan, up, s); break;
+    case CROSS_POPC: launch_c<J, CROSS_POPC>(p, lz, L, kan, up, s); break;
+    case CROSS_IMP: launch_c<J, CROSS_IMP>(p, lz, L, kan, up, s); break;
+    default: launch_c<J, CROSS_GENERAL>(p, lz, L, kan, up, s); break;
   }
 }
+
+}  // namespace
 
 HvParams make_params(const DevSector& ds, const HvArgs& a) {
   HvParams p;
@@ -938,7 +957,6 @@ HvParams make_params(const DevSector& ds, const HvArgs& a) {
   p.dot_partial = a.dot_partial;
   p.dscale = a.dscale;
   p.done = a.done;
-  p.lz = a.step;
   p.up_slices = ds.up_slices;
   p.up_in = ds.up_in;
   p.up_out = ds.up_out;
@@ -948,7 +966,12 @@ HvParams make_params(const DevSector& ds, const HvArgs& a) {
   return p;
 }
 
-}  // namespace
+HvStepParams make_step_params(const DevSector& ds, const HvArgs& a) {
+  HvStepParams p;
+  static_cast<HvParams&>(p) = make_params(ds, a);
+  p.lz = a.step;
+  return p;
+}
 
 int hv_num_blocks(const DevSector& ds) {
   if (ds.variant != HV_TWO_PASS) return plan(ds).grid;
@@ -965,18 +988,18 @@ void launch_hv(const DevSector& ds, const HvArgs& a, hipStream_t s, int variant)
   if (variant == HV_AUTO) variant = a.mode && a.wprev == a.w ? ds.variant_in_place : ds.variant;
   if (variant == HV_TWO_PASS && hv_lines_plan(ds).ok) return launch_hv_lines(ds, &a, 1, s);
   Launch L = plan(ds);
-  HvParams p = make_params(ds, a);
+  const HvParams p = make_params(ds, a);
   const bool kan = ds.kan_ml > 0;
   const bool up = variant != HV_TWO_PASS;
   switch (L.J) {
-    case 1: launch_j<1>(p, L, ds.cross_mode, kan, up, s); break;
-    case 2: launch_j<2>(p, L, ds.cross_mode, kan, up, s); break;
-    default: launch_j<4>(p, L, ds.cross_mode, kan, up, s); break;
+    case 1: launch_j<1>(p, a.step, L, ds.cross_mode, kan, up, s); break;
+    case 2: launch_j<2>(p, a.step, L, ds.cross_mode, kan, up, s); break;
+    default: launch_j<4>(p, a.step, L, ds.cross_mode, kan, up, s); break;
   }
   if (!up) {
     // the rows pass wrote the partial result; the tile pass adds the up-spin
     // term and produces the dot partials (the rows pass skips them)
-    launch_hv_up_tiles(ds, p, s);
+    launch_hv_up_tiles(ds, make_step_params(ds, a), s);
   }
 }
 
@@ -1022,7 +1045,7 @@ namespace edh {
 
 size_t hv_batch_job_bytes() { return sizeof(HvBatchJob); }
 
-HvBatchJob make_job(const DevSector& ds, const HvArgs& a) {
+void hv_batch_fill(const DevSector& ds, const HvArgs& a, int64_t row0, void* out) {
   HvBatchJob j;
   std::memset(&j, 0, sizeof(j));
   j.p = make_params(ds, a);
@@ -1032,11 +1055,6 @@ HvBatchJob make_job(const DevSector& ds, const HvArgs& a) {
   j.v_alt = a.v_alt;
   j.tdot = a.tdot;
   j.lzk = a.lzk;
-  return j;
-}
-
-void hv_batch_fill(const DevSector& ds, const HvArgs& a, int64_t row0, void* out) {
-  HvBatchJob j = make_job(ds, a);
   j.row0 = row0;
   std::memcpy(out, &j, sizeof(j));
 }

@@ -36,7 +36,13 @@ namespace edh {
 
 namespace {
 
-// The operand of a job with the scales of this launch.
+// One operand of a launch.
+struct LinesJob {
+  HvStepParams p;
+  int cross, kan;
+};
+
+// The operand with the scales of this launch.
 struct View {
   const double* V;
   double* W;
@@ -114,7 +120,7 @@ __device__ __forceinline__ void gather_line(const double* s, int ld, const doubl
 template <int B>
 struct Rows {
   int u[B], n;
-  __device__ __forceinline__ Rows(const HvParams& p, int tile) {
+  __device__ __forceinline__ Rows(const HvStepParams& p, int tile) {
     if (B == 4 && p.row_tiles) {
       n = 0;
 #pragma unroll
@@ -161,7 +167,7 @@ __device__ __forceinline__ void kan_terms(const HvParams& p, const View& o, cons
 // rows a term leads to are the same for all states of a row.  The rows' reads
 // are in flight together.
 template <int B>
-__device__ __forceinline__ void kan_targets(const HvParams& p, const double* tc, const int* td, const double* s,
+__device__ __forceinline__ void kan_targets(const HvStepParams& p, const double* tc, const int* td, const double* s,
                                             int ld, const int (&a)[B], int b, int na, int n, int d,
                                             double (&acc)[B]) {
   for (int j = 0; j < p.kan_t; ++j) {
@@ -210,8 +216,8 @@ struct RowTables {
   double *vals, *kc, *ct;
   int* kd;
   int nk;  // impurity-term table entries staged
-  __device__ __forceinline__ RowTables(const HvBatchJob& J, double* s, int ld) {
-    const HvParams& p = J.p;
+  __device__ __forceinline__ RowTables(const LinesJob& J, double* s, int ld) {
+    const HvStepParams& p = J.p;
     const int na = 1 << (p.Ns - p.nb);
     vals = s + (size_t)B * ld;
     nk = B == 4 && J.kan && p.row_tiles ? na * na * p.kan_t : 0;
@@ -222,9 +228,9 @@ struct RowTables {
 };
 
 template <int B, int NI>
-__device__ __forceinline__ void row_fetch(const HvBatchJob& J, const View& o, int tile, Ahead<B, NI>& f, int i0,
+__device__ __forceinline__ void row_fetch(const LinesJob& J, const View& o, int tile, Ahead<B, NI>& f, int i0,
                                           int i1) {
-  const HvParams& p = J.p;
+  const HvStepParams& p = J.p;
   const int D = p.Ddn;
   const Rows<B> R(p, tile);
 #pragma unroll
@@ -239,9 +245,9 @@ __device__ __forceinline__ void row_fetch(const HvBatchJob& J, const View& o, in
 // One row tile whose lines are in f; the next tile's (tn, when there are more)
 // are fetched into f on the way.
 template <int B, int NI>
-__device__ __forceinline__ void row_tile(const HvBatchJob& J, const View& o, int tile, bool tables, bool more, int tn,
+__device__ __forceinline__ void row_tile(const LinesJob& J, const View& o, int tile, bool tables, bool more, int tn,
                                          Ahead<B, NI>& f, double* s, double* s_red) {
-  const HvParams& p = J.p;
+  const HvStepParams& p = J.p;
   const int D = p.Ddn, T = blockDim.x;
   const int tid = fresh_tid();
   const int ld = D + 1;
@@ -337,16 +343,16 @@ __device__ __forceinline__ void row_tile(const HvBatchJob& J, const View& o, int
     }
     __builtin_amdgcn_sched_barrier(0);
   }
-  if (J.tdot) block_reduce_store(dsum, s_red, J.tdot + tile);
+  if (p.dot_partial) block_reduce_store(dsum, s_red, p.dot_partial + tile);
   __syncthreads();  // the next tile's lines replace this one's
 }
 
 // B consecutive lanes read the B columns of a row: a load instruction touches
 // 64 / B rows.  Load q of thread t is element q T + t of the D x B tile.
 template <int B, int NI>
-__device__ __forceinline__ void col_fetch(const HvBatchJob& J, const View& o, int c0, Ahead<B, NI>& f, int i0,
+__device__ __forceinline__ void col_fetch(const LinesJob& J, const View& o, int c0, Ahead<B, NI>& f, int i0,
                                           int i1) {
-  const HvParams& p = J.p;
+  const HvStepParams& p = J.p;
   const int nc = min(B, p.Ddn - c0);
   const int c = threadIdx.x % B, row0 = threadIdx.x / B, rstep = blockDim.x / B;
   const double* __restrict__ src = o.V + c0;
@@ -364,9 +370,9 @@ __device__ __forceinline__ void col_fetch(const HvBatchJob& J, const View& o, in
 // LDS of a column tile after its lines: the value table, then 64 x B results
 // per wavefront.
 template <int B, int NI>
-__device__ __forceinline__ void col_tile(const HvBatchJob& J, const View& o, int c0, bool tables, bool more, int cn,
+__device__ __forceinline__ void col_tile(const LinesJob& J, const View& o, int c0, bool tables, bool more, int cn,
                                          Ahead<B, NI>& f, double* s) {
-  const HvParams& p = J.p;
+  const HvStepParams& p = J.p;
   const int D = p.Dup, T = blockDim.x;
   const int tid = fresh_tid();
   const int ld = D + 1;
@@ -429,7 +435,7 @@ __device__ __forceinline__ void col_tile(const HvBatchJob& J, const View& o, int
 }
 
 struct LinesArgs {
-  HvBatchJob j[kLinesMax];
+  LinesJob j[kLinesMax];
 };
 
 // Operand blockIdx.y: row tiles blockIdx.x, blockIdx.x + gridDim.x, ...
@@ -437,7 +443,7 @@ template <int B, int NI>
 __global__ __launch_bounds__(1024) void hv_row_lines_kernel(LinesArgs a, int ntiles) {
   extern __shared__ double s_line[];
   __shared__ double s_red[16];
-  const HvBatchJob& j = a.j[blockIdx.y];
+  const LinesJob& j = a.j[blockIdx.y];
   const View o = view_of(j.p, HvScales(j.p, s_red));
   if (!o.live) return;
   Ahead<B, NI> f;
@@ -457,7 +463,7 @@ template <int B, int NI>
 __global__ __launch_bounds__(1024) void hv_col_lines_kernel(LinesArgs a, int ntiles, int per) {
   extern __shared__ double s_line[];
   __shared__ double s_red[16];
-  const HvBatchJob& j = a.j[blockIdx.y];
+  const LinesJob& j = a.j[blockIdx.y];
   const HvScales sc(j.p, s_red);
   const View o = view_of(j.p, sc);
   const int x = blockIdx.x & 7, step = gridDim.x >> 3;
@@ -581,8 +587,9 @@ void launch_hv_lines(const DevSector& ds, const HvArgs* ops, int count, hipStrea
   EDH_CHECK(count >= 1 && count <= kLinesMax, EDH_ERR_INTERNAL, "H*v lines: operand count");
   LinesArgs a;
   for (int q = 0; q < count; ++q) {
-    a.j[q] = make_job(ds, ops[q]);
-    if (ops[q].dot_partial) a.j[q].tdot = ops[q].dot_partial;
+    a.j[q].p = make_step_params(ds, ops[q]);
+    a.j[q].cross = ds.cross_mode;
+    a.j[q].kan = ds.kan_ml > 0 ? 1 : 0;
   }
   for (int q = count; q < kLinesMax; ++q) a.j[q] = a.j[0];
   const bool r1 = ds.dn.D <= 1024, c1 = ds.up.D <= 1024;

@@ -5,6 +5,12 @@
 
 namespace edh {
 
+// What an H*v reads.  Every launch copies it and every work-group begins with
+// loads from it, so size and order count in the smallest sectors: without the
+// Lanczos step, in this order, kanamori (8 sites) takes 6.40 us a call and 16-bit
+// and 32-bit entry sectors up to 13 sites 1 to 2.5 % less than with the single
+// pass's fields together in front (6.50), where the loads are merged into wider
+// ones; with the step inside 6.55.
 struct HvParams {
   int Ns, nb;  // sites per spin, bath bits (Ns - ml) below the impurity bits
   int Dup, Ddn;
@@ -54,7 +60,6 @@ struct HvParams {
   double* dot_partial;
   const double* dscale;
   const int* done;
-  LzStep lz;
   // tile pass: per slice of two up rows (start, length) of its entries within
   // the tile and outside it
   const int32_t* up_slices;
@@ -66,6 +71,11 @@ struct HvParams {
   // state is not 0 is skipped)
   const double* ctl;
   const double* v_alt;
+};
+
+// With a step of a single-sector Lanczos run (lz.k = 0: without).
+struct HvStepParams : HvParams {
+  LzStep lz;
 };
 
 template <int CROSS>
@@ -127,7 +137,7 @@ struct HvScales {
   double v = 0.0, w = 0.0;
   double beta = 0.0;  // Lanczos step after the first: |W_k|
   bool live = false;
-  __device__ __forceinline__ HvScales(const HvParams& p, double* s_red) {
+  __device__ __forceinline__ HvScales(const HvStepParams& p, double* s_red) {
     if (p.lz.k == 0) {
       if (p.done && *p.done) return;
       v = p.dscale ? p.dscale[0] : p.vscale;
@@ -152,7 +162,7 @@ struct HvScales {
   // turns them all from scalar into vector loads (the single pass then takes
   // 5.1 instead of 3.8 ms on the 16-site torus, 187 instead of 134 us on the
   // 14-site ring).
-  static __device__ __forceinline__ void record(const HvParams& p, double v, double beta, bool live) {
+  static __device__ __forceinline__ void record(const HvStepParams& p, double v, double beta, bool live) {
     if (!p.lz.write || p.lz.k == 0 || threadIdx.x != 0) return;
     if (p.lz.k == 1) {
       p.lz.scale[1] = 1.0;
@@ -189,10 +199,11 @@ struct HvBatchJob {
 // The up-spin term in tiles (hv_tiles.hip): w += Hup v and the shares of
 // <v, w>, hv_up_tiles_blocks of them.
 int hv_up_tiles_blocks(const DevSector& ds);
-void launch_hv_up_tiles(const DevSector& ds, const HvParams& p, hipStream_t s);
+void launch_hv_up_tiles(const DevSector& ds, const HvStepParams& p, hipStream_t s);
 
-// Fills the descriptor of one operand (hv.hip).
-HvBatchJob make_job(const DevSector& ds, const HvArgs& a);
+// The parameters of one operand (hv.hip).
+HvParams make_params(const DevSector& ds, const HvArgs& a);
+HvStepParams make_step_params(const DevSector& ds, const HvArgs& a);
 
 // Largest dynamic LDS a block may use on the current device, less the
 // static reduction scratch (hv.hip).

@@ -48,7 +48,7 @@ __device__ __forceinline__ double2 get_pair(const double* q, bool two) {
 }
 
 template <bool VEC>
-__global__ __launch_bounds__(kTileWG) void hv_up_tiles_kernel(HvParams p, int ntiles, int nslabs, int per) {
+__global__ __launch_bounds__(kTileWG) void hv_up_tiles_kernel(HvStepParams p, int ntiles, int nslabs, int per) {
   extern __shared__ double s_tile[];  // the tile, a zero row, the value table
   __shared__ double s_red[16];
   const HvScales sc(p, s_red);
@@ -224,7 +224,7 @@ void up_tile_tables(const SpinTables& sp, std::vector<int32_t>& slices, std::vec
 
 int hv_up_tiles_blocks(const DevSector& ds) { return tile_grid(ds).grid; }
 
-void launch_hv_up_tiles(const DevSector& ds, const HvParams& p, hipStream_t s) {
+void launch_hv_up_tiles(const DevSector& ds, const HvStepParams& p, hipStream_t s) {
   EDH_CHECK(ds.two_pass && ds.up_slices, EDH_ERR_INTERNAL, "H*v tiles: the sector has no tables for them");
   const TileGrid g = tile_grid(ds);
   const size_t smem = ((size_t)(kTileRows + 1) * kTileW + ds.nvalues) * sizeof(double);

@@ -257,11 +257,11 @@ bool lanczos_run_fits(const DevSector& ds) { return run_plan(ds).ok; }
 void dev_lanczos_run(const DevSector& ds, const double* v0, int nl, double* res, hipStream_t s) {
   const RunPlan r = run_plan(ds);
   EDH_CHECK(r.ok, EDH_ERR_INTERNAL, "Lanczos run: the sector does not fit one work-group");
-  const HvBatchJob j = make_job(ds, HvArgs{});
+  const HvParams p = make_params(ds, HvArgs{});
   auto k = r.hops <= 8 ? lanczos_run_kernel<8> : lanczos_run_kernel<16>;
   if (r.smem > 64 * 1024)
     EDH_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)r.smem));
-  hipLaunchKernelGGL(k, dim3(1), dim3(kRunWG), r.smem, s, j.p, r.t, j.cross, nl, v0, res);
+  hipLaunchKernelGGL(k, dim3(1), dim3(kRunWG), r.smem, s, p, r.t, ds.cross_mode, nl, v0, res);
   EDH_HIP(hipGetLastError());
 }
 

@@ -99,7 +99,7 @@ __global__ __launch_bounds__(kVecBlock) void lanczos_update_kernel(double* __res
 //   fold:  the H*v's shares of <v, w> into kLzFold
 __global__ __launch_bounds__(kVecBlock) void lanczos_scale_kernel(LzStep lz, double* __restrict__ pair) {
   __shared__ double s_red[16];
-  HvParams p;
+  HvStepParams p;
   p.lz = lz;
   const HvScales sc(p, s_red);
   if (threadIdx.x != 0) return;
