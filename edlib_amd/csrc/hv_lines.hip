@@ -556,6 +556,11 @@ int hv_lines_partials(const DevSector& ds) {
 //     1.17 at 42 (3432 x 3432 1.14, 0.95 at 23, 1.31, 1.10 at 30); compact 0.87,
 //     0.72 at 14, 1.24, 1.04 at 28; plain 1.08, 0.89 at 14, 1.42, 1.17 at 28
 //     (3003 x 3003 and 3432 x 3432 1.42 to 1.6, 1.11 to 1.24 at 14)
+//     Calls of several contexts, on streams of their own, overlap, and the single
+//     pass gains more by it where rows are many and short: signed 3432 x 2002
+//     0.89 at 22 (1.04 one after the other), 1.14 at 29, 3003 x 2002 0.91 at 22,
+//     1.16 at 29; compact 0.82 at 14, 1.28 at 29; plain 0.96 to 0.99 at 13 (1.12
+//     to 1.16 one after the other); 2002 x 3003 and square ones 1.06 to 1.26
 //   one spin two lines at a time (3003 x 6435, 6435 x 3003): signed 0.96 to
 //     1.00, 0.84 to 0.89 at 30, 1.16, 1.03 at 45; compact 1.13, 0.97 at 30, 1.30,
 //     1.13 at 45; plain 1.37, 1.18 at 30
@@ -569,13 +574,17 @@ bool hv_lines_faster(const DevSector& ds, bool in_place) {
   if (!L.ok) return false;
   static const double small[2][3] = {{39, 36, 28}, {56, 45, 34}};
   static const double large[2][3] = {{21, 20, 12}, {34, 28, 22}};
+  static const double tall[3] = {27, 23, 18};
   static const double mixed[2][3] = {{36, 30, 30}, {45, 36, 30}};
   static const double pairs[2][3] = {{46, 40, 30}, {62, 54, 40}};
   const int q = in_place ? 1 : 0, f = ds.dn_form;
   const bool general = f == 2 && ds.cross_mode == CROSS_GENERAL;
   if (L.row_b < 4 && L.col_b < 4) return ds.hops >= pairs[q][f];
   if (L.row_b < 4 || L.col_b < 4) return ds.hops >= mixed[q][f];
-  if (ds.N >= 2500000) return ds.hops >= (in_place && f == 2 && ds.N >= 9000000 ? 12 : large[q][f]);
+  if (ds.N >= 2500000) {
+    if (!in_place && 4 * ds.up.D > 5 * ds.dn.D) return ds.hops >= tall[f];
+    return ds.hops >= (in_place && f == 2 && ds.N >= 9000000 ? 12 : large[q][f]);
+  }
   if (ds.N < 600000) return general && ds.hops >= 28;
   // (the single pass's terms beyond the hopping make up for six hops)
   return ds.hops >= (in_place && f == 2 && (general || ds.kan_ml > 0) ? 28 : small[q][f]);

@@ -30,7 +30,10 @@ def test_choice(tmp_path):
         (dis(12), (6, 4), 0, 0),              # 18.7 : 19.5, 19.5 : 23.7
         (dis(13), (4, 4), 1, 1),              # 26.8 : 20.4, 27.6 : 23.8
         (siam(13, 1), (6, 6), 1, 0),          # 45.5 : 41.7, 49.4 : 54.3
-        (siam(14, 1), (7, 5), 1, 0),          # 92.8 : 80.0, 102 : 108
+        (siam(14, 1), (5, 6), 1, 0),          # 91.6 : 79.6 on three streams, in place 98 : 111
+        (siam(14, 1), (6, 5), 0, 0),          # 74.7 : 76.7 on three streams
+        (torus(2, 7), (8, 5), 0, 0),          # 74.6 : 82.1 on three streams
+        (torus(2, 7), (5, 6), 1, 0),          # 89.0 : 83.9 on three streams
         (siam(14, 1), (7, 7), 1, 1),          # 175 : 121, 188 : 169
         (siam(14, 3), (7, 7), 1, 1),          # 378 : 194, 394 : 241
         (torus(2, 7), (5, 5), 0, 0),          # 54.3 : 54.4, 59.3 : 70.5
