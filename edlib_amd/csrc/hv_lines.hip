@@ -77,9 +77,11 @@ __device__ __forceinline__ void get_state(const double* s, int ld, int i, double
 // acc[b] += sum over the entries of basis state i (slice i / 64) of
 // value * line b[column].  An entry holds its column's byte offset in a plane
 // and its value's byte offset in the value table (kLineOff), so decoding it
-// takes two instructions.  The slice's slot count is wavefront-uniform; U
-// entries are decoded together, the next U in flight (B = 4, U = 8 against
-// 4: 14-site Kanamori column pass 111 -> 94 us).
+// takes two instructions.  The slice's slot count is wavefront-uniform.  Entries
+// come in groups of U, the next group's loads issued before a group is worked on
+// (B = 4, U = 8 against 4: 14-site Kanamori column pass 111 -> 94 us); but the
+// tests of the count compile to a branch per entry and a wait for all loads per
+// group, so neither these loads nor an entry's LDS reads overlap much else.
 template <int B, int U>
 __device__ __forceinline__ void gather_line(const double* s, int ld, const double* s_vals, const int32_t* slptr,
                                             const int32_t* sllen, const uint32_t* ell, int i, double (&acc)[B]) {
@@ -292,8 +294,8 @@ __device__ __forceinline__ void row_tile(const LinesJob& J, const View& o, int t
     const int d = tid + i * T;
     if (d < D) {
       double acc[B], x[B], cr[B], wv[B];
-      // the column pass's part and the accumulated input: added last, so that
-      // the gathers do not wait for them
+      // the column pass's part and the accumulated input: issued here, added
+      // last (the first group of entries waits for them with its own loads)
 #pragma unroll
       for (int r = 0; r < B; ++r) wv[r] = r < R.n ? o.W[(int64_t)R.u[r] * D + d] : 0.0;
       if (accum) {

@@ -9,17 +9,19 @@
 // row's 512-byte segment from L2 or the memory-side cache.  Every slice of two
 // rows has its own two lists of entries, padded to the longer row.
 //
-// A wavefront works on two rows, two columns per lane.  While a tile is worked
-// on, the work-group's next tile is on its way into registers (one work-group
-// per CU: nothing else would fill the wait).
+// A wavefront works on two rows, two columns per lane.  The grid is one
+// work-group per CU (two of them, which LDS would hold, miss L2 for 137 M lines
+// instead of 97 M); while a tile is worked on, the work-group's next one is on
+// its way into registers, since nothing else would fill the wait.
 //
 // What bounds it: lines that miss the XCD's L2, 97 M of 183 M (128 bytes each,
 // 6 TB/s) on the 4x4 torus, 2.0 ms; a pass that gathered every hop from a slab
 // of 16 columns in L2 took 3.5 ms.  Narrower slabs fit L2 but touch more lines
 // (a row of 12,870 elements is no multiple of a line) and take more address
-// work: 16 columns x 1024 rows 2.4 ms, 32 x 512 2.2 ms, 64 x 256 2.0 ms, 128 x
-// 128 2.4 ms.  The whole H*v of that sector, one after the other for seconds: 4.8
-// -> 3.5 ms (alone 3.8 -> 3.3: the single pass's 25 GB of gathers cost clock).
+// work: 16 columns x 1024 rows 2.44 ms, 32 x 512 2.17 ms, 64 x 256 2.04 ms, 64 x
+// 128 2.02 ms (the one here: half the LDS), 128 x 128 2.44 ms.  The whole H*v of
+// that sector, one after the other for seconds: 4.8 -> 3.3 ms (from rest 3.8 ->
+// 3.3: the single pass's 25 GB of gathers cost clock).
 #include <algorithm>
 
 #include "hv_params.h"
