@@ -397,6 +397,7 @@ int hv_lines_partials(const DevSector& ds);  // shares of <v, w> per operand
 bool hv_lines_faster(const DevSector& ds, bool in_place = false);
 constexpr int kLinesMax = 4;  // operands per launch
 constexpr int64_t kLinesMin = 500000;  // smallest sector for which the line passes are taken
+bool hv_batch_lines(const DevSector& ds);  // a batch's Lanczos operands take them
 constexpr int64_t kLinesLanczos = 2500000;  // smallest sector whose Lanczos operands take them in a batch
 void launch_hv_lines(const DevSector& ds, const HvArgs* ops, int count, hipStream_t s);
 
@@ -426,8 +427,8 @@ void launch_hv_batch(const void* djobs, const HvBatchUnit* dunits, int nunits, i
 bool hv_batch_routed(int64_t dup, int64_t ddn);
 // The same for Lanczos operands (Green's-function runs): also sectors of at
 // least 256 rows of 512..4608 elements whose format has the multi-operand
-// kernel, so that their runs share launches, and sectors of kLinesLanczos
-// states and more where the line passes beat the single pass (the decision
+// kernel, so that their runs share launches, and sectors whose operands take the
+// line passes (hv_batch_lines: of kLinesLanczos states and more; the decision
 // depends on the sector only, so a run's arithmetic does not depend on the
 // other runs).
 bool hv_batch_routed_lanczos(const DevSector& ds);

@@ -1129,26 +1129,30 @@ bool multi_ok(const DevSector& ds) {
 }
 }  // namespace
 
-namespace {
-// Lanczos operands on the line passes: large sectors where they beat the
-// single pass (14-site Kanamori sector (8,7), four operands: 860 us of H*v per step
-// against 944 in the multi-operand rows kernel).
-bool lines_lanczos(const DevSector& ds) { return ds.N >= kLinesLanczos && hv_lines_faster(ds); }
-}  // namespace
+// Lanczos operands on the line passes: large sectors where they beat the single
+// pass, and with plain entries, whose sectors have the multi-operand rows kernel,
+// from 28 hops on (a Lanczos run whole, four runs, multi-operand rows : lines:
+// Anderson, 13 to 14 hops, 13 sites 4.45 : 5.06 ms, 14 sites (7,7) 16.5 : 19.4,
+// (5,5) 5.62 : 7.09, though one run alone takes 5.53 : 4.78; Kanamori, 32 hops,
+// 13 sites 7.30 : 6.60; disordered, 34 hops, 9.24 : 6.92).  The choice depends on
+// the sector alone, so that a run's bits do.
+bool hv_batch_lines(const DevSector& ds) {
+  return ds.N >= kLinesLanczos && (ds.dn_form != 2 || ds.hops >= 28) && hv_lines_faster(ds);
+}
 
 bool hv_batch_routed_lanczos(const DevSector& ds) {
-  if (lines_lanczos(ds)) return true;
+  if (hv_batch_lines(ds)) return true;
   const int64_t dup = ds.up.D, ddn = ds.dn.D;
   if (hv_batch_routed(dup, ddn)) return true;
   return dup >= 256 && ddn >= 512 && ddn <= kStageMax && multi_ok(ds);
 }
 
 int64_t hv_batch_rows_partials(const DevSector& ds) {
-  return lines_lanczos(ds) ? hv_lines_partials(ds) : std::min<int64_t>(ds.up.D, 1 << 20);
+  return hv_batch_lines(ds) ? hv_lines_partials(ds) : std::min<int64_t>(ds.up.D, 1 << 20);
 }
 
 int hv_batch_rows_multi_fit(const DevSector& ds) {
-  if (lines_lanczos(ds)) return kLinesMax;
+  if (hv_batch_lines(ds)) return kLinesMax;
   return hv_batch_routed_lanczos(ds) && multi_ok(ds) ? kMultiMax : 0;
 }
 
@@ -1178,7 +1182,7 @@ void launch_hv_batch_rows_multi(const DevSector& ds, const HvArgs* a, int count,
   for (int k = 0; k < count; ++k)
     EDH_CHECK(a[k].dscale && a[k].tdot && !a[k].lzk && !a[k].ctl, EDH_ERR_INTERNAL,
               "grouped H*v: multi-operand launch takes Lanczos operands with device scales");
-  if (lines_lanczos(ds)) {
+  if (hv_batch_lines(ds)) {
     HvArgs b[kLinesMax];
     for (int k = 0; k < count; ++k) {
       b[k] = a[k];
@@ -1215,7 +1219,7 @@ void launch_hv_batch_rows_multi(const DevSector& ds, const HvArgs* a, int count,
 void launch_hv_batch_rows(const DevSector& ds, const HvArgs& a, hipStream_t s) {
   EDH_CHECK(hv_batch_routed_lanczos(ds), EDH_ERR_INTERNAL,
             "grouped H*v: operand not routed to the rows kernel");
-  const bool lines = !a.ctl && a.tdot && lines_lanczos(ds);
+  const bool lines = !a.ctl && a.tdot && hv_batch_lines(ds);
   EDH_CHECK(lines || !a.tdot || plan(ds).grid == hv_batch_rows_partials(ds), EDH_ERR_INTERNAL,
             "grouped H*v: rows grid mismatch");
   EDH_CHECK(!a.lzk, EDH_ERR_INTERNAL, "grouped H*v: rows-kernel operands take resolved buffers");

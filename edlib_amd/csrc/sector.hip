@@ -356,8 +356,8 @@ void upload_sector(const SectorTables& st, int Ns, DevSector& ds, hipStream_t s,
   // the two passes' tables where they are taken by themselves: in a batch by
   // its Lanczos operands, else by the sector's own choice
   const int variant = stage ? HV_SINGLE : hv_choose(ds, false), in_place = stage ? HV_SINGLE : hv_choose(ds, true);
-  const bool two_pass = ds.N > 0 && (stage ? st.N >= kLinesLanczos && hv_lines_faster(ds)
-                                           : variant == HV_TWO_PASS || in_place == HV_TWO_PASS);
+  const bool two_pass =
+      ds.N > 0 && (stage ? hv_batch_lines(ds) : variant == HV_TWO_PASS || in_place == HV_TWO_PASS);
   if (two_pass) add_two_pass(pk, st, ds);
   pk.commit(ds, s, stage);
   ds.two_pass = two_pass;

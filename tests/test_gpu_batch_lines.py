@@ -1,12 +1,13 @@
 """Batched Lanczos operands on the line passes (csrc/hv_lines.hip), which sectors
-of 2.5 million states and more take where the line passes beat the single pass:
-13-site sectors of the three-orbital impurity (row tiles with slots that hold no
-row) and of the Anderson impurity (no impurity terms), alone and up to five
-together, one of them with a start vector that ends its run at the first step.
+of 2.5 million states and more take where the line passes beat the single pass
+(with 32-bit entries from 28 hops a state on): a 13-site sector of the
+three-orbital impurity (row tiles with slots that hold no row) and a 14-site
+torus with t and t' (no impurity terms), alone and up to five together, one of
+them with a start vector that ends its run at the first step.
 
 A single context makes the same choice by the same rule from that size on, and
-says which variant it took: that the batch is on the line passes follows from
-it.
+says which variant it took; tests/test_batch_routes.py counts the batch's
+launches.
 
 Tolerances: alone and grouped bit for bit; against the single-sector run and
 the oracle 1e-10 of the spectrum's scale over 8 steps (another order of sums, as
@@ -15,7 +16,7 @@ import numpy as np
 import pytest
 
 from oracle import edoracle as eo
-from tests.models import oracle_model, product_model, siam_params
+from tests.models import oracle_model, product_model, siam_params, torus_hopping
 
 pytestmark = pytest.mark.gpu
 NL = 8
@@ -62,21 +63,22 @@ def _runs(b, sid, vs, groups):
     return res
 
 
-@pytest.mark.parametrize("case", ["kanamori", "anderson", "free"])
+@pytest.mark.parametrize("case", ["kanamori", "torus", "free"])
 def test_grouped_operands(case):
     from edlib_amd.batch import Batch
-    ml = 3 if case == "kanamori" else 1
-    p = siam_params(13, ml, np.random.default_rng(21), mu=1.3, h0_offdiag=0.2 if ml > 1 else 0.0)
-    if case == "free":  # without interaction: products of one spin's eigenvectors are eigenvectors
-        p["U"] = 0.0 * p["U"]
-    sec = (7, 6) if case == "kanamori" else (6, 6)
-    m = product_model("siam", p)
+    if case == "kanamori":
+        kind, sec, p = "siam", (7, 6), siam_params(13, 3, np.random.default_rng(21), mu=1.3, h0_offdiag=0.2)
+    else:  # free: without interaction products of one spin's eigenvectors are eigenvectors
+        u = 0.0 if case == "free" else 4.0
+        kind, sec, p = "hubbard", (5, 5), dict(Ns=14, t=torus_hopping(2, 7, 1.0, -0.3), U=np.full(14, u),
+                                               xmu=np.full(14, 0.7))
+    m = product_model(kind, p)
     ctx, n = _on_lines(m, sec)
     rng = np.random.default_rng(5)
     vs = [rng.uniform(-1, 1, n) for _ in range(5)]
     vs = [v / np.linalg.norm(v) for v in vs]
     if case == "free":
-        x = _spin_vector(m, 13, 6)
+        x = _spin_vector(m, 14, 5)
         vs[1] = np.kron(x, x)
     b = Batch(0)
     sid = b.add_sector(m, *sec)[0]
@@ -94,7 +96,7 @@ def test_grouped_operands(case):
         scale = max(1.0, np.abs(a1).max())
         assert n1 == nl and np.abs(a - a1).max() <= 1e-10 * scale and np.abs(be - b1)[:nl].max() <= 1e-10 * scale
     ctx.close()
-    srs = eo.SRS(oracle_model("siam", p), *sec)
+    srs = eo.SRS(oracle_model(kind, p), *sec)
     no, ao, bo = srs.lanczos(vs[0], NL)
     scale = max(1.0, np.abs(ao).max())
     assert no == NL and np.abs(alone[0][1] - ao).max() <= 1e-10 * scale
