@@ -216,6 +216,7 @@ struct DevSector {
   DevSpin up, dn;
   double* values = nullptr;
   int nvalues = 0;  // entries of values
+  size_t lds_room = 0;  // lds_budget() of its device, asked for once
   int nkan = 0;     // impurity terms (entries of kan_off and kan_c)
   bool lines = false;      // the line passes' entries can hold the sector's columns
   bool two_pass = false;   // the two passes' tables are there

@@ -831,13 +831,13 @@ struct Launch {
 Launch plan(const DevSector& ds) {
   Launch L;
   const int64_t Ddn = ds.dn.D;
-  const size_t rowb = (size_t)(Ddn + 1) * sizeof(double);
-  L.lds = rowb <= lds_budget();
+  const size_t rowb = (size_t)(Ddn + 1) * sizeof(double), room = ds.lds_room;
+  L.lds = rowb <= room;
   L.ef = 0;
   size_t valb = 0;
   if (L.lds && ds.dn.ell_s4 != nullptr) L.ef = 3;
   else if (L.lds && ds.dn.ell_q4 != nullptr) L.ef = ds.dn.nvt16 <= 2 ? 2 : 1;
-  else if (L.lds && rowb + (size_t)ds.nvalues * sizeof(double) <= lds_budget()) {
+  else if (L.lds && rowb + (size_t)ds.nvalues * sizeof(double) <= room) {
     L.ef = 4;  // 32-bit entries with the value table beside the row in LDS
     valb = (size_t)ds.nvalues * sizeof(double);
   }

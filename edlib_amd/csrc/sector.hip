@@ -5,7 +5,7 @@
 #include <functional>
 #include <mutex>
 
-#include "edh_internal.h"
+#include "hv_params.h"
 
 namespace edh {
 
@@ -296,6 +296,7 @@ void add_two_pass(Packer& pk, const SectorTables& st, DevSector& ds) {
 void upload_sector(const SectorTables& st, int Ns, DevSector& ds, hipStream_t s, UploadStage* stage) {
   ds.release();
   ds.astream = s;
+  ds.lds_room = lds_budget();
   ds.Ns = Ns;
   ds.nup = st.nup;
   ds.ndn = st.ndn;
